@@ -76,7 +76,7 @@ struct PlanVariant {
   int per_xcd = 0;
   int splitk = 0;  // waves per tile of the split-K launch, 0 = none (mix plans: 1 = four-wave)
   int tile_class = 0;
-  int launch_kind = -1;  // mix plans: the one tile kind of the launch
+  int launch_kind = -1;  // mix plans and LDS tiles: the one tile kind of the launch
 };
 
 struct cxa_bc_plan {
@@ -104,6 +104,8 @@ struct cxa_bc_plan {
   // mix plans (cxa_mix_contract_plan): blks are items, segs their slices, outs the outputs
   bool mix = false;
   std::vector<cxa::MixOut> outs;
+  // a step of a matvec chain (bc_join_chain)
+  bool chain = false;
 };
 
 namespace cxa {
@@ -125,11 +127,29 @@ int build_variant(cxa_bc_plan *p, int prec) {
     v.tile_class = make_tiles(p->blks, p->segs, tiles, &v.per_xcd, v.launch_kind, false);
     v.splitk = v.split_mode == 1 ? 1 : 0;  // mix plans: four-wave workgroups (two slices each)
   } else {
-    v.tile_class = make_tiles(p->blks, p->segs, tiles, &v.per_xcd, v.kind, real);
-    const bool split = real && v.tile_class != 2 &&
-                       (v.split_mode >= 1 ||
-                        (v.split_mode < 0 && prefer_splitk(p->blks, p->segs, tiles,
-                                                           v.tile_class)));
+    int kind = v.kind, auto_split = -1;
+    if (kind < 0 && v.split_mode < 0 && prec != CXA_PREC_FP32X3 && !(p->chain && real)) {
+      const Tiling t = default_tiling(p->blks, p->segs, !real);
+      kind = t.kind;
+      auto_split = t.kind < 0 ? -1 : t.split;
+    }
+    // The FP32X3 arithmetic has no LDS tiles and complex plans no 64 x 64 ones, and a segment may
+    // be too wide for either: such plans take the direct (complex: the smaller) tile
+    if (kind == TK_L64 && !real) kind = TK_L32;
+    bool lds = is_lds(kind) && prec != CXA_PREC_FP32X3;
+    for (size_t i = 0; lds && i < p->blks.size(); ++i)
+      for (int s = p->blks[i].seg0; lds && s < p->blks[i].seg0 + p->blks[i].nseg; ++s)
+        lds = lds_ok(p->blks[i], p->segs[s]);
+    if (is_lds(kind) && !lds) kind = TK_2x2;
+    v.launch_kind = kind;
+    v.tile_class = make_tiles(p->blks, p->segs, tiles, &v.per_xcd, kind, real);
+    // (complex split tiles are 16 x 16)
+    const bool may_split =
+        (real || kind == TK_1x1) && v.tile_class != 2 && v.tile_class != 3;
+    const bool split =
+        may_split && (v.split_mode >= 1 || auto_split > 0 ||
+                      (v.split_mode < 0 && auto_split < 0 &&
+                       prefer_splitk(p->blks, p->segs, tiles, v.tile_class)));
     // eight-wave split-K only for MFMA tiles (row tiles always split over four waves)
     v.splitk = !split ? 0 : (v.split_mode == 2 && v.tile_class == 0 ? 8 : 4);
   }
@@ -189,6 +209,7 @@ int upload_plan(cxa_bc_plan *p) {
     p->dev_bjobsB = (const BatchCopyJob *)at(5);
     p->dev_btasksB = (const BatchCopyTask *)at(6);
   }
+  if (p->chain) return CXA_OK;  // cxa_chain_create makes the tile list (bc_join_chain)
   return build_variant(p, native_prec(p->dtype));
 }
 
@@ -239,6 +260,22 @@ int bc_ensure(const cxa_bc_plan *cp, int prec, hipStream_t s) {
   return build_variant(p, prec);
 }
 
+// Real steps of a chain keep the direct tiles: their tile list fixes the order in which a fused
+// Lanczos iteration sums its dot products, and with it the last bits of alpha and beta, from
+// which the sign of an unconverged Ritz vector follows.  (The LDS tiles would take the FP64 .R
+// launch at chi = 2048 from 37 to 35 us and change nothing at 1024.)
+int bc_join_chain(const cxa_bc_plan *cp) {
+  cxa_bc_plan *p = const_cast<cxa_bc_plan *>(cp);
+  std::lock_guard<std::mutex> lk(p->mu);
+  const int prec = native_prec(p->dtype);
+  PlanVariant &v = p->var[prec];
+  const bool was = p->chain;
+  p->chain = true;
+  const bool same = was || p->mix || is_complex(p->dtype) || v.kind >= 0 || v.split_mode >= 0;
+  if (v.built && same) return CXA_OK;
+  return build_variant(p, prec);
+}
+
 int bc_prepare(const cxa_bc_plan *p) {
   for (int q = 0; q < 3; ++q) {
     const int rc = bc_ensure(p, q, nullptr);
@@ -268,6 +305,8 @@ extern "C" int cxa_block_contract_plan(int dtype, int rankL, int nbL, const uint
                                        cxa_bc_plan **out) {
   CXA_CHECK(out, CXA_ERR_INVALID, "cxa_block_contract_plan: null output handle");
   *out = nullptr;
+  const bool chain = (dtype & CXA_PLAN_CHAIN) != 0;
+  dtype &= ~CXA_PLAN_CHAIN;
   const int es = elem_size(dtype);
   CXA_CHECK(dtype == CXA_F64 || dtype == CXA_F32 || dtype == CXA_C128 || dtype == CXA_C64,
             CXA_ERR_UNSUPPORTED, "block contract: unsupported dtype %d", dtype);
@@ -293,6 +332,7 @@ extern "C" int cxa_block_contract_plan(int dtype, int rankL, int nbL, const uint
   std::unique_ptr<cxa_bc_plan> p(new cxa_bc_plan());
   p->dtype = dtype;
   p->es = es;
+  p->chain = chain;
   CXA_HIP(hipGetDevice(&p->device));
 
   // right blocks by common-qindex tuple (ascending block order), output blocks by itoi
@@ -553,6 +593,8 @@ extern "C" int cxa_strided_batch_plan(int dtype, int64_t nbatch, int64_t M, int6
                                       int64_t c_bstride, int64_t ldc, cxa_bc_plan **out) {
   CXA_CHECK(out, CXA_ERR_INVALID, "cxa_strided_batch_plan: null output handle");
   *out = nullptr;
+  const bool chain = (dtype & CXA_PLAN_CHAIN) != 0;
+  dtype &= ~CXA_PLAN_CHAIN;
   CXA_CHECK(dtype == CXA_F64 || dtype == CXA_F32 || dtype == CXA_C128 || dtype == CXA_C64,
             CXA_ERR_UNSUPPORTED, "strided batch plan: unsupported dtype %d", dtype);
   CXA_CHECK(nbatch >= 0 && nbatch <= INT32_MAX && M >= 0 && N >= 0 && K >= 0 &&
@@ -565,6 +607,7 @@ extern "C" int cxa_strided_batch_plan(int dtype, int64_t nbatch, int64_t M, int6
   std::unique_ptr<cxa_bc_plan> p(new cxa_bc_plan());
   p->dtype = dtype;
   p->es = elem_size(dtype);
+  p->chain = chain;
   CXA_HIP(hipGetDevice(&p->device));
   const double cplx = is_complex(dtype) ? 4.0 : 1.0;
   for (int64_t b = 0; b < nbatch; ++b) {
@@ -725,10 +768,8 @@ int bc_exec_typed(const cxa_bc_plan *p, const void *L, const void *R, void *C, i
   g.conj = is_complex(p->dtype) ? conj : 0;
   g.dot_x = lay->dot_x;
   g.dot_part = lay->dot_part;
-  if (p->mix) {
-    g.outs = lay->outs ? lay->outs : p->dev_outs;
-    g.kind0 = v.launch_kind;
-  }
+  g.kind0 = v.launch_kind;
+  if (p->mix) g.outs = lay->outs ? lay->outs : p->dev_outs;
   return launch_grouped_gemm(g, s);
 }
 
@@ -981,7 +1022,8 @@ extern "C" int cxa_gemm_batch(int dtype, const char *transa, const char *transb,
   }
   std::vector<GTile> tiles;
   int per_xcd = 0;
-  const int cls = make_tiles(blks, segs, tiles, &per_xcd, -1, dtype == CXA_F64 || dtype == CXA_F32);
+  const Tiling tl = default_tiling(blks, segs, cplx);
+  const int cls = make_tiles(blks, segs, tiles, &per_xcd, tl.kind, !cplx);
   if (tiles.empty()) return CXA_OK;
   hipStream_t s = (hipStream_t)stream;
   DevBuf d_blks, d_segs, d_tiles;
@@ -1000,6 +1042,8 @@ extern "C" int cxa_gemm_batch(int dtype, const char *transa, const char *transb,
   g.ntiles = (int)tiles.size();
   g.per_xcd = per_xcd;
   g.tile_class = cls;
+  g.kind0 = tl.kind;
+  g.splitk = tl.split;
   rc = launch_grouped_gemm(g, s);
   if (rc) return rc;
   // the task arrays are freed on return: wait for the launch that reads them

@@ -80,6 +80,8 @@ bool bc_is_mix(const cxa_bc_plan *p);
 // precision at creation); refused while `s` is capturing a graph.  bc_prepare makes all three.
 int bc_ensure(const cxa_bc_plan *p, int prec, hipStream_t s);
 int bc_prepare(const cxa_bc_plan *p);
+// The plan becomes a step of a matvec chain (its FP64 default tiling is then the direct one).
+int bc_join_chain(const cxa_bc_plan *p);
 // Tile slots a dot-product epilogue of an execution at precision prec writes (the launch's tile
 // list length), or 0 when that launch cannot carry one (mix, complex, row-streaming tiles).
 int bc_dot_slots(const cxa_bc_plan *p, int prec);

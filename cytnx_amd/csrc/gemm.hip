@@ -26,6 +26,62 @@ int default_kind(int M, int N) {
   return TK_2x2;
 }
 
+namespace {
+
+int64_t tiles_of(const GBlk &b, int t) {
+  return (int64_t)((b.M + t - 1) / t) * ((b.N + t - 1) / t);
+}
+
+// The choice from the number of 16 x 16 tiles, their mean K in 16-deep chunks and the number of
+// 64 x 64 tiles.  A 16 x 16 tile is the finest split of the output, and a wave works through its
+// K one MFMA after another, so few tiles leave SIMDs idle: up to kFew of them (two, complex four,
+// times the CUs) the four waves of a workgroup share a tile's K, which then also hides their load
+// latency.  Above that the LDS tiles read every operand element once per 32 or 64 rows instead
+// of once per 16, in contiguous runs.  Measured (us, split 16 x 16 / 32 x 32 LDS):
+//   real, product of n = 128: 3.9 / 5.2, 256: 4.9 / 7.3, 512 (1024 tiles): 21.2 / 11.5;
+//   complex128, n = 256: 6.4 / 13.9, 384 x 960 x 192 (288 tiles): 27 / 43, 512: 30 / 26;
+//   block contractions of a chi = 512 complex128 MPS (about 830 tiles): 12-20 / 31 (the direct
+//   32 x 32 tiles 100); two-site .R launch in FP64, chi = 512: 4.8 / 5.8, 2048: 43 / 35.
+// 64 x 64 tiles (a quarter of the chunk loads and barriers per flop) pay once they give most CUs
+// a tile: n = 700 (121 tiles) 36 us against 23 in FP64, 900 (225 tiles) 44 against 46, 1600 165
+// against 177.  They are real-only: a complex 64 x 64 tile's registers leave one or two waves
+// per SIMD (n = 1600, complex128: 578 us against 525).
+constexpr int64_t kFewReal = 512, kFewCplx = 1024, kMany64 = 192;
+
+}  // namespace
+
+Tiling default_tiling(const std::vector<GBlk> &blks, const std::vector<GSeg> &segs, bool cplx) {
+  int64_t n16 = 0, n64 = 0, work = 0;
+  bool narrow = !cplx, lds = true;
+  for (const GBlk &b : blks) {
+    if (b.M <= 0 || b.N <= 0) continue;
+    const int64_t t = tiles_of(b, 16);
+    n16 += t;
+    n64 += tiles_of(b, 64);
+    if (b.N > kRowsN) narrow = false;
+    for (int s = b.seg0; s < b.seg0 + b.nseg; ++s) {
+      work += t * ((segs[s].K + 15) / 16);
+      lds = lds && lds_ok(b, segs[s]);
+    }
+  }
+  // K of up to two chunks: an output-bound launch (the MPO steps).  Narrow real blocks stream
+  // their rows (their default), others take one wave per tile: the smallest tiles while they
+  // are few (4.2 us against 4.5 for 128 blocks of 128 x 10, K = 10)
+  if (work <= 2 * n16) return {narrow || n16 > 4 * kFewReal ? -1 : (int)TK_1x1, 0};
+  if (n16 <= (cplx ? kFewCplx : kFewReal)) return {TK_1x1, 4};
+  if (!lds || narrow) return {-1, 0};
+  return {!cplx && n64 >= kMany64 ? TK_L64 : TK_L32, 0};
+}
+
+// One block of one segment (a dense product): the same rule with the whole K in one segment.  A
+// tall K = 10 product of 36864 x 10 takes 4.5 us in direct tiles and 7.9 in LDS tiles.
+Tiling single_tiling(const GBlk &b, const GSeg &s, bool cplx) {
+  const int64_t n16 = tiles_of(b, 16);
+  if (n16 <= (cplx ? kFewCplx : kFewReal) / 2) return {TK_1x1, s.K > 32 ? 4 : 0};
+  if (s.K <= 32 || !lds_ok(b, s)) return {default_kind(b.M, b.N), 0};
+  return {!cplx && tiles_of(b, 64) >= kMany64 ? TK_L64 : TK_L32, 0};
+}
+
 int make_tiles(const std::vector<GBlk> &blks, const std::vector<GSeg> &segs,
                std::vector<GTile> &tiles, int *per_xcd, int kind_override, bool allow_rows) {
   struct Item {
@@ -37,7 +93,8 @@ int make_tiles(const std::vector<GBlk> &blks, const std::vector<GSeg> &segs,
   for (const GBlk &b : blks)
     if (b.M > 0 && b.N > kRowsN) all_narrow = false;
   int cls = TC_MIXED;
-  if (kind_override == TK_4x2 && allow_rows) cls = TC_BIG;  // allow_rows: real dtypes only
+  if (is_lds(kind_override)) cls = TC_LDS;
+  else if (kind_override == TK_4x2 && allow_rows) cls = TC_BIG;  // allow_rows: real dtypes only
   else if (kind_override == TK_ROWS ? all_narrow : (kind_override < 0 && all_narrow))
     cls = TC_ROWS;
   // blocks in operand order: first segment's A offset, then its B offset (the scratch
@@ -62,7 +119,7 @@ int make_tiles(const std::vector<GBlk> &blks, const std::vector<GSeg> &segs,
       kind = TK_ROWS;
     else if (cls == TC_BIG)
       kind = TK_4x2;
-    else if (kind_override >= 0 && kind_override <= TK_1x2)
+    else if (cls == TC_LDS || (kind_override >= 0 && kind_override <= TK_1x2))
       kind = kind_override;
     else
       kind = default_kind(b.M, b.N);
@@ -107,7 +164,7 @@ int make_tiles(const std::vector<GBlk> &blks, const std::vector<GSeg> &segs,
 
 bool prefer_splitk(const std::vector<GBlk> &blks, const std::vector<GSeg> &segs,
                    const std::vector<GTile> &tiles, int tile_class) {
-  if (tiles.empty() || tile_class == TC_BIG) return false;
+  if (tiles.empty() || tile_class == TC_BIG || tile_class == TC_LDS) return false;
   // a tile's work is its block's: summed once per block, then once per tile
   thread_local std::vector<int64_t> bwork;
   bwork.assign(blks.size(), -1);

@@ -46,18 +46,23 @@ struct MixOut {
 };
 
 // tile shapes: MFMA wave tiles (rows x cols) and TK_ROWS, 64 rows of a block with N <= 8
-// streamed one row per lane
+// streamed one row per lane; TK_L64 and TK_L32, 64x64 and 32x32 tiles of a workgroup staged
+// through LDS
 enum TileKind : int32_t {
-  TK_1x1 = 0, TK_2x2 = 1, TK_2x1 = 2, TK_1x2 = 3, TK_4x2 = 4, TK_ROWS = 5, TK_COUNT
+  TK_1x1 = 0, TK_2x2 = 1, TK_2x1 = 2, TK_1x2 = 3, TK_4x2 = 4, TK_ROWS = 5, TK_L64 = 6,
+  TK_L32 = 7, TK_COUNT
 };
+inline bool is_lds(int kind) { return kind == TK_L64 || kind == TK_L32; }
 inline int tile_rows(int kind) {
-  static const int r[TK_COUNT] = {16, 32, 32, 16, 64, 64};
+  static const int r[TK_COUNT] = {16, 32, 32, 16, 64, 64, 64, 32};
   return r[kind];
 }
 inline int tile_cols(int kind) {
-  static const int c[TK_COUNT] = {16, 32, 16, 32, 32, 8};
+  static const int c[TK_COUNT] = {16, 32, 16, 32, 32, 8, 64, 32};
   return c[kind];
 }
+
+constexpr int kRowsN = 8;  // widest block the row-streaming path takes
 
 struct GTile {
   int32_t blk, m0, n0, kind;
@@ -131,7 +136,24 @@ int make_tiles(const std::vector<GBlk> &blks, const std::vector<GSeg> &segs,
 bool prefer_splitk(const std::vector<GBlk> &blks, const std::vector<GSeg> &segs,
                    const std::vector<GTile> &tiles, int tile_class);
 
-// Tile kind used for a block of M x N when no tuned choice is given.
+// Direct tile kind used for a block of M x N when no other choice is given.
 int default_kind(int M, int N);
+
+// Tiling of a launch when the caller gives none: a tile kind (-1: make_tiles' default kinds) and
+// the waves a tile's K range is split over (0 or 4).
+struct Tiling {
+  int kind, split;
+};
+Tiling default_tiling(const std::vector<GBlk> &blks, const std::vector<GSeg> &segs, bool cplx);
+Tiling single_tiling(const GBlk &blk, const GSeg &seg, bool cplx);
+
+// Whether an LDS tile may read a segment: its loads use 32-bit byte offsets from the tile's
+// first element (elements of up to 16 bytes, up to 64 rows and 64 values of k, also with the
+// segment remapped to a k4-packed view).
+inline bool lds_ok(const GBlk &b, const GSeg &s) {
+  const int64_t lim = (int64_t(1) << 31) / 16 / 64;
+  return s.sam + s.sak < lim && s.sbk + s.sbn < lim && (int64_t)b.M < lim / 2 &&
+         (int64_t)b.N < lim / 2;
+}
 
 }  // namespace cxa

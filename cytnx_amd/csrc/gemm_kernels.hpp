@@ -65,7 +65,6 @@ struct alignas(8) cf {
 };
 
 constexpr int kWaves = 4;
-constexpr int kRowsN = 8;  // widest block the row-streaming path takes
 
 // Operand layouts of a launch (template bit set PK): B, A k4-packed (GemmLaunch::b_k4 / a_k4),
 // mix outputs written k4-packed (GemmLaunch::c_k4).
@@ -77,6 +76,8 @@ __device__ __forceinline__ f64x4 mma64(double a, double b, f64x4 c) {
 __device__ __forceinline__ f32x4 mma32(float a, float b, f32x4 c) {
   return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0);
 }
+__device__ __forceinline__ f64x4 mma(double a, double b, f64x4 c) { return mma64(a, b, c); }
+__device__ __forceinline__ f32x4 mma(float a, float b, f32x4 c) { return mma32(a, b, c); }
 
 // Accumulator row held in register v by lane group g = lane/16 (column = lane%16), measured on
 // gfx950: v_mfma_f64_16x16x4_f64 interleaves rows (g + 4v), v_mfma_f32_16x16x4_f32 blocks
@@ -140,6 +141,11 @@ template <int PREC, int MI, int NI>
 struct RealAcc {
   static constexpr bool F64 = (PREC == CXA_PREC_FP64);
   using acc_t = typename std::conditional<F64, f64x4, f32x4>::type;
+  // Chunks in flight per wave: enough loads outstanding to cover an L2/MALL round trip with a
+  // tile's whole K range at the usual block sizes (K <= 64 is one round trip), within a register
+  // budget that keeps several waves per SIMD.
+  static constexpr int depth =
+      (MI * NI >= 8 || (PREC != CXA_PREC_FP32 && MI * NI >= 4)) ? 2 : 4;
   acc_t hi[MI][NI];
   acc_t lo[MI][NI];
   __device__ __forceinline__ void zero() {
@@ -266,12 +272,38 @@ __device__ __forceinline__ void mma_frag(RealAcc<PREC, MI, NI> &acc,
   }
 }
 
-// Chunks in flight per wave: enough loads outstanding to cover an L2/MALL round trip with a
-// tile's whole K range at the usual block sizes (K <= 64 is one round trip), within a register
-// budget that keeps several waves per SIMD.
-template <int PREC, int MI, int NI>
-constexpr int pipe_depth() {
-  return (MI * NI >= 8 || (PREC != CXA_PREC_FP32 && MI * NI >= 4)) ? 2 : 4;
+// Complex tiles (C128 on FP64 MFMA, C64 on FP32 MFMA): four real products per step.  sa, sb: -1
+// conjugates A, B as they are consumed (the adjoint contractions).
+template <typename op_t, int MI, int NI>
+struct CplxAcc {
+  static constexpr bool F64 = std::is_same<op_t, double>::value;
+  using acc_t = typename std::conditional<F64, f64x4, f32x4>::type;
+  static constexpr int depth = MI * NI == 1 ? (F64 ? 3 : 4) : (MI * NI == 2 || !F64 ? 2 : 1);
+  acc_t re[MI][NI], im[MI][NI];
+  op_t sa, sb;
+  __device__ __forceinline__ void zero() {
+#pragma unroll
+    for (int i = 0; i < MI; ++i)
+#pragma unroll
+      for (int j = 0; j < NI; ++j) re[i][j] = im[i][j] = acc_t{0, 0, 0, 0};
+  }
+};
+
+template <typename op_t, typename T, int MI, int NI>
+__device__ __forceinline__ void mma_frag(CplxAcc<op_t, MI, NI> &acc, const Frag<T, T, MI, NI> &f) {
+#pragma unroll
+  for (int k = 0; k < 4; ++k)
+#pragma unroll
+    for (int i = 0; i < MI; ++i)
+#pragma unroll
+      for (int j = 0; j < NI; ++j) {
+        const op_t ar = f.a[i][k].x, ai = acc.sa * f.a[i][k].y;
+        const op_t br = f.b[j][k].x, bi = acc.sb * f.b[j][k].y;
+        acc.re[i][j] = mma(ar, br, acc.re[i][j]);
+        acc.im[i][j] = mma(ar, bi, acc.im[i][j]);
+        acc.re[i][j] = mma(-ai, bi, acc.re[i][j]);
+        acc.im[i][j] = mma(ai, br, acc.im[i][j]);
+      }
 }
 
 // Walks the 16-deep K chunks c of a block's concatenated segments with c % nslices == slice,
@@ -315,19 +347,19 @@ struct ChunkCursor {
 };
 
 // Accumulate the chunks c with c % nslices == slice of the block's concatenated K range.
-// A ring of pipe_depth() fragment sets keeps that many chunks' loads in flight across the
+// A ring of ACC::depth fragment sets keeps that many chunks' loads in flight across the
 // whole range (segment boundaries included): the MFMAs of chunk c issue while chunks
 // c+1 .. c+depth-1 are still arriving, and chunk c+depth is loaded into the set just consumed.
 // Only real chunks are loaded: the launches are bound by the vector-memory address path, so
 // padding a wave's chunk count to whole rounds of the ring (which would let every wait count
 // be exact) costs more than the waits it saves.
-template <int PREC, typename TA, typename TB, int MI, int NI, int PK, typename SEGS>
-__device__ __forceinline__ void mfma_accumulate(RealAcc<PREC, MI, NI> &acc,
+template <typename TA, typename TB, int MI, int NI, int PK, typename ACC, typename SEGS>
+__device__ __forceinline__ void mfma_accumulate(ACC &acc,
                                                 const char *__restrict__ Abase,
                                                 const char *__restrict__ Bbase, const GBlk &blk,
                                                 SEGS segs, int m0, int n0, int lane, int slice,
                                                 int nslices) {
-  constexpr int D = pipe_depth<PREC, MI, NI>();
+  constexpr int D = ACC::depth;
   const int r = lane & 15, g = lane >> 4;
   const int mt = min(16 * MI, blk.M - m0);
   const int nt = min(16 * NI, blk.N - n0);
@@ -356,7 +388,7 @@ __device__ __forceinline__ void mfma_accumulate(RealAcc<PREC, MI, NI> &acc,
     for (int d = 0; d < D; ++d) {
       const int c = base + d;
       if (c < total) {
-        mma_frag<PREC, TA, TB, MI, NI>(acc, f[d]);
+        mma_frag(acc, f[d]);
         if (c + D < total) {
           cur.template load<MI, NI, PK>(f[d], mt, nt, r, g);
           cur.skip(nslices, Abase, Bbase);
@@ -372,6 +404,23 @@ __device__ __forceinline__ void store_c(gptr<TC> dst, double val, const GBlk &bl
   val *= blk.alpha;
   if (blk.beta != 0.0) val += blk.beta * (double)(*dst);
   *dst = (TC)val;
+}
+
+// The complex form: alpha and beta are complex (Gemm_Batch passes Scalars; contractions use
+// alpha = 1, beta = 0).
+template <typename op_t, typename C2>
+__device__ __forceinline__ void store_cplx(C2 dst, double xr, double xi, const GBlk &blk) {
+  double re = blk.alpha * xr - blk.alpha_im * xi, im = blk.alpha * xi + blk.alpha_im * xr;
+  if (blk.beta != 0.0 || blk.beta_im != 0.0) {
+    const auto o = *dst;
+    re += blk.beta * (double)o.x - blk.beta_im * (double)o.y;
+    im += blk.beta * (double)o.y + blk.beta_im * (double)o.x;
+  }
+  typedef op_t c2 __attribute__((ext_vector_type(2)));
+  c2 w;
+  w.x = (op_t)re;
+  w.y = (op_t)im;
+  *dst = w;
 }
 
 // Sum over the 64 lanes of a wave (butterfly; every lane gets the same value).
@@ -426,7 +475,7 @@ __device__ __forceinline__ void wave_tile_real(const char *__restrict__ Abase,
               row < mt && col < nt);
         }
   }
-  mfma_accumulate<PREC, TA, TB, MI, NI, PK>(acc, Abase, Bbase, blk, segs, m0, n0, lane, 0, 1);
+  mfma_accumulate<TA, TB, MI, NI, PK>(acc, Abase, Bbase, blk, segs, m0, n0, lane, 0, 1);
   gptr<TC> Cp = at<TC>(Cbase, blk.c_off);
 #pragma unroll
   for (int i = 0; i < MI; ++i)
@@ -464,12 +513,12 @@ __device__ __forceinline__ void wave_tile_real(const char *__restrict__ Abase,
 // Split-K tile: every wave of the workgroup (WAVES of them) calls this for the same tile; wave
 // w takes the K chunks c with c % WAVES == w, and the partial tiles are summed in wave order.
 template <int PREC, typename TA, typename TB, typename TC, int MI, int NI, int WAVES, int PK,
-          typename SEGS>
+          typename SEGS, typename RED>
 __device__ __forceinline__ void wg_tile_real(const char *__restrict__ Abase,
                                              const char *__restrict__ Bbase,
                                              char *__restrict__ Cbase, const GBlk &blk,
                                              SEGS segs, int m0, int n0, int lane, int wave,
-                                             double (*red)[16][64],
+                                             RED red,
                                              const double *__restrict__ dotx = nullptr,
                                              double *dslot = nullptr, int64_t nslots = 0) {
   RealAcc<PREC, MI, NI> acc;
@@ -509,7 +558,7 @@ __device__ __forceinline__ void wg_tile_real(const char *__restrict__ Abase,
       }
     }
   }
-  mfma_accumulate<PREC, TA, TB, MI, NI, PK>(acc, Abase, Bbase, blk, segs, m0, n0, lane, wave,
+  mfma_accumulate<TA, TB, MI, NI, PK>(acc, Abase, Bbase, blk, segs, m0, n0, lane, wave,
                                         WAVES);
 #pragma unroll
   for (int i = 0; i < MI; ++i)
@@ -681,126 +730,99 @@ __device__ __forceinline__ void wg_rows(const char *__restrict__ Abase,
 }
 
 // ---------------------------------------------------------------------------------------
-// complex MFMA tiles (C128 on FP64 MFMA, C64 on FP32 MFMA): four real products per step
+// complex MFMA tiles: elements move as two-wide vectors (x = real, y = imaginary; same size and
+// alignment as the structs), which load and store through global-address-space pointers.
+// conj: bit 0 conjugates A, bit 1 conjugates B.
 // ---------------------------------------------------------------------------------------
-// conj: bit 0 conjugates A, bit 1 conjugates B as they are loaded (the adjoint contractions).
+typedef double d2v __attribute__((ext_vector_type(2)));
+typedef float f2v __attribute__((ext_vector_type(2)));
+template <typename CT>
+struct CplxOf;
+template <>
+struct CplxOf<cd> {
+  using op = double;
+  using vec = d2v;
+};
+template <>
+struct CplxOf<cf> {
+  using op = float;
+  using vec = f2v;
+};
+
 template <typename CT, int MI, int NI, typename SEGS>
 __device__ __forceinline__ void wave_tile_cplx(const char *__restrict__ Abase,
                                                const char *__restrict__ Bbase,
                                                char *__restrict__ Cbase, const GBlk &blk,
                                                SEGS segs, int m0, int n0, int lane, int conj) {
-  constexpr bool F64 = std::is_same<CT, cd>::value;
-  using acc_t = typename std::conditional<F64, f64x4, f32x4>::type;
-  using op_t = typename std::conditional<F64, double, float>::type;
-  // complex elements move as two-wide vectors (x = real, y = imaginary; same size and
-  // alignment as CT), which load and store through global-address-space pointers
-  typedef op_t c2 __attribute__((ext_vector_type(2)));
+  using op_t = typename CplxOf<CT>::op;
+  using c2 = typename CplxOf<CT>::vec;
   static_assert(sizeof(c2) == sizeof(CT), "complex element layout");
-  const op_t sa = (conj & 1) ? op_t(-1) : op_t(1), sb = (conj & 2) ? op_t(-1) : op_t(1);
+  CplxAcc<op_t, MI, NI> acc;
+  acc.zero();
+  acc.sa = (conj & 1) ? op_t(-1) : op_t(1);
+  acc.sb = (conj & 2) ? op_t(-1) : op_t(1);
+  mfma_accumulate<c2, c2, MI, NI, 0>(acc, Abase, Bbase, blk, segs, m0, n0, lane, 0, 1);
   const int r = lane & 15, g = lane >> 4;
-  const int mt = min(16 * MI, blk.M - m0);
-  const int nt = min(16 * NI, blk.N - n0);
-  acc_t accr[MI][NI], acci[MI][NI];
-#pragma unroll
-  for (int i = 0; i < MI; ++i)
-#pragma unroll
-    for (int j = 0; j < NI; ++j) {
-      accr[i][j] = acc_t{0, 0, 0, 0};
-      acci[i][j] = acc_t{0, 0, 0, 0};
-    }
-  for (int s = 0; s < blk.nseg; ++s) {
-    const GSeg sg = segs(blk.seg0 + s);
-    gptr<const c2> Ap = at<const c2>(Abase, sg.a_off) + (int64_t)m0 * sg.sam;
-    gptr<const c2> Bp = at<const c2>(Bbase, sg.b_off) + (int64_t)n0 * sg.sbn;
-    const int K = sg.K;
-    for (int k0 = 0; k0 < K; k0 += 16) {
-      c2 va[MI][4], vb[NI][4];  // every load of the chunk issued before the first use
-#pragma unroll
-      for (int i = 0; i < MI; ++i) {
-        const int row = 16 * i + r;
-#pragma unroll
-        for (int j = 0; j < 4; ++j) {
-          const int k = k0 + 4 * g + j;
-          va[i][j] = load_or_zero<c2>(Ap + ((int64_t)row * sg.sam + (int64_t)k * sg.sak),
-                                      row < mt && k < K);
-        }
-      }
-#pragma unroll
-      for (int i = 0; i < NI; ++i) {
-        const int col = 16 * i + r;
-#pragma unroll
-        for (int j = 0; j < 4; ++j) {
-          const int k = k0 + 4 * g + j;
-          vb[i][j] = load_or_zero<c2>(Bp + ((int64_t)k * sg.sbk + (int64_t)col * sg.sbn),
-                                      col < nt && k < K);
-        }
-      }
-      op_t ar[MI][4], ai[MI][4], br[NI][4], bi[NI][4];
-#pragma unroll
-      for (int i = 0; i < MI; ++i)
-#pragma unroll
-        for (int j = 0; j < 4; ++j) {
-          ar[i][j] = va[i][j].x;
-          ai[i][j] = sa * va[i][j].y;
-        }
-#pragma unroll
-      for (int i = 0; i < NI; ++i)
-#pragma unroll
-        for (int j = 0; j < 4; ++j) {
-          br[i][j] = vb[i][j].x;
-          bi[i][j] = sb * vb[i][j].y;
-        }
-#pragma unroll
-      for (int j = 0; j < 4; ++j)
-#pragma unroll
-        for (int i = 0; i < MI; ++i)
-#pragma unroll
-          for (int jj = 0; jj < NI; ++jj) {
-            if constexpr (F64) {
-              accr[i][jj] = mma64(ar[i][j], br[jj][j], accr[i][jj]);
-              accr[i][jj] = mma64(-ai[i][j], bi[jj][j], accr[i][jj]);
-              acci[i][jj] = mma64(ar[i][j], bi[jj][j], acci[i][jj]);
-              acci[i][jj] = mma64(ai[i][j], br[jj][j], acci[i][jj]);
-            } else {
-              accr[i][jj] = mma32(ar[i][j], br[jj][j], accr[i][jj]);
-              accr[i][jj] = mma32(-ai[i][j], bi[jj][j], accr[i][jj]);
-              acci[i][jj] = mma32(ar[i][j], bi[jj][j], acci[i][jj]);
-              acci[i][jj] = mma32(ai[i][j], br[jj][j], acci[i][jj]);
-            }
-          }
-    }
-  }
+  const int mt = min(16 * MI, blk.M - m0), nt = min(16 * NI, blk.N - n0);
   gptr<c2> Cp = at<c2>(Cbase, blk.c_off);
-  // complex alpha and beta (Gemm_Batch passes Scalars); contractions use alpha = 1, beta = 0
-  const double ar_ = blk.alpha, ai_ = blk.alpha_im, br_ = blk.beta, bi_ = blk.beta_im;
 #pragma unroll
   for (int i = 0; i < MI; ++i)
 #pragma unroll
     for (int jj = 0; jj < NI; ++jj)
 #pragma unroll
       for (int v = 0; v < 4; ++v) {
-        const int row = 16 * i + acc_row(F64, g, v);
+        const int row = 16 * i + acc_row(CplxAcc<op_t, MI, NI>::F64, g, v);
         const int col = 16 * jj + r;
-        if (row < mt && col < nt) {
-          const double xr = (double)accr[i][jj][v], xi = (double)acci[i][jj][v];
-          double re = ar_ * xr - ai_ * xi, im = ar_ * xi + ai_ * xr;
-          gptr<c2> dst = Cp + (int64_t)(m0 + row) * blk.ldc + (n0 + col);
-          if (br_ != 0.0 || bi_ != 0.0) {
-            const c2 o = *dst;
-            re += br_ * (double)o.x - bi_ * (double)o.y;
-            im += br_ * (double)o.y + bi_ * (double)o.x;
-          }
-          c2 w;
-          w.x = (op_t)re;
-          w.y = (op_t)im;
-          *dst = w;
-        }
+        if (row < mt && col < nt)
+          store_cplx<op_t>(Cp + ((int64_t)(m0 + row) * blk.ldc + (n0 + col)),
+                           (double)acc.re[i][jj][v], (double)acc.im[i][jj][v], blk);
       }
+}
+
+// Split-K 16 x 16 tile: wave w of the workgroup takes the K chunks c with c % WAVES == w; the
+// partial tiles meet in LDS and value idx of every lane is summed in wave order and stored by
+// wave idx % WAVES.  A lone wave runs its K range's MFMAs one after another on one SIMD: where a
+// launch has fewer tiles than SIMDs, the split spreads a tile over the CU's four.
+template <typename CT, int WAVES, typename SEGS>
+__device__ __forceinline__ void wg_tile_cplx(const char *__restrict__ Abase,
+                                             const char *__restrict__ Bbase,
+                                             char *__restrict__ Cbase, const GBlk &blk, SEGS segs,
+                                             int m0, int n0, int lane, int wave, int conj,
+                                             typename CplxOf<CT>::op (*red)[8][64]) {
+  using op_t = typename CplxOf<CT>::op;
+  using c2 = typename CplxOf<CT>::vec;
+  CplxAcc<op_t, 1, 1> acc;
+  acc.zero();
+  acc.sa = (conj & 1) ? op_t(-1) : op_t(1);
+  acc.sb = (conj & 2) ? op_t(-1) : op_t(1);
+  mfma_accumulate<c2, c2, 1, 1, 0>(acc, Abase, Bbase, blk, segs, m0, n0, lane, wave, WAVES);
+#pragma unroll
+  for (int v = 0; v < 4; ++v) {
+    red[wave][v][lane] = acc.re[0][0][v];
+    red[wave][4 + v][lane] = acc.im[0][0][v];
+  }
+  __syncthreads();
+  const int r = lane & 15, g = lane >> 4;
+  const int mt = min(16, blk.M - m0), nt = min(16, blk.N - n0);
+  if (wave < 4) {
+    const int row = acc_row(CplxAcc<op_t, 1, 1>::F64, g, wave);
+    if (row < mt && r < nt) {
+      double re = (double)red[0][wave][lane], im = (double)red[0][4 + wave][lane];
+#pragma unroll
+      for (int q = 1; q < WAVES; ++q) {
+        re += (double)red[q][wave][lane];
+        im += (double)red[q][4 + wave][lane];
+      }
+      store_cplx<op_t>(at<c2>(Cbase, blk.c_off) + ((int64_t)(m0 + row) * blk.ldc + (n0 + r)), re,
+                       im, blk);
+    }
+  }
+  __syncthreads();
 }
 
 // Tile classes: each class is its own kernel instantiation so that it carries only its own
 // register budget (occupancy matters most for the memory-bound row tiles).
-enum TileClass { TC_MIXED = 0, TC_ROWS = 1, TC_BIG = 2 };
+enum TileClass { TC_MIXED = 0, TC_ROWS = 1, TC_BIG = 2, TC_LDS = 3 };
 
 template <int PREC, typename TA, typename TB, typename TC, bool CPLX, int CLS, int PK,
           typename SEGS>
@@ -926,6 +948,43 @@ __global__ __launch_bounds__(64 * WAVES) void k_grouped_split(
   }
 }
 
+// the complex form: 16 x 16 tiles
+template <typename CT, int WAVES>
+__global__ __launch_bounds__(64 * WAVES, 2) void k_grouped_split_cplx(
+    const GTile *__restrict__ tiles, int per_xcd, const GBlk *__restrict__ blks,
+    const GSeg *__restrict__ segs, const char *A, const char *B, char *C, int conj) {
+  __shared__ typename CplxOf<CT>::op red[WAVES][8][64];
+  const int lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const GTile *range = tiles + (int64_t)(blockIdx.x % kXcds) * per_xcd;
+  for (int t = blockIdx.x / kXcds; t < per_xcd; t += gridDim.x / kXcds) {
+    const GTile tl = range[t];
+    if (tl.blk < 0) continue;  // padding (uniform over the workgroup)
+    const GBlk blk = blks[tl.blk];
+    wg_tile_cplx<CT, WAVES>(A, B, C, blk, SegArray{segs}, tl.m0, tl.n0, lane, wave, conj, red);
+  }
+}
+
+// single block, 16 x 16 tiles split over the waves of a workgroup
+template <int PREC, typename TA, typename TB, typename TC, bool CPLX>
+__global__ __launch_bounds__(64 * kWaves, 2) void k_single_split(GBlk blk, GSeg seg, int tiles_n,
+                                                               const char *A, const char *B,
+                                                               char *C, int conj) {
+  const int lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int m0 = (int)(blockIdx.x / tiles_n) * 16, n0 = (int)(blockIdx.x % tiles_n) * 16;
+  if constexpr (CPLX) {
+    __shared__ typename CplxOf<TA>::op red[kWaves][8][64];
+    wg_tile_cplx<TA, kWaves>(A, B, C, blk, SegOne{seg}, m0, n0, lane, wave, conj, red);
+  } else {
+    __shared__ double red[kWaves][4][64];
+    wg_tile_real<PREC, TA, TB, TC, 1, 1, kWaves, 0>(A, B, C, blk, SegOne{seg}, m0, n0, lane, wave,
+                                                   red);
+  }
+}
+
+#include "gemm_lds.hpp"
+
 // ---------------------------------------------------------------------------------------
 // mix launches: one workgroup per tile of an item, of kMixSlices waves (wave s computes slice s:
 // the longest dependent load chain of a tile is one slice's K range) or of 4 waves (wave w
@@ -947,7 +1006,7 @@ __device__ __forceinline__ void mfma_accumulate_multi(RealAcc<PREC, MI, NI> (&ac
                                                       const char *__restrict__ Bbase, SEGS segs,
                                                       int nseg, int M, int N, int m0, int n0,
                                                       int lane) {
-  constexpr int D = pipe_depth<PREC, MI, NI>();
+  constexpr int D = RealAcc<PREC, MI, NI>::depth;
   const int r = lane & 15, g = lane >> 4;
   const int mt = min(16 * MI, M - m0);
   const int nt = min(16 * NI, N - n0);
@@ -981,7 +1040,7 @@ __device__ __forceinline__ void mfma_accumulate_multi(RealAcc<PREC, MI, NI> (&ac
   auto consume = [&](const Frag<TA, TB, MI, NI> &fr) {
 #pragma unroll
     for (int q = 0; q < NACC; ++q)
-      if (q == cs) mma_frag<PREC, TA, TB, MI, NI>(acc[q], fr);
+      if (q == cs) mma_frag(acc[q], fr);
     if (--left == 0) {
 #pragma unroll
       for (int q = 1; q < NACC; ++q)
@@ -1205,6 +1264,35 @@ __global__ __launch_bounds__(64 * kWaves) void k_single(GBlk blk, GSeg seg, int 
   }
 }
 
+template <int PREC, typename TA, typename TB, typename TC, bool CPLX, int PK, int KIND>
+void launch_lds_kind(const GemmLaunch &g, int grid, hipStream_t s) {
+  const char *A = (const char *)g.A, *B = (const char *)g.B;
+  if constexpr (PK == 0) {
+    if (g.single) {
+      const int tm = (g.blk0.M + tile_rows(KIND) - 1) / tile_rows(KIND);
+      const int tn = (g.blk0.N + tile_cols(KIND) - 1) / tile_cols(KIND);
+      hipLaunchKernelGGL((k_single_lds<PREC, TA, TB, TC, CPLX, KIND>), dim3(grid),
+                         dim3(64 * kWaves), 0, s, g.blk0, g.seg0, tm, tn, tm * tn, A, B,
+                         (char *)g.C, g.conj);
+      return;
+    }
+  }
+  hipLaunchKernelGGL((k_grouped_lds<PREC, TA, TB, TC, CPLX, KIND, PK>), dim3(grid),
+                     dim3(64 * kWaves), 0, s, g.tiles, g.per_xcd, g.blks, g.segs, A, B,
+                     (char *)g.C, g.conj, g.dot_x, g.dot_part);
+}
+
+template <int PREC, typename TA, typename TB, typename TC, bool CPLX, int PK>
+void launch_lds(const GemmLaunch &g, int kind, int grid, hipStream_t s) {
+  if constexpr (!CPLX) {
+    if (kind == TK_L64) {
+      launch_lds_kind<PREC, TA, TB, TC, CPLX, PK, TK_L64>(g, grid, s);
+      return;
+    }
+  }
+  launch_lds_kind<PREC, TA, TB, TC, CPLX, PK, TK_L32>(g, grid, s);
+}
+
 // the real-dtype grouped launches of one class / split mode
 template <int PREC, typename TA, typename TB, typename TC, int PK>
 void launch_real(const GemmLaunch &g, int cls, int wg_grid, int wave_grid, hipStream_t s) {
@@ -1213,6 +1301,12 @@ void launch_real(const GemmLaunch &g, int cls, int wg_grid, int wave_grid, hipSt
   char *C = (char *)g.C;
   const double *dx = g.dot_x;
   double *dp = g.dot_part;
+  if constexpr (PREC != CXA_PREC_FP32X3) {
+    if (cls == TC_LDS) {
+      launch_lds<PREC, TA, TB, TC, false, PK>(g, g.kind0, wg_grid, s);
+      return;
+    }
+  }
   if (g.splitk && cls == TC_ROWS)
     hipLaunchKernelGGL((k_grouped_split<PREC, TA, TB, TC, TC_ROWS, kWaves, PK>), dim3(wg_grid),
                        dim3(64 * kWaves), 0, s, g.tiles, P, g.blks, g.segs, A, B, C, nullptr,
@@ -1250,8 +1344,33 @@ int launch_t(const GemmLaunch &g, hipStream_t s) {
       return fail(CXA_ERR_INVALID, "single-block GEMM: packed layouts are not supported");
     const GBlk &b = g.blk0;
     if (b.M <= 0 || b.N <= 0) return CXA_OK;
-    int kind = g.kind0 >= 0 ? g.kind0 : default_kind(b.M, b.N);
+    const Tiling tl = single_tiling(b, g.seg0, CPLX);
+    int kind = tl.kind;
+    if constexpr (PREC != CXA_PREC_FP32X3) {
+      if (is_lds(kind)) {
+        const int64_t tm = (b.M + tile_rows(kind) - 1) / tile_rows(kind);
+        const int64_t tn = (b.N + tile_cols(kind) - 1) / tile_cols(kind);
+        if (tm * tn > INT32_MAX / 2)
+          return fail(CXA_ERR_UNSUPPORTED, "GEMM too large: %lld tiles", (long long)(tm * tn));
+        launch_lds<PREC, TA, TB, TC, CPLX, 0>(g, kind,
+                                              kXcds * (int)((tm * tn + kXcds - 1) / kXcds), s);
+        CXA_HIP(hipGetLastError());
+        return CXA_OK;
+      }
+    }
     if (kind == TK_ROWS || kind == TK_4x2) kind = TK_2x2;  // single launches: mixed class
+    if constexpr (PREC != CXA_PREC_FP32X3) {
+      if (tl.split > 0) {
+        const int64_t tn = (b.N + 15) / 16, n = (int64_t)((b.M + 15) / 16) * tn;
+        if (n > INT32_MAX)
+          return fail(CXA_ERR_UNSUPPORTED, "GEMM too large: %lld tiles", (long long)n);
+        hipLaunchKernelGGL((k_single_split<PREC, TA, TB, TC, CPLX>), dim3((unsigned)n),
+                           dim3(64 * kWaves), 0, s, b, g.seg0, (int)tn, (const char *)g.A,
+                           (const char *)g.B, (char *)g.C, g.conj);
+        CXA_HIP(hipGetLastError());
+        return CXA_OK;
+      }
+    }
     const int tiles_m = (b.M + tile_rows(kind) - 1) / tile_rows(kind);
     const int tiles_n = (b.N + tile_cols(kind) - 1) / tile_cols(kind);
     const int64_t nt64 = (int64_t)tiles_m * tiles_n;
@@ -1272,8 +1391,10 @@ int launch_t(const GemmLaunch &g, hipStream_t s) {
   if (g.grid % kXcds)
     return fail(CXA_ERR_INVALID, "grouped GEMM: grid %d is not a multiple of %d", g.grid, kXcds);
   const int cls = g.tile_class;
-  if (CPLX && cls != TC_MIXED)
-    return fail(CXA_ERR_UNSUPPORTED, "complex GEMM tiles must be MFMA tiles up to 32x32");
+  if (CPLX && cls != TC_MIXED && cls != TC_LDS)
+    return fail(CXA_ERR_UNSUPPORTED, "complex GEMM tiles must be MFMA tiles of 32x32 or LDS tiles");
+  if (cls == TC_LDS && g.kind0 != TK_L32 && (CPLX || g.kind0 != TK_L64))
+    return fail(CXA_ERR_INVALID, "grouped GEMM: no LDS tile of kind %d for this dtype", g.kind0);
   const int P = g.per_xcd;
   const int wg_grid = g.grid > 0 ? g.grid : kXcds * std::min(P, 2048);
   const int wave_grid = g.grid > 0 ? g.grid : kXcds * std::min((P + kWaves - 1) / kWaves, 1024);
@@ -1296,7 +1417,18 @@ int launch_t(const GemmLaunch &g, hipStream_t s) {
   } else {
     if (g.a_k4 || g.b_k4 || g.c_k4)
       return fail(CXA_ERR_UNSUPPORTED, "grouped GEMM: packed layouts are real-only");
-    hipLaunchKernelGGL((k_grouped<PREC, TA, TB, TC, true, TC_MIXED, 0>), dim3(wave_grid),
+    if (cls == TC_LDS)
+      launch_lds<PREC, TA, TB, TC, true, 0>(g, g.kind0, wg_grid, s);
+    else if (g.splitk == 8)
+      hipLaunchKernelGGL((k_grouped_split_cplx<TA, 8>), dim3(wg_grid), dim3(64 * 8), 0, s, g.tiles,
+                         P, g.blks, g.segs, (const char *)g.A, (const char *)g.B, (char *)g.C,
+                         g.conj);
+    else if (g.splitk)
+      hipLaunchKernelGGL((k_grouped_split_cplx<TA, 4>), dim3(wg_grid), dim3(64 * 4), 0, s, g.tiles,
+                         P, g.blks, g.segs, (const char *)g.A, (const char *)g.B, (char *)g.C,
+                         g.conj);
+    else
+      hipLaunchKernelGGL((k_grouped<PREC, TA, TB, TC, true, TC_MIXED, 0>), dim3(wave_grid),
                        dim3(64 * kWaves), 0, s, g.tiles, P, g.blks, g.segs,
                        (const char *)g.A, (const char *)g.B, (char *)g.C, g.conj, nullptr,
                        nullptr);

@@ -308,6 +308,7 @@ extern "C" int cxa_chain_create(int nsteps, cxa_bc_plan *const *plans, const voi
               k);
     CXA_CHECK(!cplx || !bc_is_mix(plans[k]), CXA_ERR_UNSUPPORTED,
               "cxa_chain_create: mix plans are real (step %d)", k);
+    CXA_RC(bc_join_chain(plans[k]));
     c->plans.push_back(plans[k]);
     c->fixed.push_back(fixed[k]);
     c->fixed_left.push_back(fixed_is_left[k] ? 1 : 0);
@@ -625,7 +626,8 @@ extern "C" int cxa_chain_tune(cxa_chain *c, const void *x, void *y, int reps, in
                                 {TK_1x1, 0}, {TK_1x1, 1}, {TK_1x1, 2}, {TK_2x1, 0},
                                 {TK_2x1, 1}, {TK_2x1, 2}, {TK_1x2, 0}, {TK_1x2, 1},
                                 {TK_1x2, 2}, {TK_2x2, 0}, {TK_2x2, 1}, {TK_2x2, 2},
-                                {TK_4x2, 0}, {TK_ROWS, 0}, {TK_ROWS, 1}};
+                                {TK_4x2, 0}, {TK_ROWS, 0}, {TK_ROWS, 1}, {TK_L64, 0},
+                                {TK_L32, 0}};
   const int ncand = (int)(sizeof(cand) / sizeof(cand[0]));
   hipEvent_t e0, e1;
   CXA_HIP(hipEventCreate(&e0));
@@ -661,10 +663,15 @@ extern "C" int cxa_chain_tune(cxa_chain *c, const void *x, void *y, int reps, in
       // mix plans: explicit 16x16, 32x16, 16x32 or 32x32 tiles; split 0 / 1 = eight / four
       // waves
       if (bc_is_mix(plan) && (cand[ci][0] < 0 || cand[ci][0] == TK_4x2 ||
-                              cand[ci][0] == TK_ROWS || cand[ci][1] == 2))
+                              cand[ci][0] == TK_ROWS || is_lds(cand[ci][0]) ||
+                              cand[ci][1] == 2))
         continue;
       // the big-tile and row classes are real-only (complex plans fall back to the default)
-      if (c->dtype != CXA_F64 && (cand[ci][0] == TK_4x2 || cand[ci][0] == TK_ROWS)) continue;
+      if (c->dtype != CXA_F64 &&
+          (cand[ci][0] == TK_4x2 || cand[ci][0] == TK_ROWS || cand[ci][0] == TK_L64))
+        continue;
+      // real FP64 steps keep the direct tiles (bc_join_chain); FP32X3 has no LDS tiles
+      if (c->dtype == CXA_F64 && c->prec != CXA_PREC_FP32 && is_lds(cand[ci][0])) continue;
       if ((rc = cxa_block_contract_set_config(plan, c->prec, cand[ci][0], cand[ci][1]))) break;
       double per = 0.0, per_plain = 0.0;
       if ((rc = time_form(pk, &per))) break;

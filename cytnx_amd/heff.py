@@ -30,7 +30,7 @@ import torch
 from . import _lib
 from .device import stream_handle, torch_device
 from .lanczos import LinOp, lanczos_gnd_native
-from .unitensor import (BD_BRA, BD_KET, PREC_FP32, PREC_FP64, Bond, Contract, UniTensor,
+from .unitensor import (BD_BRA, BD_KET, PLAN_CHAIN, PREC_FP32, PREC_FP64, Bond, Contract, UniTensor,
                         _Plan, contract_meta, meta_elems, plan_contraction)
 
 
@@ -507,13 +507,13 @@ class Heff2(_HeffBase):
         psi_m = psi.clone_meta()
         ref_steps = []
         X, c1, c2 = contract_meta(Lp, psi_m, dt, dev)
-        ref_steps.append((plan_contraction(Lp, psi_m, X, c1, c2, dt), Lp, True, X))
+        ref_steps.append((plan_contraction(Lp, psi_m, X, c1, c2, dt, True), Lp, True, X))
         Y, c1, c2 = contract_meta(X, M1, dt, dev)
-        ref_steps.append((plan_contraction(X, M1, Y, c1, c2, dt), M1, False, Y))
+        ref_steps.append((plan_contraction(X, M1, Y, c1, c2, dt, True), M1, False, Y))
         Z, c1, c2 = contract_meta(Y, M2, dt, dev)
-        ref_steps.append((plan_contraction(Y, M2, Z, c1, c2, dt), M2, False, Z))
+        ref_steps.append((plan_contraction(Y, M2, Z, c1, c2, dt, True), M2, False, Z))
         O, c1, c2 = contract_meta(Z, Rp, dt, dev)
-        ref_steps.append((plan_contraction(Z, Rp, O, c1, c2, dt), Rp, False, O))
+        ref_steps.append((plan_contraction(Z, Rp, O, c1, c2, dt, True), Rp, False, O))
         if O.itoi() != psi.itoi() or [b.dim() for b in O.bonds()] != psi.shape():
             raise ValueError("Heff2: output block layout differs from psi's")
         self.ref_flops = float(sum(st[0].flops for st in ref_steps))
@@ -526,7 +526,7 @@ class Heff2(_HeffBase):
             Zf, c1, c2 = contract_meta(X, W12, dt, dev)
             if Zf.labels() != Z.labels() or Zf.itoi() != Z.itoi():
                 raise ValueError("Heff2: fused MPO step changed the intermediate layout")
-            steps = [ref_steps[0], (plan_contraction(X, W12, Zf, c1, c2, dt), W12, False, Zf),
+            steps = [ref_steps[0], (plan_contraction(X, W12, Zf, c1, c2, dt, True), W12, False, Zf),
                      ref_steps[3]]
             self.step_names = ["L.psi", ".W12", ".R"]
             self.mode = "w12"
@@ -594,7 +594,7 @@ class Heff2(_HeffBase):
         if O.itoi() != psi.itoi() or [b.dim() for b in O.bonds()] != psi.shape():
             raise ValueError("Heff2 mix chain: output block layout differs from psi's")
         return [(plan, Lp, not psi_left, Y),
-                (plan_contraction(Y, Rpp, O, c1, c2, 3), Rpp, False, O)]
+                (plan_contraction(Y, Rpp, O, c1, c2, 3, True), Rpp, False, O)]
 
     @property
     def flops(self) -> float:
@@ -622,13 +622,13 @@ class _Flat:
 
 
 def strided_batch_plan(nbatch: int, M: int, N: int, K: int, a: Sequence[int],
-                       b: Sequence[int], c: Sequence[int], dtype: int = 3) -> _Plan:
+                       b: Sequence[int], c: Sequence[int], dtype: int = 3, chain: bool = False) -> _Plan:
     """cxa_strided_batch_plan: C_b = A_b . B_b for b < nbatch with A_b[m, k] at
     a[0]*b + a[1]*m + a[2]*k, B_b[k, n] at b[0]*b + b[1]*k + b[2]*n and C_b[m, n] at
-    c[0]*b + c[1]*m + n (element offsets)."""
+    c[0]*b + c[1]*m + n (element offsets); ``chain`` for a step of a matvec chain."""
     h = ctypes.c_void_p(0)
     _lib.check(_lib.lib().cxa_strided_batch_plan(
-        dtype, nbatch, M, N, K, a[0], a[1], a[2], b[0], b[1], b[2], c[0], c[1],
+        dtype | (PLAN_CHAIN if chain else 0), nbatch, M, N, K, a[0], a[1], a[2], b[0], b[1], b[2], c[0], c[1],
         ctypes.byref(h)))
     return _Plan(h.value, torch.cuda.current_device())
 
@@ -658,11 +658,11 @@ class Heff1Dense(_HeffBase):
         self._Wp = _Flat(W.to(torch.float64).permute(0, 2, 1, 3))   # (w, s, w', s')
         self._R = _Flat(R.to(torch.float64))                        # (r, w', r')
         p1 = strided_batch_plan(1, nlp * D, d * ar, nl, (0, nl, 1), (0, d * ar, 1),
-                                (0, d * ar))
+                                (0, d * ar), chain=True)
         p2 = strided_batch_plan(ar, nlp, Dwp * dsp, D * d, (1, D * d * ar, ar),
-                                (0, Dwp * dsp, 1), (Dwp * dsp, ar * Dwp * dsp))
+                                (0, Dwp * dsp, 1), (Dwp * dsp, ar * Dwp * dsp), chain=True)
         p3 = strided_batch_plan(dsp, nlp, nrp, ar * Dwp, (1, ar * Dwp * dsp, dsp),
-                                (0, nrp, 1), (nrp, dsp * nrp))
+                                (0, nrp, 1), (nrp, dsp * nrp), chain=True)
         steps = [(p1, self._Lp, True, nlp * D * d * ar),
                  (p2, self._Wp, False, nlp * ar * Dwp * dsp),
                  (p3, self._R, False, nlp * dsp * nrp)]

@@ -142,8 +142,13 @@ class _Plan:
 _PLAN_CACHE: Dict[tuple, _Plan] = {}
 
 
+PLAN_CHAIN = 256  # CXA_PLAN_CHAIN
+
+
 def _plan_for(dtype: int, A: "UniTensor", B: "UniTensor", c1: List[int], c2: List[int],
-              C: "UniTensor") -> _Plan:
+              C: "UniTensor", chain: bool = False) -> _Plan:
+    if chain:
+        dtype |= PLAN_CHAIN
     key = (dtype, A.device(), A._itoi.tobytes(), A._shapes.tobytes(), A._offsets.tobytes(),
            B._itoi.tobytes(), B._shapes.tobytes(), B._offsets.tobytes(), tuple(c1), tuple(c2),
            C._itoi.tobytes(), C._shapes.tobytes(), C._offsets.tobytes(), A.rank(), B.rank())
@@ -728,9 +733,11 @@ def meta_elems(T: UniTensor) -> int:
     return int(np.sum(np.prod(T._shapes.astype(np.int64), axis=1))) if T.Nblocks() else 0
 
 
-def plan_contraction(A: UniTensor, B: UniTensor, C: UniTensor, c1, c2, dtype: int) -> "_Plan":
-    """Cached cxa_block_contract_plan for A x B -> C (metadata only)."""
-    return _plan_for(dtype, A, B, list(c1), list(c2), C)
+def plan_contraction(A: UniTensor, B: UniTensor, C: UniTensor, c1, c2, dtype: int,
+                     chain: bool = False) -> "_Plan":
+    """Cached cxa_block_contract_plan for A x B -> C (metadata only); ``chain`` for a step of a
+    matvec chain."""
+    return _plan_for(dtype, A, B, list(c1), list(c2), C, chain)
 
 
 def Contract(A, B=None, *args, **kwargs) -> UniTensor:

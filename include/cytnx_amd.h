@@ -186,6 +186,9 @@ int cxa_u1_enumerate_blocks(int rank, const int *btype, const int64_t *nq, const
  * (an exec inside a capture that would need the upload returns CXA_ERR_INVALID).
  */
 typedef struct cxa_bc_plan cxa_bc_plan;
+/* or'ed into the dtype of a plan that will be a step of a matvec chain: its tile list is made by
+ * cxa_chain_create (or its first exec) instead of at creation, with the tilings of chain steps. */
+#define CXA_PLAN_CHAIN 256
 int cxa_block_contract_plan(int dtype, int rankL, int nbL, const uint64_t *itoiL,
                             const uint64_t *shapeL, const int64_t *offL, int rankR, int nbR,
                             const uint64_t *itoiR, const uint64_t *shapeR, const int64_t *offR,
@@ -195,8 +198,9 @@ int cxa_block_contract_plan(int dtype, int rankL, int nbL, const uint64_t *itoiL
 /* flops: sum over block pairs of 2*M*N*K (x4 for complex); npairs: number of block pairs. */
 int cxa_block_contract_info(const cxa_bc_plan *plan, double *flops, int64_t *workspace_bytes,
                             int64_t *npairs);
-/* Override the tile shape of every tile (-1 = per-block default: MFMA 16x16..32x32 tiles,
- * row streaming for blocks with N <= 8) and the workgroup split-K mode (-1 automatic, 0 off,
+/* Override the tile shape of every tile (-1 = chosen from the blocks' sizes: MFMA 16x16..32x32
+ * wave tiles, row streaming for blocks with N <= 8, or 64x64 / 32x32 workgroup tiles staged
+ * through LDS, kinds 6 and 7) and the workgroup split-K mode (-1 automatic, 0 off,
  * 1 on with four waves per tile, 2 on with eight waves per tile for MFMA tiles); used by the
  * tuner.  get_config reports the split mode in the same 0 / 1 / 2 form. */
 int cxa_block_contract_set_tile(cxa_bc_plan *plan, int kind);
