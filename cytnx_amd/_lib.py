@@ -60,6 +60,9 @@ def _declare(L):
         "cxa_block_contract_plan": (ci, [ci, ci, ci, u64p, u64p, i64p, ci, ci, u64p, u64p, i64p,
                                          ci, u64p, u64p, ci, u64p, u64p, i64p,
                                          ctypes.POINTER(vp)]),
+        "cxa_block_contract_plan_out": (ci, [ci, ci, ci, u64p, u64p, i64p, ci, ci, u64p, u64p,
+                                             i64p, ci, u64p, u64p, ci, u64p, u64p, i64p, u64p,
+                                             ctypes.POINTER(vp)]),
         "cxa_block_contract_info": (ci, [vp, dblp, i64p, i64p]),
         "cxa_block_contract_set_tile": (ci, [vp, ci]),
         "cxa_block_contract_set_split": (ci, [vp, ci]),

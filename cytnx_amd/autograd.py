@@ -8,9 +8,8 @@ MFMA GEMM: for C = A . B over the common legs,
     dB = conj(A) . dC   over A's free legs,  written into B's blocks with axes (common ++ free),
 
 each one planned contraction (the operands are read through strides, conjugated on load for
-complex dtypes: ``cxa_block_contract_exec_ex``) followed by the inverse permute of every block
-into the caller's axis order.  The adjoint outputs use A's (B's) own block list and offsets, so
-the inverse permute lands directly in A's (B's) layout.  PyTorch's convention for complex
+complex dtypes: ``cxa_block_contract_exec_ex``) that writes every block in A's (B's) own axis
+order, block list and offsets (``cxa_block_contract_plan_out``).  PyTorch's convention for complex
 tensors holds: for a real loss, ``grad`` is the conjugate Wirtinger derivative, so
 dLoss = Re(sum(conj(grad) * dA)).
 
@@ -29,7 +28,7 @@ import torch
 from . import _lib
 from .device import stream_handle, torch_device
 from .unitensor import (CPU, PREC_FP64, TORCH_OF, UniTensor, _common, _plan_for, _Plan,
-                        _promote_pair, _scalar_block, block_permute_plan)
+                        _promote_pair, _scalar_block)
 
 
 def _permuted_meta(T: UniTensor, axes: Sequence[int]) -> UniTensor:
@@ -41,15 +40,6 @@ def _permuted_meta(T: UniTensor, axes: Sequence[int]) -> UniTensor:
     out._shapes = np.ascontiguousarray(T._shapes[:, list(axes)])
     out._storage = T._storage[:0]
     return out
-
-
-def _block_permute(src: torch.Tensor, meta: UniTensor, mapper: Sequence[int],
-                   dst: torch.Tensor) -> None:
-    """Every block of `src` (layout `meta`) permuted by `mapper` into the same offsets of dst."""
-    dt = {torch.float64: 3, torch.float32: 4, torch.complex128: 1, torch.complex64: 2}[src.dtype]
-    plan = block_permute_plan(dt, src.device.index, meta._shapes, meta._offsets, mapper)
-    _lib.check(_lib.lib().cxa_block_permute_exec(plan.handle, src.data_ptr(), dst.data_ptr(),
-                                                 stream_handle(src.device.index)))
 
 
 class _Spec:
@@ -70,16 +60,14 @@ class _Spec:
         # B's axis order); each B common leg stands for its A partner
         comm_by_b = sorted(range(len(c2)), key=lambda i: c2[i])
         pa = nc1 + [c1[i] for i in comm_by_b]
-        self.Ap = _permuted_meta(A, pa)
-        self.inv_a = [pa.index(j) for j in range(ra)]
-        self.ga = _plan_for(dt, out, B, [na + k for k in range(len(nc2))], nc2, self.Ap) \
+        self.ga = _plan_for(dt, out, B, [na + k for k in range(len(nc2))], nc2,
+                            _permuted_meta(A, pa), out_axes=[pa.index(j) for j in range(ra)]) \
             if nc2 else None
         # dB = A x dC over A's free legs -> (A common legs in A's axis order ++ B free)
         comm_by_a = sorted(range(len(c1)), key=lambda i: c1[i])
         pb = [c2[i] for i in comm_by_a] + nc2
-        self.Bp = _permuted_meta(B, pb)
-        self.inv_b = [pb.index(j) for j in range(rb)]
-        self.gb = _plan_for(dt, A, out, nc1, list(range(na)), self.Bp) if nc1 else None
+        self.gb = _plan_for(dt, A, out, nc1, list(range(na)), _permuted_meta(B, pb),
+                            out_axes=[pb.index(j) for j in range(rb)]) if nc1 else None
         self.A, self.B = A, B
 
     def exec(self, plan: _Plan, L: torch.Tensor, R: torch.Tensor, C: torch.Tensor,
@@ -127,21 +115,17 @@ class BlockContractFn(torch.autograd.Function):
         g = g.contiguous()
         ga = gb = None
         if ctx.needs_input_grad[0]:
-            tmp = torch.empty_like(a)
             if sp.ga is None:  # B has no free legs: dA = dC (scalar per A element) * conj(B)
                 raise NotImplementedError("adjoint of a contraction that consumes all of B")
-            sp.exec(sp.ga, g, b, tmp, 2)  # conj(B)
-            FLOPS["adjoint"] += sp.ga.flops
             ga = torch.empty_like(a)
-            _block_permute(tmp, sp.Ap, sp.inv_a, ga)
+            sp.exec(sp.ga, g, b, ga, 2)  # conj(B)
+            FLOPS["adjoint"] += sp.ga.flops
         if ctx.needs_input_grad[1]:
-            tmp = torch.empty_like(b)
             if sp.gb is None:
                 raise NotImplementedError("adjoint of a contraction that consumes all of A")
-            sp.exec(sp.gb, a, g, tmp, 1)  # conj(A)
-            FLOPS["adjoint"] += sp.gb.flops
             gb = torch.empty_like(b)
-            _block_permute(tmp, sp.Bp, sp.inv_b, gb)
+            sp.exec(sp.gb, a, g, gb, 1)  # conj(A)
+            FLOPS["adjoint"] += sp.gb.flops
         return ga, gb, None
 
 

@@ -92,13 +92,15 @@ struct cxa_bc_plan {
   PlanVariant var[3];  // indexed by CXA_PREC_*
   std::mutex mu;       // guards building a variant on first use
   bool copyA = false, copyB = false;
-  std::vector<cxa::CopyJob> jobsA, jobsB;  // blocks too large for the batched copy
-  // the other operand blocks, permuted into the workspace by one batched launch per operand
-  std::vector<cxa::BatchCopyJob> bjobsA, bjobsB;
-  std::vector<cxa::BatchCopyTask> btasksA, btasksB;
-  const cxa::BatchCopyJob *dev_bjobsA = nullptr, *dev_bjobsB = nullptr;
-  const cxa::BatchCopyTask *dev_btasksA = nullptr, *dev_btasksB = nullptr;
-  int64_t wsA = 0, wsB = 0;  // workspace elements for A and B copies
+  std::vector<cxa::CopyJob> jobsA, jobsB, jobsC;  // blocks too large for the batched copy
+  // the other operand (output) blocks, permuted into (out of) the workspace by one batched
+  // launch each
+  std::vector<cxa::BatchCopyJob> bjobsA, bjobsB, bjobsC;
+  std::vector<cxa::BatchCopyTask> btasksA, btasksB, btasksC;
+  const cxa::BatchCopyJob *dev_bjobsA = nullptr, *dev_bjobsB = nullptr, *dev_bjobsC = nullptr;
+  const cxa::BatchCopyTask *dev_btasksA = nullptr, *dev_btasksB = nullptr,
+                           *dev_btasksC = nullptr;
+  int64_t wsA = 0, wsB = 0, wsC = 0;  // workspace elements for A, B and C copies
   double flops = 0;
   int64_t npairs = 0;
   // mix plans (cxa_mix_contract_plan): blks are items, segs their slices, outs the outputs
@@ -106,6 +108,8 @@ struct cxa_bc_plan {
   std::vector<cxa::MixOut> outs;
   // a step of a matvec chain (bc_join_chain)
   bool chain = false;
+  // blks / segs describe the transposed products: their A operand is R's buffer, B is L's
+  bool swapped = false;
 };
 
 namespace cxa {
@@ -179,13 +183,15 @@ int upload_plan(cxa_bc_plan *p) {
     const void *src;
     size_t bytes, at;
   };
-  Part parts[7] = {{p->blks.data(), p->blks.size() * sizeof(GBlk), 0},
+  Part parts[9] = {{p->blks.data(), p->blks.size() * sizeof(GBlk), 0},
                    {p->segs.data(), p->segs.size() * sizeof(GSeg), 0},
                    {p->outs.data(), p->mix ? p->outs.size() * sizeof(MixOut) : 0, 0},
                    {p->bjobsA.data(), p->bjobsA.size() * sizeof(BatchCopyJob), 0},
                    {p->btasksA.data(), p->btasksA.size() * sizeof(BatchCopyTask), 0},
                    {p->bjobsB.data(), p->bjobsB.size() * sizeof(BatchCopyJob), 0},
-                   {p->btasksB.data(), p->btasksB.size() * sizeof(BatchCopyTask), 0}};
+                   {p->btasksB.data(), p->btasksB.size() * sizeof(BatchCopyTask), 0},
+                   {p->bjobsC.data(), p->bjobsC.size() * sizeof(BatchCopyJob), 0},
+                   {p->btasksC.data(), p->btasksC.size() * sizeof(BatchCopyTask), 0}};
   size_t total = 0;
   for (Part &q : parts) {
     q.at = total;
@@ -208,6 +214,8 @@ int upload_plan(cxa_bc_plan *p) {
     p->dev_btasksA = (const BatchCopyTask *)at(4);
     p->dev_bjobsB = (const BatchCopyJob *)at(5);
     p->dev_btasksB = (const BatchCopyTask *)at(6);
+    p->dev_bjobsC = (const BatchCopyJob *)at(7);
+    p->dev_btasksC = (const BatchCopyTask *)at(8);
   }
   if (p->chain) return CXA_OK;  // cxa_chain_create makes the tile list (bc_join_chain)
   return build_variant(p, native_prec(p->dtype));
@@ -293,16 +301,19 @@ using namespace cxa;
 // (src/BlockUniTensor.cpp:948-1228): left blocks in order, right blocks whose common-qindex
 // tuple matches (in order), target = the output block with itoi (L free ++ R free).  Each pair
 // becomes one GEMM segment of its target block: M = prod(L free dims), K = prod(common dims),
-// N = prod(R free dims).  Operands are read through strides when the permuted block is still a
-// strided matrix; otherwise the plan copies the operand blocks to the workspace first.
+// N = prod(R free dims).  Operands are read (and a permuted output is written) through strides:
+// the axes of an index whose strides do not merge are taken apart into several blocks or
+// segments; only where those would be many or short are operand blocks copied to the workspace
+// first.
 // ------------------------------------------------------------------------------------------
-extern "C" int cxa_block_contract_plan(int dtype, int rankL, int nbL, const uint64_t *itoiL,
-                                       const uint64_t *shapeL, const int64_t *offL, int rankR,
-                                       int nbR, const uint64_t *itoiR, const uint64_t *shapeR,
-                                       const int64_t *offR, int ncomm, const uint64_t *comm1,
-                                       const uint64_t *comm2, int nbC, const uint64_t *itoiC,
-                                       const uint64_t *shapeC, const int64_t *offC,
-                                       cxa_bc_plan **out) {
+namespace {
+
+int make_block_plan(int dtype, int rankL, int nbL, const uint64_t *itoiL, const uint64_t *shapeL,
+                    const int64_t *offL, int rankR, int nbR, const uint64_t *itoiR,
+                    const uint64_t *shapeR, const int64_t *offR, int ncomm,
+                    const uint64_t *comm1, const uint64_t *comm2, int nbC, const uint64_t *itoiC,
+                    const uint64_t *shapeC, const int64_t *offC, const uint64_t *out_axes,
+                    cxa_bc_plan **out) {
   CXA_CHECK(out, CXA_ERR_INVALID, "cxa_block_contract_plan: null output handle");
   *out = nullptr;
   const bool chain = (dtype & CXA_PLAN_CHAIN) != 0;
@@ -383,31 +394,177 @@ extern "C" int cxa_block_contract_plan(int dtype, int rankL, int nbL, const uint
   }
   p->npairs = (int64_t)pairs.size();
 
-  // can every operand be read in place?
+  // Row-major strides of an array with `rank` extents.
+  auto strides_of = [](int rank, const uint64_t *ext, int64_t *st) {
+    int64_t acc = 1;
+    for (int i = rank - 1; i >= 0; --i) {
+      st[i] = acc;
+      acc *= (int64_t)ext[i];
+    }
+  };
+  // Axis order of the GEMM operands (free ++ common, common ++ free), the operands' strides per
+  // axis in that order, and those of the output: out_axes permutes the stored axes.
   int axA[32], axB[32];
   for (int i = 0; i < n1; ++i) axA[i] = nc1[i];
   for (int c = 0; c < ncomm; ++c) axA[n1 + c] = (int)comm1[c];
   for (int c = 0; c < ncomm; ++c) axB[c] = (int)comm2[c];
   for (int i = 0; i < n2; ++i) axB[ncomm + i] = nc2[i];
-  std::vector<int64_t> sam(nbL), sak(nbL), sbk(nbR), sbn(nbR);
   std::vector<char> usedA(nbL, 0), usedB(nbR, 0);
   for (const Pair &pr : pairs) {
     usedA[pr.a] = 1;
     usedB[pr.b] = 1;
   }
-  for (int a = 0; a < nbL; ++a) {
-    if (!usedA[a]) continue;
-    const uint64_t *sa = shapeL + (int64_t)a * rankL;
-    if (!merged_stride(rankL, sa, axA, n1, &sam[a]) ||
-        !merged_stride(rankL, sa, axA + n1, ncomm, &sak[a]))
-      p->copyA = true;
+  std::vector<int64_t> stA((size_t)nbL * 16, 0), stB((size_t)nbR * 16, 0), stC((size_t)nbC * 32, 0);
+  for (int b = 0; b < nbL; ++b) {
+    int64_t st[16];
+    strides_of(rankL, shapeL + (int64_t)b * rankL, st);
+    for (int i = 0; i < rankL; ++i) stA[(size_t)b * 16 + i] = st[axA[i]];
   }
   for (int b = 0; b < nbR; ++b) {
-    if (!usedB[b]) continue;
-    const uint64_t *sb = shapeR + (int64_t)b * rankR;
-    if (!merged_stride(rankR, sb, axB, ncomm, &sbk[b]) ||
-        !merged_stride(rankR, sb, axB + ncomm, n2, &sbn[b]))
-      p->copyB = true;
+    int64_t st[16];
+    strides_of(rankR, shapeR + (int64_t)b * rankR, st);
+    for (int i = 0; i < rankR; ++i) stB[(size_t)b * 16 + i] = st[axB[i]];
+  }
+  for (int b = 0; b < nbC; ++b) {
+    uint64_t ext[32];
+    int64_t st[32];
+    for (int i = 0; i < rankC; ++i)
+      ext[i] = shapeC[(int64_t)b * rankC + (out_axes ? (int)out_axes[i] : i)];
+    strides_of(rankC, ext, st);
+    for (int i = 0; i < rankC; ++i)
+      stC[(size_t)b * 32 + (out_axes ? (int)out_axes[i] : i)] = st[i];
+  }
+  std::vector<std::vector<int>> by_target(nbC);
+  for (size_t i = 0; i < pairs.size(); ++i) by_target[pairs[i].t].push_back((int)i);
+
+  // One index of a GEMM that the strides of several axes do not merge into: runs of axes [at, at
+  // + n) that do, the longest of which becomes the GEMM index while the others are taken apart
+  // (rows and columns into blocks of their own, K into segments).
+  struct Run {
+    int at, n;
+    int64_t ext;
+  };
+  struct Runs {
+    Run r[16];
+    int n = 0, main = 0;
+    int64_t split = 1;  // product of the extents taken apart
+  };
+  auto runs_of = [](int n, const uint64_t *ext, auto merges) {
+    Runs R;
+    int prev = -1;
+    for (int i = 0; i < n; ++i) {
+      if (ext[i] == 1) continue;
+      if (prev >= 0 && merges(prev, i)) {
+        R.r[R.n - 1].n = i - R.r[R.n - 1].at + 1;
+        R.r[R.n - 1].ext *= (int64_t)ext[i];
+      } else {
+        R.r[R.n++] = Run{i, 1, (int64_t)ext[i]};
+      }
+      prev = i;
+    }
+    if (R.n == 0) R.r[R.n++] = Run{0, 0, 1};
+    for (int q = 1; q < R.n; ++q)
+      if (R.r[q].ext >= R.r[R.main].ext) R.main = q;
+    for (int q = 0; q < R.n; ++q)
+      if (q != R.main) R.split *= R.r[q].ext;
+    return R;
+  };
+  auto runs_m = [&](int t) {
+    const uint64_t *sc = shapeC + (int64_t)t * rankC;
+    return runs_of(n1, sc, [&, t](int i, int j) {
+      if (stC[(size_t)t * 32 + i] != (int64_t)sc[j] * stC[(size_t)t * 32 + j]) return false;
+      for (int pi : by_target[t]) {
+        const int64_t *st = &stA[(size_t)pairs[pi].a * 16];
+        if (st[i] != (int64_t)sc[j] * st[j]) return false;
+      }
+      return true;
+    });
+  };
+  auto runs_n = [&](int t) {
+    const uint64_t *sc = shapeC + (int64_t)t * rankC + n1;
+    return runs_of(n2, sc, [&, t](int i, int j) {
+      if (stC[(size_t)t * 32 + n1 + i] != (int64_t)sc[j] * stC[(size_t)t * 32 + n1 + j])
+        return false;
+      for (int pi : by_target[t]) {
+        const int64_t *st = &stB[(size_t)pairs[pi].b * 16] + ncomm;
+        if (st[i] != (int64_t)sc[j] * st[j]) return false;
+      }
+      return true;
+    });
+  };
+  auto runs_k = [&](const Pair &pr) {
+    uint64_t ext[16];
+    for (int c = 0; c < ncomm; ++c) ext[c] = shapeL[(int64_t)pr.a * rankL + comm1[c]];
+    const int64_t *sa = &stA[(size_t)pr.a * 16] + n1, *sb = &stB[(size_t)pr.b * 16];
+    return runs_of(ncomm, ext, [&, sa, sb](int i, int j) {
+      return sa[i] == (int64_t)ext[j] * sa[j] && sb[i] == (int64_t)ext[j] * sb[j];
+    });
+  };
+
+  // Operands are read in place, and a permuted output is written in place, where taking indices
+  // apart costs little: the work on whole 16 x 16 x 16 tiles grows by at most half (or stays
+  // within a few tiles per CU) and the lists stay short.  Otherwise the operand blocks that are
+  // no strided matrix are permuted into the workspace first, and the output from it afterwards.
+  // (First contraction of an environment update at chi = 2048, three MPO states taken apart:
+  // 103 us with the copies, of which 58 us are 18 permute launches, 39 us in place.  Gradient of
+  // a 32-site MPS energy, chi = 512, complex: 11.5 -> 8.8 ms, 286 permutes of adjoints fewer.)
+  // Real steps of chains keep their copies, and with them the order of their K.
+  auto worth = [&]() {
+    auto pad = [](int64_t x) { return (double)((x + 15) / 16 * 16); };
+    double cost = 0.0, whole = 0.0;
+    int64_t nblk = 0, nseg = 0;
+    for (int t = 0; t < nbC; ++t) {
+      const Runs rm = runs_m(t), rn = runs_n(t);
+      const int64_t mn = rm.split * rn.split;
+      nblk += mn;
+      for (int pi : by_target[t]) {
+        const Pair &pr = pairs[pi];
+        const Runs rk = runs_k(pr);
+        nseg += mn * rk.split;
+        cost += (double)mn * (double)rk.split * pad(rm.r[rm.main].ext) *
+                pad(rn.r[rn.main].ext) * pad(rk.r[rk.main].ext);
+        whole += pad(pr.M) * pad(pr.N) * pad(pr.K);
+      }
+    }
+    return cost <= 1.5 * whole + 4194304.0 && nblk <= 16 * (int64_t)nbC + 64 &&
+           nseg <= 16 * (int64_t)pairs.size() + 64;
+  };
+  std::vector<int64_t> offT(offC, offC + nbC);  // where the products' output blocks go
+  bool in_place = !(p->chain && !is_complex(dtype)) && worth();
+  std::vector<CopyJob> copiesC;
+  if (!in_place && out_axes && rankC <= 16) {
+    for (int t = 0; t < nbC; ++t) {
+      const uint64_t *sc = shapeC + (int64_t)t * rankC;
+      CopyJob j{};
+      int64_t n = 1;
+      for (int i = 0; i < rankC; ++i) {
+        j.shape[i] = sc[i];
+        j.mapper[i] = out_axes[i];
+        n *= (int64_t)sc[i];
+      }
+      j.rank = rankC;
+      j.src_off = offT[t] = p->wsC;
+      j.dst_off = offC[t];
+      p->wsC += (n + 15) / 16 * 16;
+      strides_of(rankC, sc, &stC[(size_t)t * 32]);
+      copiesC.push_back(j);
+    }
+    in_place = worth();
+  }
+  if (!in_place) {
+    int64_t st;
+    for (int a = 0; a < nbL; ++a) {
+      const uint64_t *sa = shapeL + (int64_t)a * rankL;
+      if (usedA[a] && (!merged_stride(rankL, sa, axA, n1, &st) ||
+                       !merged_stride(rankL, sa, axA + n1, ncomm, &st)))
+        p->copyA = true;
+    }
+    for (int b = 0; b < nbR; ++b) {
+      const uint64_t *sb = shapeR + (int64_t)b * rankR;
+      if (usedB[b] && (!merged_stride(rankR, sb, axB, ncomm, &st) ||
+                       !merged_stride(rankR, sb, axB + ncomm, n2, &st)))
+        p->copyB = true;
+    }
   }
   std::vector<int64_t> wsoffA(nbL, 0), wsoffB(nbR, 0);
   std::vector<CopyJob> copiesA, copiesB;
@@ -419,20 +576,18 @@ extern "C" int cxa_block_contract_plan(int dtype, int rankL, int nbL, const uint
       j.src_off = offL[a];
       j.dst_off = p->wsA;
       j.rank = rankL;
-      int64_t M = 1, K = 1, n = 1;
+      int64_t n = 1;
+      uint64_t ext[16];
       for (int i = 0; i < rankL; ++i) {
         j.shape[i] = sa[i];
         j.mapper[i] = (uint64_t)axA[i];
+        ext[i] = sa[axA[i]];
         n *= (int64_t)sa[i];
       }
-      for (int i = 0; i < n1; ++i) M *= (int64_t)sa[nc1[i]];
-      for (int c = 0; c < ncomm; ++c) K *= (int64_t)sa[comm1[c]];
+      strides_of(rankL, ext, &stA[(size_t)a * 16]);
       wsoffA[a] = p->wsA;
-      sam[a] = K;
-      sak[a] = 1;
       p->wsA += (n + 15) / 16 * 16;
       copiesA.push_back(j);
-      (void)M;
     }
   }
   if (p->copyB) {
@@ -443,16 +598,16 @@ extern "C" int cxa_block_contract_plan(int dtype, int rankL, int nbL, const uint
       j.src_off = offR[b];
       j.dst_off = p->wsB;
       j.rank = rankR;
-      int64_t N = 1, n = 1;
+      int64_t n = 1;
+      uint64_t ext[16];
       for (int i = 0; i < rankR; ++i) {
         j.shape[i] = sb[i];
         j.mapper[i] = (uint64_t)axB[i];
+        ext[i] = sb[axB[i]];
         n *= (int64_t)sb[i];
       }
-      for (int i = 0; i < n2; ++i) N *= (int64_t)sb[nc2[i]];
+      strides_of(rankR, ext, &stB[(size_t)b * 16]);
       wsoffB[b] = p->wsB;
-      sbk[b] = N;
-      sbn[b] = 1;
       p->wsB += (n + 15) / 16 * 16;
       copiesB.push_back(j);
     }
@@ -460,50 +615,149 @@ extern "C" int cxa_block_contract_plan(int dtype, int rankL, int nbL, const uint
 
   split_copies(copiesA, p->jobsA, p->bjobsA, p->btasksA);
   split_copies(copiesB, p->jobsB, p->bjobsB, p->btasksB);
+  split_copies(copiesC, p->jobsC, p->bjobsC, p->btasksC);
 
-  // one GBlk per output block, segments grouped by target in pair order
-  std::vector<std::vector<int>> by_target(nbC);
-  for (size_t i = 0; i < pairs.size(); ++i) by_target[pairs[i].t].push_back((int)i);
-  p->blks.resize(nbC);
+  // The products: one GBlk per output block and combination of the row and column indices taken
+  // apart, its segments in pair order.  A block whose rows are the contiguous ones of C (a
+  // permuted output) is better computed transposed, with the operands' roles exchanged: done for
+  // the plan as a whole when more of its output is of that kind.
   const double cplx = is_complex(dtype) ? 4.0 : 1.0;
+  int64_t rows_unit = 0, cols_unit = 0;  // output elements whose m or n is C's unit stride
+  p->blks.reserve(nbC);
   for (int t = 0; t < nbC; ++t) {
-    GBlk &g = p->blks[t];
     const uint64_t *sc = shapeC + (int64_t)t * rankC;
     int64_t M = 1, N = 1;
     for (int i = 0; i < n1; ++i) M *= (int64_t)sc[i];
     for (int i = 0; i < n2; ++i) N *= (int64_t)sc[n1 + i];
     CXA_CHECK(M <= INT32_MAX && N <= INT32_MAX, CXA_ERR_UNSUPPORTED,
               "block contract: output block too large");
-    g.c_off = offC[t];
-    g.ldc = N;
-    g.alpha = 1.0;
-    g.beta = 0.0;
-    g.M = (int32_t)M;
-    g.N = (int32_t)N;
-    g.seg0 = (int32_t)p->segs.size();
-    g.nseg = (int32_t)by_target[t].size();
     for (int pi : by_target[t]) {
       const Pair &pr = pairs[pi];
       CXA_CHECK(pr.M == M && pr.N == N, CXA_ERR_INVALID,
                 "block contract: output block %d shape does not match its pair (%lld x %lld)", t,
                 (long long)pr.M, (long long)pr.N);
       CXA_CHECK(pr.K <= INT32_MAX, CXA_ERR_UNSUPPORTED, "block contract: K too large");
-      GSeg s{};
-      s.a_off = p->copyA ? wsoffA[pr.a] : offL[pr.a];
-      s.b_off = p->copyB ? wsoffB[pr.b] : offR[pr.b];
-      s.sam = sam[pr.a];
-      s.sak = sak[pr.a];
-      s.sbk = sbk[pr.b];
-      s.sbn = sbn[pr.b];
-      s.K = (int32_t)pr.K;
-      p->segs.push_back(s);
       p->flops += 2.0 * cplx * (double)pr.M * (double)pr.N * (double)pr.K;
+    }
+    const Runs rm = runs_m(t), rn = runs_n(t);
+    const Run &mr = rm.r[rm.main], &nr = rn.r[rn.main];
+    const int64_t *sC = &stC[(size_t)t * 32];
+    // stride of a run in a per-axis table (its innermost axis); 0 for a run without axes
+    auto run_stride = [](const int64_t *st, const Run &r) { return r.n ? st[r.at + r.n - 1] : 0; };
+    for (int64_t sm = 0; sm < rm.split; ++sm) {
+      for (int64_t sn = 0; sn < rn.split; ++sn) {
+        GBlk g{};
+        g.ldc = run_stride(sC, mr);
+        g.csn = run_stride(sC + n1, nr);
+        if (!mr.n) g.ldc = N;
+        if (!nr.n) g.csn = 1;
+        g.alpha = 1.0;
+        g.beta = 0.0;
+        g.M = (int32_t)mr.ext;
+        g.N = (int32_t)nr.ext;
+        g.c_off = offT[t];
+        // the indices of the runs taken apart (innermost run fastest)
+        int64_t idm[16] = {0}, idn[16] = {0}, x = sm;
+        for (int q = rm.n - 1; q >= 0; --q)
+          if (q != rm.main) {
+            idm[q] = x % rm.r[q].ext;
+            x /= rm.r[q].ext;
+            g.c_off += idm[q] * run_stride(sC, rm.r[q]);
+          }
+        x = sn;
+        for (int q = rn.n - 1; q >= 0; --q)
+          if (q != rn.main) {
+            idn[q] = x % rn.r[q].ext;
+            x /= rn.r[q].ext;
+            g.c_off += idn[q] * run_stride(sC + n1, rn.r[q]);
+          }
+        g.seg0 = (int32_t)p->segs.size();
+        for (int pi : by_target[t]) {
+          const Pair &pr = pairs[pi];
+          const int64_t *sA = &stA[(size_t)pr.a * 16], *sB = &stB[(size_t)pr.b * 16];
+          const Runs rk = runs_k(pr);
+          const Run &kr = rk.r[rk.main];
+          GSeg s{};
+          s.a_off = p->copyA ? wsoffA[pr.a] : offL[pr.a];
+          s.b_off = p->copyB ? wsoffB[pr.b] : offR[pr.b];
+          for (int q = 0; q < rm.n; ++q) s.a_off += idm[q] * run_stride(sA, rm.r[q]);
+          for (int q = 0; q < rn.n; ++q) s.b_off += idn[q] * run_stride(sB + ncomm, rn.r[q]);
+          s.sam = run_stride(sA, mr);
+          s.sak = run_stride(sA + n1, kr);
+          s.sbk = run_stride(sB, kr);
+          s.sbn = run_stride(sB + ncomm, nr);
+          s.K = (int32_t)kr.ext;
+          for (int64_t sk = 0; sk < rk.split; ++sk) {
+            GSeg e = s;
+            x = sk;
+            for (int q = rk.n - 1; q >= 0; --q)
+              if (q != rk.main) {
+                const int64_t i = x % rk.r[q].ext;
+                x /= rk.r[q].ext;
+                e.a_off += i * run_stride(sA + n1, rk.r[q]);
+                e.b_off += i * run_stride(sB, rk.r[q]);
+              }
+            p->segs.push_back(e);
+          }
+        }
+        g.nseg = (int32_t)((int64_t)p->segs.size() - g.seg0);
+        if (g.csn == 1)
+          cols_unit += (int64_t)g.M * g.N;
+        else if (g.ldc == 1)
+          rows_unit += (int64_t)g.M * g.N;
+        p->blks.push_back(g);
+      }
+    }
+  }
+  if (rows_unit > cols_unit) {
+    p->swapped = true;
+    for (GBlk &g : p->blks) {
+      std::swap(g.M, g.N);
+      std::swap(g.ldc, g.csn);
+    }
+    for (GSeg &s : p->segs) {
+      std::swap(s.a_off, s.b_off);
+      std::swap(s.sam, s.sbn);
+      std::swap(s.sak, s.sbk);
     }
   }
   int rc = upload_plan(p.get());
   if (rc) return rc;
   *out = p.release();
   return CXA_OK;
+}
+
+}  // namespace
+
+extern "C" int cxa_block_contract_plan(int dtype, int rankL, int nbL, const uint64_t *itoiL,
+                                       const uint64_t *shapeL, const int64_t *offL, int rankR,
+                                       int nbR, const uint64_t *itoiR, const uint64_t *shapeR,
+                                       const int64_t *offR, int ncomm, const uint64_t *comm1,
+                                       const uint64_t *comm2, int nbC, const uint64_t *itoiC,
+                                       const uint64_t *shapeC, const int64_t *offC,
+                                       cxa_bc_plan **out) {
+  return make_block_plan(dtype, rankL, nbL, itoiL, shapeL, offL, rankR, nbR, itoiR, shapeR, offR,
+                         ncomm, comm1, comm2, nbC, itoiC, shapeC, offC, nullptr, out);
+}
+
+extern "C" int cxa_block_contract_plan_out(
+    int dtype, int rankL, int nbL, const uint64_t *itoiL, const uint64_t *shapeL,
+    const int64_t *offL, int rankR, int nbR, const uint64_t *itoiR, const uint64_t *shapeR,
+    const int64_t *offR, int ncomm, const uint64_t *comm1, const uint64_t *comm2, int nbC,
+    const uint64_t *itoiC, const uint64_t *shapeC, const int64_t *offC, const uint64_t *out_axes,
+    cxa_bc_plan **out) {
+  const int rankC = rankL + rankR - 2 * ncomm;
+  bool seen[32] = {false};
+  CXA_CHECK(rankC >= 0 && rankC <= 32 && (rankC == 0 || out_axes), CXA_ERR_INVALID,
+            "cxa_block_contract_plan_out: bad output axes");
+  for (int i = 0; i < rankC; ++i) {
+    CXA_CHECK(out_axes[i] < (uint64_t)rankC && !seen[out_axes[i]], CXA_ERR_INVALID,
+              "cxa_block_contract_plan_out: the output axes are not a permutation");
+    seen[out_axes[i]] = true;
+  }
+  return make_block_plan(dtype, rankL, nbL, itoiL, shapeL, offL, rankR, nbR, itoiR, shapeR, offR,
+                         ncomm, comm1, comm2, nbC, itoiC, shapeC, offC, rankC ? out_axes : nullptr,
+                         out);
 }
 
 // ------------------------------------------------------------------------------------------
@@ -643,7 +897,7 @@ extern "C" int cxa_block_contract_info(const cxa_bc_plan *p, double *flops,
                                        int64_t *workspace_bytes, int64_t *npairs) {
   CXA_CHECK(p, CXA_ERR_INVALID, "cxa_block_contract_info: null plan");
   if (flops) *flops = p->flops;
-  if (workspace_bytes) *workspace_bytes = (p->wsA + p->wsB) * p->es;
+  if (workspace_bytes) *workspace_bytes = (p->wsA + p->wsB + p->wsC) * p->es;
   if (npairs) *npairs = p->npairs;
   return CXA_OK;
 }
@@ -715,9 +969,10 @@ int bc_exec_typed(const cxa_bc_plan *p, const void *L, const void *R, void *C, i
   CXA_CHECK(!lay->c_k4 || (p->mix && lay->outs), CXA_ERR_INVALID,
             "block contract exec: packed outputs need a mix plan and its packed outputs");
   CXA_CHECK(p, CXA_ERR_INVALID, "block contract exec: null plan");
-  CXA_CHECK(!(p->copyA || p->copyB) || workspace, CXA_ERR_INVALID,
+  const int64_t ws_elems = p->wsA + p->wsB + p->wsC;
+  CXA_CHECK(ws_elems == 0 || workspace, CXA_ERR_INVALID,
             "block contract exec: this plan needs a workspace of %lld bytes",
-            (long long)((p->wsA + p->wsB) * 16));
+            (long long)(ws_elems * 16));
   const int esA = elem_size(a_dt), esB = elem_size(b_dt);
   char *ws = (char *)workspace;
   for (const CopyJob &j : p->jobsA) {
@@ -752,6 +1007,11 @@ int bc_exec_typed(const cxa_bc_plan *p, const void *L, const void *R, void *C, i
   g.A = p->copyA ? (const void *)ws : L;
   g.B = p->copyB ? (const void *)wsB : R;
   g.C = C;
+  if (p->swapped) {
+    std::swap(g.A, g.B);
+    std::swap(g.a_dt, g.b_dt);
+    conj = (conj & 1) << 1 | (conj & 2) >> 1;
+  }
   int rc = bc_ensure(p, prec_eff, s);
   if (rc) return rc;
   const PlanVariant &v = p->var[prec_eff];
@@ -770,7 +1030,19 @@ int bc_exec_typed(const cxa_bc_plan *p, const void *L, const void *R, void *C, i
   g.dot_part = lay->dot_part;
   g.kind0 = v.launch_kind;
   if (p->mix) g.outs = lay->outs ? lay->outs : p->dev_outs;
-  return launch_grouped_gemm(g, s);
+  if (!p->wsC) return launch_grouped_gemm(g, s);
+  const int esC = elem_size(c_dt);
+  char *wsC = wsB + p->wsB * esB;
+  g.C = wsC;
+  rc = launch_grouped_gemm(g, s);
+  if (rc) return rc;
+  for (const CopyJob &j : p->jobsC) {
+    rc = cxa_permute(c_dt, j.rank, j.shape, j.mapper, wsC + j.src_off * esC,
+                     (char *)C + j.dst_off * esC, s);
+    if (rc) return rc;
+  }
+  if (p->btasksC.empty()) return CXA_OK;
+  return launch_batch_copy(esC, p->dev_bjobsC, p->dev_btasksC, (int)p->btasksC.size(), wsC, C, s);
 }
 
 namespace {
@@ -782,7 +1054,7 @@ int pack_views(const cxa_bc_plan *p, int which, int64_t elems, std::vector<GSeg>
   CXA_CHECK(p && packed_elems, CXA_ERR_INVALID, "pack views: bad arguments");
   if (segs.empty()) segs = p->segs;
   CXA_CHECK(segs.size() == p->segs.size(), CXA_ERR_INVALID, "pack views: segment count");
-  if ((which == 0 ? p->copyA : p->copyB) || is_complex(p->dtype))
+  if ((which == 0 ? p->copyA : p->copyB) || is_complex(p->dtype) || p->swapped)
     return fail(CXA_ERR_UNSUPPORTED, "pack views: operand permuted into a workspace or complex");
   regions.clear();
   std::map<std::array<int64_t, 5>, int64_t> at;  // view -> packed offset
@@ -873,10 +1145,13 @@ int bc_mix_pack_outs(const cxa_bc_plan *mix, const std::vector<PackRegion> &regi
 }
 
 bool bc_is_mix(const cxa_bc_plan *p) { return p->mix; }
-int64_t bc_workspace_elems(const cxa_bc_plan *p) { return p->wsA + p->wsB; }
+int64_t bc_workspace_elems(const cxa_bc_plan *p) { return p->wsA + p->wsB + p->wsC; }
 
 int bc_dot_slots(const cxa_bc_plan *p, int prec) {
   if (!p || p->mix || is_complex(p->dtype) || prec < 0 || prec > CXA_PREC_FP32X3) return 0;
+  if (p->wsC) return 0;  // the epilogue takes the output in place, unit-stride along n
+  for (const GBlk &b : p->blks)
+    if (b.csn != 1) return 0;
   if (bc_ensure(p, prec, nullptr)) return 0;
   const PlanVariant &v = p->var[prec];
   if (v.tile_class == 1 || v.ntiles == 0) return 0;  // make_tiles' row-streaming class
@@ -940,7 +1215,7 @@ extern "C" int cxa_matmul(int dtype, void *out, const void *inl, const void *inr
   g.A = inl;
   g.B = inr;
   g.C = out;
-  g.blk0 = GBlk{0, Nr, 1.0, 0.0, (int32_t)Ml, (int32_t)Nr, 0, Comm > 0 ? 1 : 0};
+  g.blk0 = GBlk{0, Nr, 1, 1.0, 0.0, (int32_t)Ml, (int32_t)Nr, 0, Comm > 0 ? 1 : 0};
   g.seg0 = GSeg{0, 0, Comm, 1, Nr, 1, (int32_t)Comm, 0};
   return launch_grouped_gemm(g, (hipStream_t)stream);
 }
@@ -1169,7 +1444,7 @@ extern "C" int cxa_tensordot(int dtype, void *out, const void *L, int rankL,
   g.A = A;
   g.B = B;
   g.C = out;
-  g.blk0 = GBlk{0, N, 1.0, 0.0, (int32_t)M, (int32_t)N, 0, K > 0 ? 1 : 0};
+  g.blk0 = GBlk{0, N, 1, 1.0, 0.0, (int32_t)M, (int32_t)N, 0, K > 0 ? 1 : 0};
   g.seg0 = GSeg{0, 0, sam, sak, sbk, sbn, (int32_t)K, 0};
   return launch_grouped_gemm(g, (hipStream_t)stream);
 }

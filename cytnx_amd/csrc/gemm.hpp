@@ -27,7 +27,8 @@ struct GSeg {
 
 struct GBlk {
   int64_t c_off;  // element offset of C[0,0] from the C base pointer
-  int64_t ldc;    // element stride of C along m (C is unit-stride along n)
+  int64_t ldc;    // element stride of C along m
+  int64_t csn = 1;  // and along n (1 in mix items, and in launches with a dot-product epilogue)
   double alpha, beta;
   int32_t M, N;
   int32_t seg0, nseg;

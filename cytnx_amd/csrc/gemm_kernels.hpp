@@ -486,7 +486,8 @@ __device__ __forceinline__ void wave_tile_real(const char *__restrict__ Abase,
         const int row = 16 * i + acc_row(RealAcc<PREC, MI, NI>::F64, g, v);
         const int col = 16 * jj + r;
         if (row < mt && col < nt)
-          store_c(Cp + (int64_t)(m0 + row) * blk.ldc + (n0 + col), acc.get(i, jj, v), blk);
+          store_c(Cp + (int64_t)(m0 + row) * blk.ldc + (n0 + col) * blk.csn, acc.get(i, jj, v),
+                  blk);
       }
   if (dslot) {  // uniform over the wave; only launches with an FP64 C and alpha 1, beta 0
     double cx = 0.0, xx = 0.0;
@@ -578,7 +579,7 @@ __device__ __forceinline__ void wg_tile_real(const char *__restrict__ Abase,
       double s = red[0][idx][lane];
 #pragma unroll
       for (int q = 1; q < WAVES; ++q) s += red[q][idx][lane];
-      store_c(Cp + (int64_t)(m0 + row) * blk.ldc + (n0 + col), s, blk);
+      store_c(Cp + (int64_t)(m0 + row) * blk.ldc + (n0 + col) * blk.csn, s, blk);
       cx += s * xpre[t];
       xx += xpre[t] * xpre[t];
     }
@@ -702,7 +703,7 @@ __device__ __forceinline__ void wave_rows(const char *__restrict__ Abase,
   gptr<TC> Cp = at<TC>(Cbase, blk.c_off) + (int64_t)row * blk.ldc;
 #pragma unroll
   for (int n = 0; n < kRowsN; ++n)
-    if (n < blk.N) store_c(Cp + n, acc[n], blk);
+    if (n < blk.N) store_c(Cp + n * blk.csn, acc[n], blk);
 }
 
 // Split-K row tile: the four waves take interleaved k values of the same 64 rows.
@@ -723,8 +724,8 @@ __device__ __forceinline__ void wg_rows(const char *__restrict__ Abase,
 #pragma unroll
     for (int n = 0; n < kRowsN; ++n)
       if (n < blk.N)
-        store_c(Cp + n, ((red[0][n][lane] + red[1][n][lane]) + red[2][n][lane]) + red[3][n][lane],
-                blk);
+        store_c(Cp + n * blk.csn,
+                ((red[0][n][lane] + red[1][n][lane]) + red[2][n][lane]) + red[3][n][lane], blk);
   }
   __syncthreads();
 }
@@ -774,7 +775,7 @@ __device__ __forceinline__ void wave_tile_cplx(const char *__restrict__ Abase,
         const int row = 16 * i + acc_row(CplxAcc<op_t, MI, NI>::F64, g, v);
         const int col = 16 * jj + r;
         if (row < mt && col < nt)
-          store_cplx<op_t>(Cp + ((int64_t)(m0 + row) * blk.ldc + (n0 + col)),
+          store_cplx<op_t>(Cp + ((int64_t)(m0 + row) * blk.ldc + (n0 + col) * blk.csn),
                            (double)acc.re[i][jj][v], (double)acc.im[i][jj][v], blk);
       }
 }
@@ -813,8 +814,9 @@ __device__ __forceinline__ void wg_tile_cplx(const char *__restrict__ Abase,
         re += (double)red[q][wave][lane];
         im += (double)red[q][4 + wave][lane];
       }
-      store_cplx<op_t>(at<c2>(Cbase, blk.c_off) + ((int64_t)(m0 + row) * blk.ldc + (n0 + r)), re,
-                       im, blk);
+      store_cplx<op_t>(
+          at<c2>(Cbase, blk.c_off) + ((int64_t)(m0 + row) * blk.ldc + (n0 + r) * blk.csn), re, im,
+          blk);
     }
   }
   __syncthreads();

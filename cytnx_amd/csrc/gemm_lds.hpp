@@ -393,7 +393,7 @@ __device__ __forceinline__ void wg_tile_lds(char *smem, const char *__restrict__
       for (int v = 0; v < 4; ++v) {
         const int row = 16 * i + acc_row(F64, g, v), col = 16 * jj + r;
         if (row >= mw || col >= nw) continue;
-        const int64_t e = (int64_t)(m0 + wm + row) * blk.ldc + (n0 + wn + col);
+        const int64_t e = (int64_t)(m0 + wm + row) * blk.ldc + (n0 + wn + col) * blk.csn;
         if constexpr (CPLX) {
           store_cplx<op_t>(at<typename EA::g>(Cbase, blk.c_off) + e, (double)acc[0][i][jj][v],
                            (double)aci[i][jj][v], blk);

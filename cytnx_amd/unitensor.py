@@ -146,19 +146,24 @@ PLAN_CHAIN = 256  # CXA_PLAN_CHAIN
 
 
 def _plan_for(dtype: int, A: "UniTensor", B: "UniTensor", c1: List[int], c2: List[int],
-              C: "UniTensor", chain: bool = False) -> _Plan:
+              C: "UniTensor", chain: bool = False,
+              out_axes: Optional[Sequence[int]] = None) -> _Plan:
+    """The (cached) plan of A x B -> C; with ``out_axes`` axis j of every stored output block is
+    axis out_axes[j] of C."""
     if chain:
         dtype |= PLAN_CHAIN
+    out_axes = None if out_axes is None else tuple(int(x) for x in out_axes)
     key = (dtype, A.device(), A._itoi.tobytes(), A._shapes.tobytes(), A._offsets.tobytes(),
            B._itoi.tobytes(), B._shapes.tobytes(), B._offsets.tobytes(), tuple(c1), tuple(c2),
-           C._itoi.tobytes(), C._shapes.tobytes(), C._offsets.tobytes(), A.rank(), B.rank())
+           C._itoi.tobytes(), C._shapes.tobytes(), C._offsets.tobytes(), A.rank(), B.rank(),
+           out_axes)
     p = _PLAN_CACHE.get(key)
     if p is not None:
         return p
     L = _lib.lib()
     h = ctypes.c_void_p(0)
     torch.cuda.set_device(A.device())
-    _lib.check(L.cxa_block_contract_plan(
+    args = (
         dtype,
         A.rank(), A.Nblocks(), A._itoi.ctypes.data_as(_lib.u64p),
         A._shapes.ctypes.data_as(_lib.u64p), A._offsets.ctypes.data_as(_lib.i64p),
@@ -166,7 +171,12 @@ def _plan_for(dtype: int, A: "UniTensor", B: "UniTensor", c1: List[int], c2: Lis
         B._shapes.ctypes.data_as(_lib.u64p), B._offsets.ctypes.data_as(_lib.i64p),
         len(c1), _lib.u64_array(c1), _lib.u64_array(c2),
         C.Nblocks(), C._itoi.ctypes.data_as(_lib.u64p), C._shapes.ctypes.data_as(_lib.u64p),
-        C._offsets.ctypes.data_as(_lib.i64p), ctypes.byref(h)))
+        C._offsets.ctypes.data_as(_lib.i64p))
+    if out_axes is None:
+        _lib.check(L.cxa_block_contract_plan(*args, ctypes.byref(h)))
+    else:
+        _lib.check(L.cxa_block_contract_plan_out(*args, _lib.u64_array(out_axes),
+                                                 ctypes.byref(h)))
     p = _Plan(h.value, A.device())
     if len(_PLAN_CACHE) > 4096:
         _PLAN_CACHE.clear()

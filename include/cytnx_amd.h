@@ -195,6 +195,19 @@ int cxa_block_contract_plan(int dtype, int rankL, int nbL, const uint64_t *itoiL
                             int ncomm, const uint64_t *comm1, const uint64_t *comm2, int nbC,
                             const uint64_t *itoiC, const uint64_t *shapeC, const int64_t *offC,
                             cxa_bc_plan **plan);
+/*
+ * The same with every output block stored permuted: axis j of a stored block (row-major, at
+ * offC) is axis out_axes[j] of the contraction's result (L free ++ R free, the order of itoiC and
+ * shapeC).  No counterpart in the reference, which permutes the result afterwards; used by the
+ * adjoint contractions, whose results belong in the layout of the operand they differentiate.
+ */
+int cxa_block_contract_plan_out(int dtype, int rankL, int nbL, const uint64_t *itoiL,
+                                const uint64_t *shapeL, const int64_t *offL, int rankR, int nbR,
+                                const uint64_t *itoiR, const uint64_t *shapeR,
+                                const int64_t *offR, int ncomm, const uint64_t *comm1,
+                                const uint64_t *comm2, int nbC, const uint64_t *itoiC,
+                                const uint64_t *shapeC, const int64_t *offC,
+                                const uint64_t *out_axes, cxa_bc_plan **plan);
 /* flops: sum over block pairs of 2*M*N*K (x4 for complex); npairs: number of block pairs. */
 int cxa_block_contract_info(const cxa_bc_plan *plan, double *flops, int64_t *workspace_bytes,
                             int64_t *npairs);
