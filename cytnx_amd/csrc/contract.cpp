@@ -178,6 +178,7 @@ int native_prec(int dtype) {
 // precision is made now, the others on first use (a tile list of a large contraction takes
 // about a millisecond of host time, and most plans only ever run one precision).
 int upload_plan(cxa_bc_plan *p) {
+  for (GBlk &b : p->blks) seal_block(b, p->segs.data());
   // blks, segs, outs and the batched copy jobs / tasks of both operands, each 256-byte aligned
   struct Part {
     const void *src;
@@ -1217,6 +1218,7 @@ extern "C" int cxa_matmul(int dtype, void *out, const void *inl, const void *inr
   g.C = out;
   g.blk0 = GBlk{0, Nr, 1, 1.0, 0.0, (int32_t)Ml, (int32_t)Nr, 0, Comm > 0 ? 1 : 0};
   g.seg0 = GSeg{0, 0, Comm, 1, Nr, 1, (int32_t)Comm, 0};
+  seal_block(g.blk0, &g.seg0);
   return launch_grouped_gemm(g, (hipStream_t)stream);
 }
 
@@ -1295,6 +1297,7 @@ extern "C" int cxa_gemm_batch(int dtype, const char *transa, const char *transb,
       }
     }
   }
+  for (GBlk &b : blks) seal_block(b, segs.data());
   std::vector<GTile> tiles;
   int per_xcd = 0;
   const Tiling tl = default_tiling(blks, segs, cplx);
@@ -1446,6 +1449,7 @@ extern "C" int cxa_tensordot(int dtype, void *out, const void *L, int rankL,
   g.C = out;
   g.blk0 = GBlk{0, N, 1, 1.0, 0.0, (int32_t)M, (int32_t)N, 0, K > 0 ? 1 : 0};
   g.seg0 = GSeg{0, 0, sam, sak, sbk, sbn, (int32_t)K, 0};
+  seal_block(g.blk0, &g.seg0);
   return launch_grouped_gemm(g, (hipStream_t)stream);
 }
 

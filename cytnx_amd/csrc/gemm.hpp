@@ -34,6 +34,8 @@ struct GBlk {
   int32_t seg0, nseg;
   int32_t out0, nout;  // mix launches only: the item's outputs (MixOut)
   double alpha_im, beta_im;  // imaginary parts of alpha / beta (complex dtypes only)
+  int32_t chunks;  // 16-deep K chunks of all segments (set by seal_blocks)
+  int32_t wide;    // a segment's strides are too large for 32-bit offsets in a direct tile
 };
 
 // Mix launches (a grouped GEMM with a linear-combination epilogue).  An item is a GBlk whose
@@ -147,6 +149,9 @@ struct Tiling {
 };
 Tiling default_tiling(const std::vector<GBlk> &blks, const std::vector<GSeg> &segs, bool cplx);
 Tiling single_tiling(const GBlk &blk, const GSeg &seg, bool cplx);
+
+// Fill in what the kernels need to know about a block's segments (chunks, wide).
+void seal_block(GBlk &blk, const GSeg *segs);
 
 // Whether an LDS tile may read a segment: its loads use 32-bit byte offsets from the tile's
 // first element (elements of up to 16 bytes, up to 64 rows and 64 values of k, also with the

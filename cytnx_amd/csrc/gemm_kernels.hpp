@@ -125,6 +125,39 @@ __device__ __forceinline__ T load_or_zero(gptr<const T> p, bool valid) {
   return *reinterpret_cast<gptr<const T>>(a);
 }
 
+// Loads through a buffer descriptor: 32-bit offsets per lane from a scalar base plus a scalar
+// offset, so a chunk's addresses cost no vector arithmetic, and an offset of kNoLoad reads as
+// zero without a memory access (elements outside the block or past the segment's K).  The
+// elements of a tile's chunk lie within 2^31 bytes of the base (checked on the host: seal_block,
+// lds_ok), and so do the scalar offsets, so no sum wraps.
+constexpr uint32_t kNoLoad = 0x80000000u;
+
+__device__ __forceinline__ __amdgpu_buffer_rsrc_t buffer_at(uint64_t base) {
+  return __builtin_amdgcn_make_buffer_rsrc((void *)base, 0, (int)kNoLoad, 0x00027000);
+}
+
+template <typename V>
+__device__ __forceinline__ V buffer_get(__amdgpu_buffer_rsrc_t r, uint32_t off, uint32_t soff) {
+  typedef int i2 __attribute__((ext_vector_type(2)));
+  typedef int i4 __attribute__((ext_vector_type(4)));
+  if constexpr (sizeof(V) == 4) {
+    return __builtin_bit_cast(V, __builtin_amdgcn_raw_buffer_load_b32(r, off, soff, 0));
+  } else if constexpr (sizeof(V) == 8) {
+    return __builtin_bit_cast(V, __builtin_amdgcn_raw_buffer_load_b64(r, off, soff, 0));
+  } else if constexpr (sizeof(V) == 16) {
+    return __builtin_bit_cast(V, __builtin_amdgcn_raw_buffer_load_b128(r, off, soff, 0));
+  } else {
+    static_assert(sizeof(V) == 32, "load width");
+    struct Two {
+      i4 a, b;
+    };
+    return __builtin_bit_cast(
+        V, Two{__builtin_bit_cast(i4, __builtin_amdgcn_raw_buffer_load_b128(r, off, soff, 0)),
+               __builtin_bit_cast(
+                   i4, __builtin_amdgcn_raw_buffer_load_b128(r, off, soff + 16, 0))});
+  }
+}
+
 struct SegArray {
   const GSeg *p;
   __device__ __forceinline__ GSeg operator()(int i) const { return p[i]; }
@@ -145,7 +178,7 @@ struct RealAcc {
   // tile's whole K range at the usual block sizes (K <= 64 is one round trip), within a register
   // budget that keeps several waves per SIMD.
   static constexpr int depth =
-      (MI * NI >= 8 || (PREC != CXA_PREC_FP32 && MI * NI >= 4)) ? 2 : 4;
+      (MI * NI >= 8 || (PREC != CXA_PREC_FP32 && MI * NI >= 4)) ? 2 : F64 && MI * NI == 2 ? 3 : 4;
   acc_t hi[MI][NI];
   acc_t lo[MI][NI];
   __device__ __forceinline__ void zero() {
@@ -346,57 +379,208 @@ struct ChunkCursor {
   }
 };
 
+// One operand's part of a wave's chunks: NR groups of 16 rows (A's m or B's n), one row per lane
+// and group, 4 consecutive k.
+template <typename T, int NR, bool QUAD>
+struct ChunkSide {
+  using qe = typename std::conditional<QUAD, T, float>::type;  // (packed operands are real)
+  typedef qe t4 __attribute__((ext_vector_type(4)));
+  uint64_t base;     // address of (row 0, k 0) of the next chunk (uniform)
+  int64_t adv;       // bytes from chunk to chunk (uniform)
+  uint32_t sk;       // bytes from k to k + 1 (uniform; QUAD: not used)
+  uint32_t off[NR];  // this lane's first element of each group; kNoLoad: outside the block
+  // first: the address of (row 0, k 0); sr, st: the segment's strides along the rows and k (QUAD:
+  // from quad to quad); step: chunks from one of the wave's chunks to its next
+  __device__ __forceinline__ void enter(uint64_t first, int64_t sr, int64_t st, int rows,
+                                        int step, int r, int g) {
+    base = first;
+    adv = (int64_t)(QUAD ? 4 : 16) * step * st * (int64_t)sizeof(T);
+    sk = (uint32_t)st * (uint32_t)sizeof(T);
+#pragma unroll
+    for (int i = 0; i < NR; ++i) {
+      const uint32_t row = 16 * i + r;
+      const uint32_t e = row * (QUAD ? 4u : (uint32_t)sr) +
+                         (uint32_t)(QUAD ? g : 4 * g) * (uint32_t)st;
+      off[i] = (int)row < rows ? e * (uint32_t)sizeof(T) : kNoLoad;
+    }
+  }
+  // kleft: k left in the segment (QUAD: whole quads, zero past K)
+  __device__ __forceinline__ void load(T (&v)[NR][4], int kleft, int g) const {
+    const __amdgpu_buffer_rsrc_t rs = buffer_at(base);
+    if constexpr (QUAD) {
+#pragma unroll
+      for (int i = 0; i < NR; ++i) {
+        const t4 x = buffer_get<t4>(rs, 4 * g < kleft ? off[i] : kNoLoad, 0);
+        v[i][0] = x.x;
+        v[i][1] = x.y;
+        v[i][2] = x.z;
+        v[i][3] = x.w;
+      }
+    } else {
+#pragma unroll
+      for (int j = 0; j < 4; ++j)
+#pragma unroll
+        for (int i = 0; i < NR; ++i)
+          v[i][j] = buffer_get<T>(rs, 4 * g + j < kleft ? off[i] : kNoLoad, j * sk);
+    }
+  }
+};
+
+// The chunks of a wave in order, like ChunkCursor, for tiles whose addresses fit 32-bit offsets.
+// Past the last chunk every load reads zeros.  ONE: the block has a single segment.
+template <typename TA, typename TB, int MI, int NI, int PK, bool ONE, typename SEGS>
+struct ChunkStream {
+  SEGS segs;
+  int seg0, nseg, step, m0, n0, mt, nt, r, g;
+  int s, k0, K;  // current segment, chunk start within it, and its extent
+  GSeg nx;       // the next segment, read while this one's chunks run
+  ChunkSide<TA, MI, (PK & kPackA) != 0> a;
+  ChunkSide<TB, NI, (PK & kPackB) != 0> b;
+  // to the chunk `first` chunks from the start (nseg > 0)
+  __device__ __forceinline__ void start(int first, const char *Abase, const char *Bbase) {
+    s = 0;
+    k0 = 16 * first;
+    nx = segs(seg0);
+    enter(Abase, Bbase);
+  }
+  // into segment s, whose descriptor is nx, k0 from its start, stepping over whole segments
+  __device__ __forceinline__ void enter(const char *Abase, const char *Bbase) {
+    GSeg sg = nx;
+    if constexpr (!ONE) {
+      while (true) {
+        nx = segs(seg0 + min(s + 1, nseg - 1));
+        const int span = 16 * ((sg.K + 15) >> 4);
+        if (k0 < span) break;
+        k0 -= span;
+        if (++s >= nseg) {
+          K = k0 = 0;
+          return;
+        }
+        sg = nx;
+      }
+    }
+    K = sg.K;
+    a.enter((uint64_t)(uintptr_t)(at<const TA>(Abase, sg.a_off) + (int64_t)m0 * stride_a(sg)),
+            sg.sam, sg.sak, mt, step, r, g);
+    b.enter((uint64_t)(uintptr_t)(at<const TB>(Bbase, sg.b_off) + (int64_t)n0 * stride_b(sg)),
+            sg.sbn, sg.sbk, nt, step, r, g);
+    a.base += (int64_t)((PK & kPackA) ? k0 >> 2 : k0) * sg.sak * (int64_t)sizeof(TA);
+    b.base += (int64_t)((PK & kPackB) ? k0 >> 2 : k0) * sg.sbk * (int64_t)sizeof(TB);
+  }
+  static __device__ __forceinline__ int64_t stride_a(const GSeg &sg) {
+    return (PK & kPackA) ? 4 : sg.sam;
+  }
+  static __device__ __forceinline__ int64_t stride_b(const GSeg &sg) {
+    return (PK & kPackB) ? 4 : sg.sbn;
+  }
+  __device__ __forceinline__ void load(Frag<TA, TB, MI, NI> &f) const {
+    a.load(f.a, K - k0, g);
+    b.load(f.b, K - k0, g);
+  }
+  __device__ __forceinline__ void next(const char *Abase, const char *Bbase) {
+    k0 += 16 * step;
+    a.base += a.adv;
+    b.base += b.adv;
+    if constexpr (!ONE) {
+      if (k0 >= K) {
+        k0 -= 16 * ((K + 15) >> 4);
+        if (++s < nseg)
+          enter(Abase, Bbase);
+        else
+          s = nseg, K = k0 = 0;
+      }
+    }
+  }
+};
+
+// Run `total` > 0 chunks through a ring of D fragment sets, D of them in flight: load(d) fetches
+// the next chunk into set d and next() goes on to the one after it, use(d) consumes set d.  No
+// load of the ring is conditional: the compiler's wait for a set then leaves the D - 1 newer ones
+// in flight, where a load under a condition would make it wait for all of them at every chunk.
+// TAIL: ranges shorter than D and the last, partial round take only their own loads, in code of
+// their own; without it (next() is long) ranges of one chunk do, and the loads past the last
+// chunk, fewer than D chunks, read zeros without a memory access.
+template <int D, bool TAIL, typename LOAD, typename NEXT, typename USE>
+__device__ __forceinline__ void run_chunks(int total, LOAD load, NEXT next, USE use) {
+  constexpr int SHORT = TAIL ? D - 1 : 1;
+  if (total <= SHORT) {
+#pragma unroll
+    for (int d = 0; d < SHORT; ++d)
+      if (d < total) {
+        load(d);
+        if (d + 1 < SHORT) next();
+      }
+#pragma unroll
+    for (int d = 0; d < SHORT; ++d)
+      if (d < total) use(d);
+  } else {
+#pragma unroll
+    for (int d = 0; d < D; ++d) {
+      load(d);
+      next();
+    }
+    for (; total > (TAIL ? 2 * D - 1 : D); total -= D) {
+#pragma unroll
+      for (int d = 0; d < D; ++d) {
+        use(d);
+        load(d);
+        next();
+      }
+    }
+    if constexpr (TAIL) {  // D .. 2 D - 1 chunks left, D of them loaded
+#pragma unroll
+      for (int d = 0; d < D; ++d) {
+        use(d);
+        if (d < total - D) {
+          load(d);
+          next();
+        }
+      }
+      total -= D;
+    }
+#pragma unroll
+    for (int d = 0; d < (TAIL ? D - 1 : D); ++d)
+      if (d < total) use(d);
+  }
+  drain_loads();
+}
+
 // Accumulate the chunks c with c % nslices == slice of the block's concatenated K range.
 // A ring of ACC::depth fragment sets keeps that many chunks' loads in flight across the
 // whole range (segment boundaries included): the MFMAs of chunk c issue while chunks
 // c+1 .. c+depth-1 are still arriving, and chunk c+depth is loaded into the set just consumed.
-// Only real chunks are loaded: the launches are bound by the vector-memory address path, so
-// padding a wave's chunk count to whole rounds of the ring (which would let every wait count
-// be exact) costs more than the waits it saves.
 template <typename TA, typename TB, int MI, int NI, int PK, typename ACC, typename SEGS>
 __device__ __forceinline__ void mfma_accumulate(ACC &acc,
                                                 const char *__restrict__ Abase,
                                                 const char *__restrict__ Bbase, const GBlk &blk,
                                                 SEGS segs, int m0, int n0, int lane, int slice,
                                                 int nslices) {
-  constexpr int D = ACC::depth;
   const int r = lane & 15, g = lane >> 4;
   const int mt = min(16 * MI, blk.M - m0);
   const int nt = min(16 * NI, blk.N - n0);
-  // chunks of this slice over all segments
-  int total = 0, cb = 0;
-  for (int s = 0; s < blk.nseg; ++s) {
-    const int nc = (segs(blk.seg0 + s).K + 15) >> 4;
-    const int first = ((slice - cb) % nslices + nslices) % nslices;
-    if (first < nc) total += (nc - first + nslices - 1) / nslices;
-    cb += nc;
-  }
-  if (total == 0) return;
-  ChunkCursor<TA, TB, SEGS> cur{segs, blk.seg0, blk.nseg, nslices, m0, n0, 0, 0};
-  cur.enter(Abase, Bbase);
-  cur.skip(slice, Abase, Bbase);  // also steps over empty leading segments
-  Frag<TA, TB, MI, NI> f[D];
-#pragma unroll
-  for (int d = 0; d < D; ++d) {
-    if (d < total) {
-      cur.template load<MI, NI, PK>(f[d], mt, nt, r, g);
+  const int total = (blk.chunks - slice + nslices - 1) / nslices;
+  if (total <= 0) return;
+  if (blk.wide) {
+    ChunkCursor<TA, TB, SEGS> cur{segs, blk.seg0, blk.nseg, nslices, m0, n0, 0, 0};
+    cur.enter(Abase, Bbase);
+    cur.skip(slice, Abase, Bbase);  // also steps over empty leading segments
+    for (int c = 0; c < total; ++c) {
+      Frag<TA, TB, MI, NI> f;
+      cur.template load<MI, NI, PK>(f, mt, nt, r, g);
       cur.skip(nslices, Abase, Bbase);
+      mma_frag(acc, f);
     }
+    drain_loads();
+    return;
   }
-  for (int base = 0; base < total; base += D) {
-#pragma unroll
-    for (int d = 0; d < D; ++d) {
-      const int c = base + d;
-      if (c < total) {
-        mma_frag(acc, f[d]);
-        if (c + D < total) {
-          cur.template load<MI, NI, PK>(f[d], mt, nt, r, g);
-          cur.skip(nslices, Abase, Bbase);
-        }
-      }
-    }
-  }
-  drain_loads();
+  ChunkStream<TA, TB, MI, NI, PK, std::is_same<SEGS, SegOne>::value, SEGS> st{
+      segs, blk.seg0, blk.nseg, nslices, m0, n0, mt, nt, r, g};
+  st.start(slice, Abase, Bbase);
+  constexpr int D = ACC::depth;
+  Frag<TA, TB, MI, NI> f[D];
+  run_chunks<D, std::is_same<SEGS, SegOne>::value>(
+      total, [&](int d) { st.load(f[d]); }, [&]() { st.next(Abase, Bbase); },
+      [&](int d) { mma_frag(acc, f[d]); });
 }
 
 template <typename TC>
@@ -869,7 +1053,7 @@ __device__ __forceinline__ void run_tile(int kind, const char *A, const char *B,
 // grouped launch: tiles, blocks and segments come from device arrays; one wave per tile.
 // Workgroup w runs on XCD w % kXcds and takes tiles from that XCD's range of the list.
 template <int PREC, typename TA, typename TB, typename TC, bool CPLX, int CLS, int PK>
-__global__ __launch_bounds__(64 * kWaves) void k_grouped(const GTile *__restrict__ tiles,
+__global__ __launch_bounds__(64 * kWaves, 2) void k_grouped(const GTile *__restrict__ tiles,
                                                         int per_xcd, const GBlk *__restrict__ blks,
                                                         const GSeg *__restrict__ segs,
                                                         const char *A, const char *B, char *C,
@@ -897,7 +1081,7 @@ __global__ __launch_bounds__(64 * kWaves) void k_grouped(const GTile *__restrict
 // grouped launch with workgroup split-K: one workgroup per tile (real dtypes; the mixed MFMA
 // class or the row class)
 template <int PREC, typename TA, typename TB, typename TC, int CLS, int WAVES, int PK>
-__global__ __launch_bounds__(64 * WAVES) void k_grouped_split(
+__global__ __launch_bounds__(64 * WAVES, 2) void k_grouped_split(
     const GTile *__restrict__ tiles, int per_xcd, const GBlk *__restrict__ blks,
     const GSeg *__restrict__ segs, const char *A, const char *B, char *C,
     const double *dotx, double *dotp) {
@@ -1007,7 +1191,7 @@ __device__ __forceinline__ void mfma_accumulate_multi(RealAcc<PREC, MI, NI> (&ac
                                                       const char *__restrict__ Abase,
                                                       const char *__restrict__ Bbase, SEGS segs,
                                                       int nseg, int M, int N, int m0, int n0,
-                                                      int lane) {
+                                                      int lane, bool wide) {
   constexpr int D = RealAcc<PREC, MI, NI>::depth;
   const int r = lane & 15, g = lane >> 4;
   const int mt = min(16 * MI, M - m0);
@@ -1020,9 +1204,6 @@ __device__ __forceinline__ void mfma_accumulate_multi(RealAcc<PREC, MI, NI> (&ac
     total += nc[q];
   }
   if (total == 0) return;
-  ChunkCursor<TA, TB, SEGS> cur{segs, 0, nseg, 1, m0, n0, 0, 0};
-  cur.enter(Abase, Bbase);
-  cur.skip(0, Abase, Bbase);
   int cs = 0, left = nc[0];
 #pragma unroll
   for (int q = 1; q < NACC; ++q)
@@ -1030,14 +1211,6 @@ __device__ __forceinline__ void mfma_accumulate_multi(RealAcc<PREC, MI, NI> (&ac
       cs = q;
       left = nc[q];
     }
-  Frag<TA, TB, MI, NI> f[D];
-#pragma unroll
-  for (int d = 0; d < D; ++d) {
-    if (d < total) {
-      cur.template load<MI, NI, PK>(f[d], mt, nt, r, g);
-      cur.skip(1, Abase, Bbase);
-    }
-  }
   // chunk -> accumulator bookkeeping
   auto consume = [&](const Frag<TA, TB, MI, NI> &fr) {
 #pragma unroll
@@ -1052,24 +1225,29 @@ __device__ __forceinline__ void mfma_accumulate_multi(RealAcc<PREC, MI, NI> (&ac
         }
     }
   };
-  for (int base = 0; base < total; base += D) {
-#pragma unroll
-    for (int d = 0; d < D; ++d) {
-      const int c = base + d;
-      if (c < total) {
-        consume(f[d]);
-        if (c + D < total) {
-          cur.template load<MI, NI, PK>(f[d], mt, nt, r, g);
-          cur.skip(1, Abase, Bbase);
-        }
-      }
+  if (wide) {
+    ChunkCursor<TA, TB, SEGS> cur{segs, 0, nseg, 1, m0, n0, 0, 0};
+    cur.enter(Abase, Bbase);
+    cur.skip(0, Abase, Bbase);
+    for (int c = 0; c < total; ++c) {
+      Frag<TA, TB, MI, NI> f;
+      cur.template load<MI, NI, PK>(f, mt, nt, r, g);
+      cur.skip(1, Abase, Bbase);
+      consume(f);
     }
+    drain_loads();
+    return;
   }
-  drain_loads();
+  ChunkStream<TA, TB, MI, NI, PK, NACC == 1, SEGS> st{segs, 0, nseg, 1, m0, n0, mt, nt, r, g};
+  st.start(0, Abase, Bbase);
+  Frag<TA, TB, MI, NI> f[D];
+  run_chunks<D, NACC == 1>(
+      total, [&](int d) { st.load(f[d]); }, [&]() { st.next(Abase, Bbase); },
+      [&](int d) { consume(f[d]); });
 }
 
 template <int PREC, typename TA, typename TB, typename TC, int MI, int NI, int WAVES, int PK>
-__global__ __launch_bounds__(64 * WAVES) void k_mix(const GTile *__restrict__ tiles,
+__global__ __launch_bounds__(64 * WAVES, MI *NI == 4 && WAVES == 4 ? 2 : 4) void k_mix(const GTile *__restrict__ tiles,
                                                    int per_xcd, const GBlk *__restrict__ items,
                                                    const GSeg *__restrict__ slices,
                                                    const MixOut *__restrict__ outs,
@@ -1099,7 +1277,7 @@ __global__ __launch_bounds__(64 * WAVES) void k_mix(const GTile *__restrict__ ti
       for (int q = 0; q < NACC; ++q) acc[q].zero();
       mfma_accumulate_multi<PREC, TA, TB, MI, NI, NACC, PK>(
           acc, A, B, SegStride{slices, it.seg0 + wave, WAVES}, mine, it.M, it.N, tl.m0, tl.n0,
-          lane);
+          lane, it.wide != 0);
 #pragma unroll
       for (int q = 0; q < NACC; ++q) {
         const int sl = wave + q * WAVES;
@@ -1251,7 +1429,7 @@ int launch_mix_t(const GemmLaunch &g, hipStream_t s) {
 // single-block launch: one block with one segment, tiles derived from the launch index, so a
 // plain GEMM needs no device-side task list (mixed MFMA class)
 template <int PREC, typename TA, typename TB, typename TC, bool CPLX>
-__global__ __launch_bounds__(64 * kWaves) void k_single(GBlk blk, GSeg seg, int kind,
+__global__ __launch_bounds__(64 * kWaves, 2) void k_single(GBlk blk, GSeg seg, int kind,
                                                        int tiles_n, int ntiles, const char *A,
                                                        const char *B, char *C, int conj) {
   const int lane = threadIdx.x & 63;

@@ -58,33 +58,6 @@ struct LdsGeo {
   static constexpr size_t bytes = 2 * (size_t)(BM + BN) * LD * sizeof(ES);
 };
 
-// Loads through a buffer descriptor: 32-bit offsets per lane from a scalar base, so a chunk's
-// addresses cost no vector arithmetic, and an offset at kLdsOut or above reads as zero without
-// a memory access (elements outside the block or past the segment's K).  A tile's and a chunk's
-// elements lie within kLdsSpan bytes of the base (checked on the host, lds_ok).
-constexpr uint32_t kLdsOut = 0x80000000u;
-
-template <typename V>
-__device__ __forceinline__ V buffer_get(__amdgpu_buffer_rsrc_t r, uint32_t off) {
-  typedef int i2 __attribute__((ext_vector_type(2)));
-  typedef int i4 __attribute__((ext_vector_type(4)));
-  if constexpr (sizeof(V) == 4) {
-    return __builtin_bit_cast(V, __builtin_amdgcn_raw_buffer_load_b32(r, off, 0, 0));
-  } else if constexpr (sizeof(V) == 8) {
-    return __builtin_bit_cast(V, __builtin_amdgcn_raw_buffer_load_b64(r, off, 0, 0));
-  } else if constexpr (sizeof(V) == 16) {
-    return __builtin_bit_cast(V, __builtin_amdgcn_raw_buffer_load_b128(r, off, 0, 0));
-  } else {
-    static_assert(sizeof(V) == 32, "load width");
-    struct Two {
-      i4 a, b;
-    };
-    return __builtin_bit_cast(
-        V, Two{__builtin_bit_cast(i4, __builtin_amdgcn_raw_buffer_load_b128(r, off, 0, 0)),
-               __builtin_bit_cast(i4, __builtin_amdgcn_raw_buffer_load_b128(r, off, 16, 0))});
-  }
-}
-
 // One operand of a tile: this thread's part of the chunk being loaded.  Rows are A's m or B's n.
 template <typename T, typename op_t, int BR, int BK, int LD, int NT, bool QUAD>
 struct LdsSide {
@@ -98,7 +71,7 @@ struct LdsSide {
   static_assert(N >= 1 && NT % BR == 0 && NT % BK == 0, "staging layout");
   uint64_t base;    // address of (row 0, k 0) of the next chunk (uniform)
   int64_t adv;      // bytes from chunk to chunk (uniform)
-  uint32_t off[N];  // this thread's elements from base; kLdsOut: not read
+  uint32_t off[N];  // this thread's elements from base; kNoLoad: not read
   int put_at[N];    // where they go in an LDS buffer
   int row0, dr;     // row of its first element within the tile, and the step of the others
   int k0, dk;       // the same for k within the chunk
@@ -129,7 +102,7 @@ struct LdsSide {
     for (int i = 0; i < N; ++i) {
       const uint32_t row = row0 + i * dr, k = k0 + i * dk;
       off[i] = (int)row < rows ? (row * s_r + (QUAD ? k >> 2 : k) * s_k) * (uint32_t)sizeof(G)
-                               : kLdsOut;
+                               : kNoLoad;
     }
     if (kleft < BK) last(kleft);
   }
@@ -137,13 +110,12 @@ struct LdsSide {
   __device__ __forceinline__ void last(int kleft) {
 #pragma unroll
     for (int i = 0; i < N; ++i)
-      if (k0 + i * dk >= kleft) off[i] = kLdsOut;
+      if (k0 + i * dk >= kleft) off[i] = kNoLoad;
   }
   __device__ __forceinline__ void load(V (&v)[N]) {
-    const __amdgpu_buffer_rsrc_t r = __builtin_amdgcn_make_buffer_rsrc(
-        (void *)base, 0, (int)kLdsOut, 0x00027000);
+    const __amdgpu_buffer_rsrc_t r = buffer_at(base);
 #pragma unroll
-    for (int i = 0; i < N; ++i) v[i] = buffer_get<V>(r, off[i]);
+    for (int i = 0; i < N; ++i) v[i] = buffer_get<V>(r, off[i], 0);
     base += adv;
   }
   __device__ __forceinline__ void store(const V (&v)[N], ES *lds, op_t sign) const {
