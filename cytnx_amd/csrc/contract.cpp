@@ -95,9 +95,9 @@ struct cxa_bc_plan {
   std::vector<cxa::CopyJob> jobsA, jobsB, jobsC;  // blocks too large for the batched copy
   // the other operand (output) blocks, permuted into (out of) the workspace by one batched
   // launch each
-  std::vector<cxa::BatchCopyJob> bjobsA, bjobsB, bjobsC;
+  std::vector<char> bjobsA, bjobsB, bjobsC;
   std::vector<cxa::BatchCopyTask> btasksA, btasksB, btasksC;
-  const cxa::BatchCopyJob *dev_bjobsA = nullptr, *dev_bjobsB = nullptr, *dev_bjobsC = nullptr;
+  const void *dev_bjobsA = nullptr, *dev_bjobsB = nullptr, *dev_bjobsC = nullptr;
   const cxa::BatchCopyTask *dev_btasksA = nullptr, *dev_btasksB = nullptr,
                            *dev_btasksC = nullptr;
   int64_t wsA = 0, wsB = 0, wsC = 0;  // workspace elements for A, B and C copies
@@ -187,11 +187,11 @@ int upload_plan(cxa_bc_plan *p) {
   Part parts[9] = {{p->blks.data(), p->blks.size() * sizeof(GBlk), 0},
                    {p->segs.data(), p->segs.size() * sizeof(GSeg), 0},
                    {p->outs.data(), p->mix ? p->outs.size() * sizeof(MixOut) : 0, 0},
-                   {p->bjobsA.data(), p->bjobsA.size() * sizeof(BatchCopyJob), 0},
+                   {p->bjobsA.data(), p->bjobsA.size(), 0},
                    {p->btasksA.data(), p->btasksA.size() * sizeof(BatchCopyTask), 0},
-                   {p->bjobsB.data(), p->bjobsB.size() * sizeof(BatchCopyJob), 0},
+                   {p->bjobsB.data(), p->bjobsB.size(), 0},
                    {p->btasksB.data(), p->btasksB.size() * sizeof(BatchCopyTask), 0},
-                   {p->bjobsC.data(), p->bjobsC.size() * sizeof(BatchCopyJob), 0},
+                   {p->bjobsC.data(), p->bjobsC.size(), 0},
                    {p->btasksC.data(), p->btasksC.size() * sizeof(BatchCopyTask), 0}};
   size_t total = 0;
   for (Part &q : parts) {
@@ -211,43 +211,33 @@ int upload_plan(cxa_bc_plan *p) {
     p->dev_blks = (const GBlk *)at(0);
     p->dev_segs = (const GSeg *)at(1);
     p->dev_outs = (const MixOut *)at(2);
-    p->dev_bjobsA = (const BatchCopyJob *)at(3);
+    p->dev_bjobsA = at(3);
     p->dev_btasksA = (const BatchCopyTask *)at(4);
-    p->dev_bjobsB = (const BatchCopyJob *)at(5);
+    p->dev_bjobsB = at(5);
     p->dev_btasksB = (const BatchCopyTask *)at(6);
-    p->dev_bjobsC = (const BatchCopyJob *)at(7);
+    p->dev_bjobsC = at(7);
     p->dev_btasksC = (const BatchCopyTask *)at(8);
   }
   if (p->chain) return CXA_OK;  // cxa_chain_create makes the tile list (bc_join_chain)
   return build_variant(p, native_prec(p->dtype));
 }
 
-// Split an operand's permute-to-workspace jobs: small blocks into one batched launch (jobs +
-// tasks), the rest (large blocks, or a lone small block, which the tiled permute moves faster)
-// onto the one-by-one list.
-void split_copies(const std::vector<CopyJob> &all, std::vector<CopyJob> &big,
-                  std::vector<BatchCopyJob> &bj, std::vector<BatchCopyTask> &bt) {
-  std::vector<BatchCopyJob> small;
+// Split the permute-to-workspace jobs of an operand: one batched launch (jobs + tasks), and a
+// one-by-one list of the largest blocks, or of a lone one, which cxa_permute moves faster.
+void split_copies(int es, const std::vector<CopyJob> &all, std::vector<CopyJob> &big,
+                  std::vector<char> &bj, std::vector<BatchCopyTask> &bt) {
   std::vector<const CopyJob *> from;
   for (const CopyJob &j : all) {
-    BatchCopyJob b;
-    if (batch_copy_job(j.rank, j.shape, j.mapper, j.src_off, j.dst_off, &b)) {
-      small.push_back(b);
+    if (batch_copy_job(es, j.rank, j.shape, j.mapper, j.src_off, j.dst_off, (int)from.size(), bj,
+                       bt))
       from.push_back(&j);
-    } else {
+    else
       big.push_back(j);
-    }
   }
-  if (small.size() < 2) {
-    for (const CopyJob *j : from) big.push_back(*j);
-    return;
-  }
-  for (const BatchCopyJob &b : small) {
-    const int id = (int)bj.size();
-    bj.push_back(b);
-    for (int32_t at = 0; at < b.n; at += kBatchCopyTaskElems)
-      bt.push_back({id, at, std::min(kBatchCopyTaskElems, b.n - at), 0});
-  }
+  if (from.size() >= 2) return;
+  for (const CopyJob *j : from) big.push_back(*j);
+  bj.clear();
+  bt.clear();
 }
 
 }  // namespace
@@ -614,9 +604,9 @@ int make_block_plan(int dtype, int rankL, int nbL, const uint64_t *itoiL, const 
     }
   }
 
-  split_copies(copiesA, p->jobsA, p->bjobsA, p->btasksA);
-  split_copies(copiesB, p->jobsB, p->bjobsB, p->btasksB);
-  split_copies(copiesC, p->jobsC, p->bjobsC, p->btasksC);
+  split_copies(es, copiesA, p->jobsA, p->bjobsA, p->btasksA);
+  split_copies(es, copiesB, p->jobsB, p->bjobsB, p->btasksB);
+  split_copies(es, copiesC, p->jobsC, p->bjobsC, p->btasksC);
 
   // The products: one GBlk per output block and combination of the row and column indices taken
   // apart, its segments in pair order.  A block whose rows are the contiguous ones of C (a

@@ -22,28 +22,28 @@ struct ExecLayout {
   double *dot_part = nullptr;
 };
 
-// Batched permute of many small blocks in one launch (permute.hip).  Job j writes its
-// n elements contiguously: dst[dst_off + e] = src[src_off + sum_d idx_d(e) * sstr[d]], idx(e)
-// the row-major coordinates of e over ext[0 .. rank); a task is a contiguous element range of
-// one job, one workgroup each.
-constexpr int kBatchCopyMaxElems = 1 << 15;  // larger blocks go through cxa_permute one by one
-constexpr int kBatchCopyTaskElems = 4096;
-struct BatchCopyJob {
-  int64_t src_off, dst_off;  // elements
-  int32_t n, rank;
-  int32_t ext[16];
-  int32_t sstr[16];
-};
+// Batched permute of many blocks in one launch (permute.hip).  A task is a range of one job's
+// elements or tiles, one workgroup each.  Blocks above kBatchCopyMaxElems go through cxa_permute
+// one by one: such a block takes longer than a launch by itself (2^20 elements of 8 bytes: 4 us at
+// the rate of a large copy), and the single kernel overlaps a tile's loads with the last one's
+// stores.
+constexpr int kBatchCopyMaxElems = 1 << 20;
+constexpr int kBatchCopyTaskElems = 1024;
 struct BatchCopyTask {
   int32_t job, start, count, pad;
 };
-// The job that permutes one row-major block of extents shape[rank] by mapper (new axis d = old
-// axis mapper[d]); false when the block is too large for the batched launch.
-bool batch_copy_job(int rank, const uint64_t *shape, const uint64_t *mapper, int64_t src_off,
-                    int64_t dst_off, BatchCopyJob *job);
-// One launch over ntasks tasks (device arrays) for elements of elem_size bytes (4, 8 or 16).
-int launch_batch_copy(int elem_size, const BatchCopyJob *jobs, const BatchCopyTask *tasks,
-                      int ntasks, const void *src, void *dst, hipStream_t s);
+size_t batch_job_bytes();  // of one job in a job list
+// Append the job (number id of the list) that permutes one row-major block of extents shape[rank]
+// by mapper (new axis d = old axis mapper[d]), and its tasks; false when the block is too large
+// for the batched launch.
+bool batch_copy_job(int elem_size, int rank, const uint64_t *shape, const uint64_t *mapper,
+                    int64_t src_off, int64_t dst_off, int id, std::vector<char> &jobs,
+                    std::vector<BatchCopyTask> &tasks);
+// One launch over ntasks tasks (device arrays) for elements of elem_size bytes (4, 8 or 16).  Jobs
+// made for 8-byte elements also serve FP32 copies of the same layout: offsets are in elements, and
+// the tiles of both hold as many.
+int launch_batch_copy(int elem_size, const void *jobs, const BatchCopyTask *tasks, int ntasks,
+                      const void *src, void *dst, hipStream_t s);
 
 // conj (complex plans): bit 0 conjugates L, bit 1 conjugates R as they are read.
 int bc_exec_typed(const cxa_bc_plan *p, const void *L, const void *R, void *C, int a_dt,

@@ -188,6 +188,11 @@ __device__ __forceinline__ uint32_t decode32(uint32_t x, int n, const FastDiv *d
   return off;
 }
 
+template <typename T>
+constexpr int max_tile() {  // elements of a tile
+  return sizeof(T) >= 16 ? 1024 : 2048;
+}
+
 struct TileAt {
   uint32_t oin, oout, a0, b0, tw, th, tc;
 };
@@ -497,9 +502,10 @@ int grid_for(int64_t work_items, int per_block) {
   return (int)std::max<int64_t>(1, std::min<int64_t>(g, 256 * 64));
 }
 
-template <typename T>
-int launch_tiled(const Reduced &r, const void *src, void *dst, hipStream_t s) {
-  const int es = (int)sizeof(T);
+// The tiles of a reduced permutation that moves its innermost axis, for elements of es bytes;
+// *small32: q holds them in 32-bit form (p is filled in either way).  False: more axes outside the
+// tiles than the kernels take.
+bool plan_tiles(int es, const Reduced &r, TileArgs *args, TileArgs32 *args32, bool *small32) {
   const int r_ = r.rank;
   int64_t istr[16], ostr[16], nshape[16];
   int64_t acc = 1;
@@ -542,7 +548,8 @@ int launch_tiled(const Reduced &r, const void *src, void *dst, hipStream_t s) {
     inB[x] = true;
     prodB *= r.shape[x];
   }
-  TileArgs p{};
+  TileArgs &p = *args;
+  p = TileArgs{};
   p.na = na;
   p.nb = nb;
   // store groups outermost first
@@ -559,14 +566,14 @@ int launch_tiled(const Reduced &r, const void *src, void *dst, hipStream_t s) {
   int no = 0;
   for (int i = 0; i < r_; ++i) {
     if (inA[i] || inB[i]) continue;
-    if (no >= kMaxOuter) return -1;
+    if (no >= kMaxOuter) return false;
     p.o_ext[no] = r.shape[i];
     p.o_istr[no] = istr[i];
     p.o_ostr[no] = ostr[i];
     ++no;
   }
   p.no = no;
-  constexpr int MAXE = (sizeof(T) >= 16) ? 1024 : 2048;
+  const int MAXE = es >= 16 ? 1024 : 2048;
   // Tile shape and grid, measured on the rank-6 sweep (16 MiB / 32 MiB tensors, 32 seeded
   // permutations): 8-byte and smaller elements run the pipelined kernel on tiles 128 bytes wide
   // with at most 1024 workgroups (several tiles each, so loads and stores overlap); 16-byte
@@ -599,14 +606,10 @@ int launch_tiled(const Reduced &r, const void *src, void *dst, hipStream_t s) {
   int64_t outer = 1;
   for (int k = 0; k < no; ++k) outer *= p.o_ext[k];
   p.ntiles = outer * p.nca * p.ncb;
-  // pipelined: about two tiles per workgroup, at least 1024 workgroups (a single round when the
-  // tensor is small), at most 16384
-  const int64_t grid_cap = pipelined
-                               ? std::min<int64_t>(256 * 64, std::max<int64_t>(1024, p.ntiles / 2))
-                               : 4096;
-  const int grid = (int)std::max<int64_t>(1, std::min<int64_t>(p.ntiles, grid_cap));
-  if (r.total < (int64_t(1) << 31)) {  // every offset and index fits in 32 bits
-    TileArgs32 q{};
+  *small32 = r.total < (int64_t(1) << 31);  // every offset and index fits in 32 bits
+  if (*small32) {
+    TileArgs32 &q = *args32;
+    q = TileArgs32{};
     q.na = p.na;
     q.nb = p.nb;
     q.no = p.no;
@@ -649,28 +652,44 @@ int launch_tiled(const Reduced &r, const void *src, void *dst, hipStream_t s) {
       q.o_istr[k] = (uint32_t)p.o_istr[k];
       q.o_ostr[k] = (uint32_t)p.o_ostr[k];
     }
-    const int grid32 =
-        (int)std::max<int64_t>(1, std::min<int64_t>((int64_t)q.ntiles,
-                                                    pipelined ? std::min<int64_t>(
-                                                                    256 * 64,
-                                                                    std::max<int64_t>(
-                                                                        1024, q.ntiles / 2))
-                                                              : 4096));
-    if (pipelined && q.c > 1)
-      hipLaunchKernelGGL((permute_tiled32<T, MAXE, true>), dim3(grid32), dim3(kThreads), 0, s,
-                         (const T *)src, (T *)dst, q);
-    else if (pipelined)
-      hipLaunchKernelGGL((permute_tiled32<T, MAXE, false>), dim3(grid32), dim3(kThreads), 0, s,
-                         (const T *)src, (T *)dst, q);
-    else if (q.c > 1)
-      hipLaunchKernelGGL((permute_tiled32_once<T, MAXE, true>), dim3(grid32), dim3(kThreads), 0,
-                         s, (const T *)src, (T *)dst, q);
-    else
-      hipLaunchKernelGGL((permute_tiled32_once<T, MAXE, false>), dim3(grid32), dim3(kThreads), 0,
-                         s, (const T *)src, (T *)dst, q);
+  }
+  return true;
+}
+
+template <typename T>
+int launch_tiled(const Reduced &r, const void *src, void *dst, hipStream_t s) {
+  constexpr bool pipelined = sizeof(T) <= 8;
+  constexpr int MAXE = max_tile<T>();
+  TileArgs p;
+  TileArgs32 q;
+  bool small32;
+  if (!plan_tiles((int)sizeof(T), r, &p, &q, &small32)) return -1;
+  // pipelined: about two tiles per workgroup, at least 1024 workgroups (a single round when the
+  // tensor is small), at most 16384
+  auto grid_of = [](int64_t ntiles) {
+    const int64_t cap = pipelined ? std::min<int64_t>(256 * 64, std::max<int64_t>(1024, ntiles / 2))
+                                  : 4096;
+    return dim3((unsigned)std::max<int64_t>(1, std::min<int64_t>(ntiles, cap)));
+  };
+  if (small32) {
+    if constexpr (pipelined) {
+      if (q.c > 1)
+        hipLaunchKernelGGL((permute_tiled32<T, MAXE, true>), grid_of(q.ntiles), dim3(kThreads), 0,
+                           s, (const T *)src, (T *)dst, q);
+      else
+        hipLaunchKernelGGL((permute_tiled32<T, MAXE, false>), grid_of(q.ntiles), dim3(kThreads),
+                           0, s, (const T *)src, (T *)dst, q);
+    } else {
+      if (q.c > 1)
+        hipLaunchKernelGGL((permute_tiled32_once<T, MAXE, true>), grid_of(q.ntiles), dim3(kThreads), 0,
+                           s, (const T *)src, (T *)dst, q);
+      else
+        hipLaunchKernelGGL((permute_tiled32_once<T, MAXE, false>), grid_of(q.ntiles), dim3(kThreads), 0,
+                           s, (const T *)src, (T *)dst, q);
+    }
     return 0;
   }
-  hipLaunchKernelGGL((permute_tiled<T, MAXE>), dim3(grid), dim3(kThreads), 0, s,
+  hipLaunchKernelGGL((permute_tiled<T, MAXE>), grid_of(p.ntiles), dim3(kThreads), 0, s,
                      (const T *)src, (T *)dst, p);
   return 0;
 }
@@ -744,72 +763,157 @@ int run_permute(const Reduced &r, const void *src, void *dst, hipStream_t s) {
   return CXA_OK;
 }
 
-// Batched small-block permute: one workgroup per task; the job's reduced extents and source
-// strides sit in LDS, every thread decodes its elements' coordinates (32-bit: a job holds at
-// most kBatchCopyMaxElems elements) and gathers them; writes are contiguous.
+// One tile of a batched job (permute_tiled32_once's steps; in one function for both, that kernel
+// took 124 registers instead of 56 and 46 us instead of 44 for 84 MB).
+template <typename T, bool BATCH>
+__device__ __forceinline__ void move_tile(const T *__restrict__ src, T *__restrict__ dst,
+                                          const TileArgs32 &p, uint32_t t,
+                                          T (&tile)[max_tile<T>() + 64],
+                                          uint32_t (&aoff)[kMaxTile],
+                                          uint32_t (&boff)[kMaxTile]) {
+  constexpr int PER = max_tile<T>() / kThreads;
+  const int w = p.w, h = p.h, ws = w + 1;
+  const uint32_t n = (uint32_t)(w * h * p.c);
+  const TileAt x = tile_at(p, t);
+  __syncthreads();  // the previous tile is fully written out
+  for (int i = threadIdx.x; i < w + h; i += kThreads) {
+    if (i < w)
+      aoff[i] = decode32(x.a0 + i, p.na, p.a_div, p.a_ostr);
+    else
+      boff[i - w] = decode32(x.b0 + (i - w), p.nb, p.b_div, p.b_istr);
+  }
+  __syncthreads();
+  const T *s = src + x.oin + x.a0;
+  T r[PER];
+#pragma unroll
+  for (int k = 0; k < PER; ++k) {
+    const uint32_t i = threadIdx.x + k * kThreads;
+    const TileIdx e = read_idx<BATCH>(p, i);
+    if (i < n && in_tile<BATCH>(e, x)) r[k] = s[e.cc * p.c_istr + boff[e.b] + e.a];
+  }
+#pragma unroll
+  for (int k = 0; k < PER; ++k) {
+    const uint32_t i = threadIdx.x + k * kThreads;
+    const TileIdx e = read_idx<BATCH>(p, i);
+    if (i < n && in_tile<BATCH>(e, x)) tile[(e.cc * h + e.b) * ws + e.a] = r[k];
+  }
+  __syncthreads();
+  T *d = dst + x.oout + x.b0;
+#pragma unroll
+  for (int k = 0; k < PER; ++k) {
+    const uint32_t i = threadIdx.x + k * kThreads;
+    const TileIdx e = write_idx<BATCH>(p, i);
+    if (i < n && in_tile<BATCH>(e, x)) r[k] = tile[(e.cc * h + e.b) * ws + e.a];
+  }
+#pragma unroll
+  for (int k = 0; k < PER; ++k) {
+    const uint32_t i = threadIdx.x + k * kThreads;
+    const TileIdx e = write_idx<BATCH>(p, i);
+    if (i < n && in_tile<BATCH>(e, x)) d[e.cc * p.c_ostr + aoff[e.a] + e.b] = r[k];
+  }
+}
+
+// A job of the batched block permute: a block whose innermost axis moves goes in tiles (task
+// range: tile indices), the others element by element in output order, neighbours of the output
+// being neighbours of the input (task range: elements).
+struct BatchJob {
+  int64_t src_off, dst_off;  // elements
+  int32_t tiled, rank;
+  FastDiv div[16];    // gathered: the output's extents, outermost first
+  uint32_t str[16];   // and their input strides
+  TileArgs32 tile;
+};
+
+// Batched block permute: one workgroup per task.  Every block's reads and writes are coalesced,
+// whatever its permutation (the tile in LDS turns one order into the other), and a thread has
+// four loads in flight.  The block permute of an environment update at bond dimension 2048 (1.2 M
+// elements of 8 bytes) takes 7.8 us with tasks of 1024 elements and 10.9 with 4096 (one per CU);
+// element by element with a 32-bit division per axis it took 12.3 us for the blocks of up to 2^15
+// elements and nine launches of 3.4 us for the others.
 template <typename T>
-__global__ __launch_bounds__(kThreads) void k_batch_copy(const BatchCopyJob *__restrict__ jobs,
+__global__ __launch_bounds__(kThreads) void k_batch_copy(const BatchJob *__restrict__ jobs,
                                                          const BatchCopyTask *__restrict__ tasks,
                                                          const T *__restrict__ src,
                                                          T *__restrict__ dst) {
-  __shared__ int32_t ext[16], sstr[16];
+  __shared__ T tile[max_tile<T>() + 64];
+  __shared__ uint32_t aoff[kMaxTile];
+  __shared__ uint32_t boff[kMaxTile];
   const BatchCopyTask tk = tasks[blockIdx.x];
-  const BatchCopyJob *j = jobs + tk.job;
-  const int rank = j->rank;
-  if (threadIdx.x < 16) {
-    ext[threadIdx.x] = threadIdx.x < (unsigned)rank ? j->ext[threadIdx.x] : 1;
-    sstr[threadIdx.x] = threadIdx.x < (unsigned)rank ? j->sstr[threadIdx.x] : 0;
+  const BatchJob &j = jobs[tk.job];
+  const T *s = src + j.src_off;
+  T *d = dst + j.dst_off;
+  if (j.tiled) {  // (uniform)
+    if (j.tile.c > 1)
+      for (int t = 0; t < tk.count; ++t)
+        move_tile<T, true>(s, d, j.tile, tk.start + t, tile, aoff, boff);
+    else
+      for (int t = 0; t < tk.count; ++t)
+        move_tile<T, false>(s, d, j.tile, tk.start + t, tile, aoff, boff);
+    return;
   }
-  __syncthreads();
-  const T *s = src + j->src_off;
-  T *d = dst + j->dst_off;
-  const int end = tk.start + tk.count;
-  for (int e = tk.start + (int)threadIdx.x; e < end; e += kThreads) {
-    int rem = e, off = 0;
-    for (int a = rank - 1; a > 0; --a) {
-      const int q = rem / ext[a];
-      off += (rem - q * ext[a]) * sstr[a];
-      rem = q;
+  constexpr int U = 4;
+  const uint32_t end = tk.start + tk.count;
+  for (uint32_t e0 = tk.start + threadIdx.x; e0 < end; e0 += U * kThreads) {
+    uint32_t in[U];
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      const uint32_t e = e0 + u * kThreads;
+      in[u] = decode32(e < end ? e : e0, j.rank, j.div, j.str);
     }
-    off += rem * sstr[0];
-    d[e] = s[off];
+    T r[U];
+#pragma unroll
+    for (int u = 0; u < U; ++u) r[u] = s[in[u]];
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      const uint32_t e = e0 + u * kThreads;
+      if (e < end) d[e] = r[u];
+    }
   }
 }
 
 }  // namespace
 
-bool batch_copy_job(int rank, const uint64_t *shape, const uint64_t *mapper, int64_t src_off,
-                    int64_t dst_off, BatchCopyJob *job) {
+size_t batch_job_bytes() { return sizeof(BatchJob); }
+
+bool batch_copy_job(int elem_size, int rank, const uint64_t *shape, const uint64_t *mapper,
+                    int64_t src_off, int64_t dst_off, int id, std::vector<char> &jobs,
+                    std::vector<BatchCopyTask> &tasks) {
   if (rank < 0 || rank > 16) return false;
   const Reduced r = reduce_perm(rank, shape, mapper);
   if (r.total > kBatchCopyMaxElems) return false;
-  *job = BatchCopyJob{};
-  job->src_off = src_off;
-  job->dst_off = dst_off;
-  job->n = (int32_t)r.total;
-  job->rank = std::max(1, r.rank);
-  // row-major strides of the reduced old axes, then the new axes' extents and source strides
-  int64_t ostr[16];
-  int64_t acc = 1;
-  for (int i = r.rank - 1; i >= 0; --i) {
-    ostr[i] = acc;
-    acc *= r.shape[i];
+  BatchJob job{};
+  job.src_off = src_off;
+  job.dst_off = dst_off;
+  TileArgs wide;
+  bool small32 = false;
+  if (r.total > 0 && r.rank > 1 && r.perm[r.rank - 1] != r.rank - 1)
+    job.tiled = plan_tiles(elem_size, r, &wide, &job.tile, &small32) && small32;
+  if (!job.tiled) {
+    int64_t ostr[16], acc = 1;
+    for (int i = r.rank - 1; i >= 0; --i) {
+      ostr[i] = acc;
+      acc *= r.shape[i];
+    }
+    job.rank = r.rank;
+    for (int a = 0; a < r.rank; ++a) {
+      job.div[a] = FastDiv::make((uint32_t)std::max<int64_t>(1, r.shape[r.perm[a]]));
+      job.str[a] = (uint32_t)ostr[r.perm[a]];
+    }
   }
-  if (r.rank == 0) {
-    job->ext[0] = (int32_t)r.total;
-    job->sstr[0] = 1;
-    return true;
-  }
-  for (int d = 0; d < r.rank; ++d) {
-    job->ext[d] = (int32_t)r.shape[r.perm[d]];
-    job->sstr[d] = (int32_t)ostr[r.perm[d]];
-  }
+  // tasks of about kBatchCopyTaskElems elements
+  const int32_t n = job.tiled ? (int32_t)job.tile.ntiles : (int32_t)r.total;
+  const int32_t per_tile = job.tiled ? std::max(1, job.tile.w * job.tile.h * job.tile.c) : 1;
+  const int32_t step = std::max(1, kBatchCopyTaskElems / per_tile);
+  for (int32_t at = 0; at < n; at += step)
+    tasks.push_back({id, at, std::min(step, n - at), 0});
+  jobs.insert(jobs.end(), (const char *)&job, (const char *)(&job + 1));
   return true;
 }
 
-int launch_batch_copy(int elem_size, const BatchCopyJob *jobs, const BatchCopyTask *tasks,
-                      int ntasks, const void *src, void *dst, hipStream_t s) {
+int launch_batch_copy(int elem_size, const void *dev_jobs, const BatchCopyTask *tasks, int ntasks,
+                      const void *src, void *dst, hipStream_t s) {
   if (ntasks <= 0) return CXA_OK;
+  const BatchJob *jobs = (const BatchJob *)dev_jobs;
   switch (elem_size) {
     case 4:
       hipLaunchKernelGGL((k_batch_copy<uint32_t>), dim3(ntasks), dim3(kThreads), 0, s, jobs,
@@ -874,7 +978,7 @@ struct cxa_bp_plan {
   std::vector<Big> big;  // blocks moved by cxa_permute one by one
   int ntasks = 0;
   void *dev = nullptr;  // batched jobs, then tasks (256-byte aligned)
-  const cxa::BatchCopyJob *jobs = nullptr;
+  const void *jobs = nullptr;
   const cxa::BatchCopyTask *tasks = nullptr;
   ~cxa_bp_plan() {
     if (dev) (void)hipFree(dev);
@@ -906,49 +1010,40 @@ extern "C" int cxa_block_permute_plan(int dtype, int rank, int64_t nblocks,
   p->es = es;
   p->rank = rank;
   for (int i = 0; i < rank; ++i) p->mapper[i] = mapper[i];
-  std::vector<BatchCopyJob> jobs;
+  std::vector<char> jobs;
   std::vector<BatchCopyTask> tasks;
   std::vector<int64_t> small_ids;  // blocks in the batched launch (two or more of them)
   const bool batched = es == 4 || es == 8 || es == 16;
-  for (int64_t b = 0; b < nblocks; ++b) {
-    CXA_CHECK(src_offsets[b] >= 0 && dst_offsets[b] >= 0, CXA_ERR_INVALID,
-              "cxa_block_permute_plan: negative offset of block %lld", (long long)b);
-    BatchCopyJob j;
-    if (batched &&
-        batch_copy_job(rank, shapes + b * rank, mapper, src_offsets[b], dst_offsets[b], &j)) {
-      small_ids.push_back(b);
-      jobs.push_back(j);
-      continue;
-    }
+  auto alone = [&](int64_t b) {
     cxa_bp_plan::Big g{};
     for (int i = 0; i < rank; ++i) g.shape[i] = shapes[b * rank + i];
     g.src_off = src_offsets[b];
     g.dst_off = dst_offsets[b];
     p->big.push_back(g);
+  };
+  for (int64_t b = 0; b < nblocks; ++b) {
+    CXA_CHECK(src_offsets[b] >= 0 && dst_offsets[b] >= 0, CXA_ERR_INVALID,
+              "cxa_block_permute_plan: negative offset of block %lld", (long long)b);
+    if (batched && batch_copy_job(es, rank, shapes + b * rank, mapper, src_offsets[b],
+                                  dst_offsets[b], (int)small_ids.size(), jobs, tasks))
+      small_ids.push_back(b);
+    else
+      alone(b);
   }
-  if (jobs.size() < 2) {  // a lone small block: the tiled permute moves it faster
-    for (int64_t b : small_ids) {
-      cxa_bp_plan::Big g{};
-      for (int i = 0; i < rank; ++i) g.shape[i] = shapes[b * rank + i];
-      g.src_off = src_offsets[b];
-      g.dst_off = dst_offsets[b];
-      p->big.push_back(g);
-    }
-    jobs.clear();
+  if (small_ids.size() < 2) {  // a lone block: cxa_permute moves it faster
+    for (int64_t b : small_ids) alone(b);
+    tasks.clear();
   }
-  for (size_t id = 0; id < jobs.size(); ++id)
-    for (int32_t at = 0; at < jobs[id].n; at += kBatchCopyTaskElems)
-      tasks.push_back({(int32_t)id, at, std::min(kBatchCopyTaskElems, jobs[id].n - at), 0});
   if (!tasks.empty()) {
-    const size_t nj = (jobs.size() * sizeof(BatchCopyJob) + 255) / 256 * 256;
+    const size_t nj = (jobs.size() + 255) / 256 * 256;
     const size_t nt = tasks.size() * sizeof(BatchCopyTask);
     std::vector<char> host(nj + nt, 0);
-    std::memcpy(host.data(), jobs.data(), jobs.size() * sizeof(BatchCopyJob));
+    std::memcpy(host.data(), jobs.data(), jobs.size());
     std::memcpy(host.data() + nj, tasks.data(), nt);
     CXA_HIP(hipMalloc(&p->dev, host.size()));
     const int rc = upload_now(p->dev, host.data(), host.size());
     if (rc) return rc;
-    p->jobs = (const BatchCopyJob *)p->dev;
+    p->jobs = p->dev;
     p->tasks = (const BatchCopyTask *)((char *)p->dev + nj);
     p->ntasks = (int)tasks.size();
   }

@@ -75,7 +75,7 @@ int cxa_permute(int dtype, int rank, const uint64_t *old_shape, const uint64_t *
  * permutes block by block).  Block b is the row-major array of extents shapes[b*rank ..] at
  * element offset src_offsets[b] of src; its permuted copy (axis j = old axis mapper[j]) goes to
  * element offset dst_offsets[b] of dst.  The plan is built once from the metadata (host): blocks
- * of up to 2^15 elements of 4-, 8- or 16-byte dtypes are moved by one batched launch when there
+ * of up to 2^20 elements of 4-, 8- or 16-byte dtypes are moved by one batched launch when there
  * are two or more of them, the others by cxa_permute each.  exec enqueues on `stream`; dst must
  * not overlap src.  A plan with batched blocks holds their task list in the memory of the
  * device current at its creation and runs there only.
