@@ -155,7 +155,7 @@ def contract_ad(A: UniTensor, B: UniTensor) -> UniTensor:
     # one made for the same structure (a sweep contracts the same structures again and again)
     key = (dt, dev, A._itoi.tobytes(), A._shapes.tobytes(), B._itoi.tobytes(),
            B._shapes.tobytes(), tuple(c1), tuple(c2),
-           tuple((b._type, tuple(b._qnums), tuple(b._degs), b._dim) for b in out_bonds))
+           tuple((b._type, b._qnums, b._degs, b._dim) for b in out_bonds))
     hit = _OUTS.get(key)
     if hit is None:
         if out_bonds:

@@ -1294,19 +1294,32 @@ extern "C" int cxa_gemm_batch(int dtype, const char *transa, const char *transb,
   const int cls = make_tiles(blks, segs, tiles, &per_xcd, tl.kind, !cplx);
   if (tiles.empty()) return CXA_OK;
   hipStream_t s = (hipStream_t)stream;
-  DevBuf d_blks, d_segs, d_tiles;
-  int rc;
-  if ((rc = upload(d_blks, blks)) || (rc = upload(d_segs, segs)) || (rc = upload(d_tiles, tiles)))
-    return rc;
+  // the task arrays in one block of the library's pool and one copy (three allocations, copies
+  // and frees took half of a call's host time)
+  const size_t nb = (blks.size() * sizeof(GBlk) + 255) / 256 * 256;
+  const size_t ns = (segs.size() * sizeof(GSeg) + 255) / 256 * 256;
+  const size_t nt = tiles.size() * sizeof(GTile);
+  std::vector<char> host(nb + ns + nt, 0);
+  std::memcpy(host.data(), blks.data(), blks.size() * sizeof(GBlk));
+  if (!segs.empty()) std::memcpy(host.data() + nb, segs.data(), segs.size() * sizeof(GSeg));
+  std::memcpy(host.data() + nb + ns, tiles.data(), nt);
+  struct Block {
+    char *p = nullptr;
+    ~Block() {
+      if (p) pool_release(p);
+    }
+  } dev;
+  int rc = pool_alloc((void **)&dev.p, host.size());
+  if (rc || (rc = upload_now(dev.p, host.data(), host.size()))) return rc;
   GemmLaunch g;
   g.prec = (dtype == CXA_F64 || dtype == CXA_C128) ? CXA_PREC_FP64 : CXA_PREC_FP32;
   g.a_dt = g.b_dt = g.c_dt = dtype;
   g.A = nullptr;  // absolute addresses (in elements) are carried in the offsets
   g.B = nullptr;
   g.C = nullptr;
-  g.tiles = (const GTile *)d_tiles.p;
-  g.blks = (const GBlk *)d_blks.p;
-  g.segs = (const GSeg *)d_segs.p;
+  g.tiles = (const GTile *)(dev.p + nb + ns);
+  g.blks = (const GBlk *)dev.p;
+  g.segs = (const GSeg *)(dev.p + nb);
   g.ntiles = (int)tiles.size();
   g.per_xcd = per_xcd;
   g.tile_class = cls;
@@ -1314,7 +1327,7 @@ extern "C" int cxa_gemm_batch(int dtype, const char *transa, const char *transb,
   g.splitk = tl.split;
   rc = launch_grouped_gemm(g, s);
   if (rc) return rc;
-  // the task arrays are freed on return: wait for the launch that reads them
+  // the task arrays go back to the pool on return: wait for the launch that reads them
   CXA_HIP(hipStreamSynchronize(s));
   return CXA_OK;
 }

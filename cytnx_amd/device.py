@@ -73,4 +73,6 @@ def torch_device(dev: int) -> torch.device:
 
 def stream_handle(dev: int = 0) -> int:
     """hipStream_t of torch's current stream on ``dev`` (an int for ctypes)."""
-    return torch.cuda.current_stream(dev).cuda_stream
+    if not torch.cuda.is_initialized():
+        torch.cuda.init()
+    return torch._C._cuda_getCurrentRawStream(dev)

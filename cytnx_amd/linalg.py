@@ -101,8 +101,7 @@ def Tensordot(Tl: Tensor, Tr: Tensor, idxl: Sequence[int], idxr: Sequence[int],
                                sl, B.storage().data_ptr(), B.rank(), sr, len(idxl), il, ir,
                                wbuf.data_ptr() if wbuf is not None else None,
                                stream_handle(dev)))
-    if wbuf is not None:
-        torch.cuda.current_stream(dev).synchronize()  # keep the workspace alive until done
+    # (wbuf comes from this stream's pool: its memory goes to later work on this stream only)
     return out
 
 
@@ -118,54 +117,46 @@ def Gemm_Batch(alpha: Sequence[complex], a: Sequence[Tensor], b: Sequence[Tensor
         raise ValueError("[Gemm_Batch] alpha/beta need one entry per group")
     dev = _require_device(*a, *b, *c)
     dt = c[0].dtype()
-    ms, ns, ks, lda, ldb, ldc = [], [], [], [], [], []
+    td = TORCH_OF[dt]
+    # row-major -> BLAS column-major: pass B before A, n before m (Gemm_Batch.cpp:210-230)
+    ms, ns, ks, flat_a, flat_b, flat_c = [], [], [], [], [], []
+    alphas, betas = [], []
     idx = 0
     for g, gs in enumerate(group_size):
         for _ in range(gs):
             A, B, C = a[idx], b[idx], c[idx]
             for t in (A, B, C):
-                if t.dtype() != dt or not t.is_contiguous() or t.rank() != 2:
+                if t._storage.dtype != td or not t._contiguous or len(t._shape) != 2:
                     raise ValueError("[Gemm_Batch] operands must be contiguous rank-2 tensors "
                                      "of one dtype")
-            if A.shape()[1] != B.shape()[0] or C.shape() != [A.shape()[0], B.shape()[1]]:
+            (M, K), (Kb, N) = A._shape, B._shape
+            if K != Kb or C._shape[0] != M or C._shape[1] != N:
                 raise ValueError("[Gemm_Batch] shape mismatch in batch entry %d" % idx)
-            idx += 1
-    # row-major -> BLAS column-major: pass B before A, n before m (Gemm_Batch.cpp:210-230)
-    flat_a, flat_b, flat_c = [], [], []
-    alphas, betas, gsz = [], [], []
-    idx = 0
-    for g, gs in enumerate(group_size):
-        for _ in range(gs):
-            A, B, C = a[idx], b[idx], c[idx]
-            M, K = A.shape()
-            N = B.shape()[1]
             ms.append(N), ns.append(M), ks.append(K)
-            lda.append(N), ldb.append(K), ldc.append(N)
-            flat_a.append(B.storage().data_ptr())
-            flat_b.append(A.storage().data_ptr())
-            flat_c.append(C.storage().data_ptr())
-            alphas.append(alpha[g])
-            betas.append(beta[g])
-            gsz.append(1)
+            flat_a.append(B._storage.data_ptr())
+            flat_b.append(A._storage.data_ptr())
+            flat_c.append(C._storage.data_ptr())
             idx += 1
-    cnt = len(gsz)
+        alphas += [alpha[g]] * gs
+        betas += [beta[g]] * gs
+    cnt = idx  # (lda = ldc = n, ldb = k)
     VP = ctypes.c_void_p * max(1, cnt)
     if dt in (1, 2):  # complex: (re, im) per group
         def pairs(v):
             return [float(x) for z in v for x in (complex(z).real, complex(z).imag)]
         alphas, betas = pairs(alphas), pairs(betas)
     else:
-        for z in list(alphas) + list(betas):
-            if complex(z).imag != 0:
-                raise ValueError("[Gemm_Batch] complex alpha/beta need complex operands")
-        alphas = [complex(z).real for z in alphas]
-        betas = [complex(z).real for z in betas]
+        alphas, betas = [complex(z) for z in alphas], [complex(z) for z in betas]
+        if any(z.imag != 0 for z in alphas + betas):
+            raise ValueError("[Gemm_Batch] complex alpha/beta need complex operands")
+        alphas, betas = [z.real for z in alphas], [z.real for z in betas]
     D = ctypes.c_double * max(1, len(alphas))
     tr = b"N" * max(1, cnt)
+    I = ctypes.c_int64 * max(1, cnt)
+    cm, ck = I(*ms), I(*ks)
     _lib.check(_lib.lib().cxa_gemm_batch(
-        dt, tr, tr, _lib.i64_array(ms), _lib.i64_array(ns), _lib.i64_array(ks), D(*alphas),
-        VP(*flat_a), _lib.i64_array(lda), VP(*flat_b), _lib.i64_array(ldb), D(*betas),
-        VP(*flat_c), _lib.i64_array(ldc), cnt, _lib.i64_array(gsz), stream_handle(dev)))
+        dt, tr, tr, cm, I(*ns), ck, D(*alphas), VP(*flat_a), cm, VP(*flat_b), ck, D(*betas),
+        VP(*flat_c), cm, cnt, I(*[1] * cnt), stream_handle(dev)))
 
 
 _VEC_WS = {}

@@ -36,15 +36,16 @@ class Bond:
     def __init__(self, btype_or_dim, qnums=None, degs=None):
         if qnums is None:
             self._type = BD_REG
-            self._qnums: List[int] = []
-            self._degs: List[int] = []
+            self._qnums: Tuple[int, ...] = ()
+            self._degs: Tuple[int, ...] = ()
             self._dim = int(btype_or_dim)
         else:
             self._type = int(btype_or_dim)
             if self._type == BD_REG:
                 raise ValueError("a bond with qnums must be KET or BRA")
-            self._qnums = [int(q[0]) if isinstance(q, (list, tuple)) else int(q) for q in qnums]
-            self._degs = [int(d) for d in (degs if degs is not None else [1] * len(qnums))]
+            self._qnums = tuple(int(q[0]) if isinstance(q, (list, tuple)) else int(q)
+                                for q in qnums)
+            self._degs = tuple(int(d) for d in (degs if degs is not None else [1] * len(qnums)))
             if len(self._degs) != len(self._qnums):
                 raise ValueError("qnums and degeneracies differ in length")
             self._dim = int(sum(self._degs))
@@ -71,8 +72,7 @@ class Bond:
 
     def clone(self) -> "Bond":
         b = Bond.__new__(Bond)
-        b._type, b._qnums, b._degs, b._dim = self._type, list(self._qnums), list(self._degs), \
-            self._dim
+        b._type, b._qnums, b._degs, b._dim = self._type, self._qnums, self._degs, self._dim
         return b
 
     def __eq__(self, other) -> bool:
@@ -84,7 +84,7 @@ class Bond:
         if not self._qnums:
             return "Bond(dim=%d)" % self._dim
         return "Bond(%s, qnums=%s, degs=%s)" % ("KET" if self._type == BD_KET else "BRA",
-                                               self._qnums, self._degs)
+                                               list(self._qnums), list(self._degs))
 
 
 def enumerate_blocks(bonds: Sequence[Bond]) -> np.ndarray:
@@ -239,6 +239,27 @@ def _block_layout(bonds: Sequence[Bond], itoi: np.ndarray) -> Tuple[np.ndarray, 
     return shapes, offsets, total
 
 
+_LAYOUTS: Dict[tuple, Tuple[np.ndarray, np.ndarray, np.ndarray, int]] = {}
+
+
+def _layout_of(bonds: Sequence[Bond]) -> Tuple[np.ndarray, np.ndarray, np.ndarray, int]:
+    """(itoi, shapes, offsets, elements) of the zero-flux blocks over ``bonds``.  A sweep makes
+    tensors over the same legs again and again, and enumerating 170 blocks takes 50 us of host
+    time: the arrays, read-only and shared, are kept by the legs' structure."""
+    key = tuple((b._type, b._qnums, b._degs) for b in bonds)
+    hit = _LAYOUTS.get(key)
+    if hit is None:
+        itoi = enumerate_blocks(bonds)
+        shapes, offsets, total = _block_layout(bonds, itoi)
+        for a in (itoi, shapes, offsets):
+            a.setflags(write=False)
+        hit = (itoi, shapes, offsets, total)
+        if len(_LAYOUTS) > 4096:
+            _LAYOUTS.clear()
+        _LAYOUTS[key] = hit
+    return hit
+
+
 class UniTensor:
     """Dense or U(1)-block UniTensor.
 
@@ -267,8 +288,7 @@ class UniTensor:
         if self._is_block:
             nket = sum(1 for b in self._bonds if b.type() == BD_KET)
             self._rowrank = nket if rowrank == -1 else int(rowrank)
-            self._itoi = enumerate_blocks(self._bonds)
-            self._shapes, self._offsets, total = _block_layout(self._bonds, self._itoi)
+            self._itoi, self._shapes, self._offsets, total = _layout_of(self._bonds)
             self._storage = torch.zeros(total if _alloc else 0, dtype=TORCH_OF[dtype],
                                         device=torch_device(device))
             self._block = None
@@ -807,9 +827,9 @@ def _contract_pair(A: UniTensor, B: UniTensor) -> UniTensor:
         raise NotImplementedError("block contraction runs on one GPU; move both operands there")
     out = UniTensor(out_bonds, out_labels, max(0, min(rr, len(out_bonds))), dt, dev,
                     _alloc=False) if out_bonds else _scalar_block(dt, dev)
-    out._storage = torch.empty(int(np.sum(np.prod(out._shapes.astype(np.int64), axis=1)))
-                               if out.Nblocks() and out.rank() else max(1, out.Nblocks()),
-                               dtype=TORCH_OF[dt], device=torch_device(dev))
+    n = int(out._offsets[-1]) + int(out._shapes[-1].prod()) if out.Nblocks() and out.rank() \
+        else max(1, out.Nblocks())
+    out._storage = torch.empty(n, dtype=TORCH_OF[dt], device=torch_device(dev))
     plan = _plan_for(dt, A, B, c1, c2, out)
     _lib.check(_lib.lib().cxa_block_contract_exec(
         plan.handle, A._storage.data_ptr(), B._storage.data_ptr(), out._storage.data_ptr(),
