@@ -136,12 +136,16 @@ int make_tiles(const std::vector<GBlk> &blks, const std::vector<GSeg> &segs,
       kind = kind_override;
     else
       kind = default_kind(b.M, b.N);
-    const int tr = tile_rows(kind), tc = kind == TK_ROWS ? b.N : tile_cols(kind);
     int64_t ksum = 0;
     for (int s = 0; s < b.nseg; ++s) ksum += segs[b.seg0 + s].K;
+    int tr = tile_rows(kind), tc = kind == TK_ROWS ? b.N : tile_cols(kind);
+    // rows of short K (the MPO steps, K of a few): a wave's four loads and stores take less than
+    // reading its tile, block and segment records, so it takes four times the rows
+    if (kind == TK_ROWS && ksum <= kShortRowsK && b.N <= kShortRowsN && b.M > tr)
+      tr *= kShortRows;
     for (int m0 = 0; m0 < b.M; m0 += tr)
       for (int n0 = 0; n0 < b.N; n0 += tc)
-        items.push_back({GTile{(int32_t)bi, m0, n0, kind}, (ksum + 16) * tr * tc});
+        items.push_back({GTile{(int32_t)bi, m0, kind == TK_ROWS ? tr : n0, kind}, (ksum + 16) * tr * tc});
   }
   // kXcds contiguous ranges of equal tile count (at these sizes a tile's time is mostly its
   // fixed chain of dependent loads, so equal counts balance better than equal flops, and the

@@ -66,9 +66,11 @@ inline int tile_cols(int kind) {
 }
 
 constexpr int kRowsN = 8;  // widest block the row-streaming path takes
+// Rows per lane of a row tile with short K, and the K and N up to which it is taken.
+constexpr int kShortRows = 4, kShortRowsK = 32, kShortRowsN = 4;
 
 struct GTile {
-  int32_t blk, m0, n0, kind;
+  int32_t blk, m0, n0, kind;  // (TK_ROWS: n0 is the tile's rows, 64 or 64 * kShortRows)
 };
 
 struct GemmLaunch {

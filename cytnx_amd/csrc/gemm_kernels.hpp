@@ -890,6 +890,91 @@ __device__ __forceinline__ void wave_rows(const char *__restrict__ Abase,
     if (n < blk.N) store_c(Cp + n * blk.csn, acc[n], blk);
 }
 
+// Row tile of short K: kShortRows rows per lane (64 apart), N <= kShortRowsN.  Bound by the chain
+// of dependent loads (records, then B, then A) and by its stores: the A values of four k run
+// ahead for all rows, B comes through scalar loads, and where the block is contiguous in C its
+// rows are put together in LDS, so that the stores are.  `out`: kShortRows * 64 * kShortRowsN
+// values of this wave.  The MPO step of an environment update at bond dimension 2048 (19 MB
+// written, K of 1 to 4, N of 1 or 3): 22.2 us with one row per lane, @@ us so.
+template <typename TA, typename TB, typename TC, int PK, typename SEGS>
+__device__ __forceinline__ void wave_rows_short(const char *__restrict__ Abase,
+                                                const char *__restrict__ Bbase,
+                                                char *__restrict__ Cbase, const GBlk &blk,
+                                                SEGS segs, int m0, int lane, double *out) {
+  constexpr int R = kShortRows, NB = kShortRowsN, D = 4;
+  const int N = blk.N;
+  int total = 0;
+  for (int s = 0; s < blk.nseg; ++s) total += segs(blk.seg0 + s).K;
+  double acc[R][NB];
+#pragma unroll
+  for (int q = 0; q < R; ++q)
+#pragma unroll
+    for (int n = 0; n < NB; ++n) acc[q][n] = 0.0;
+  if (total > 0) {
+    RowCursor<SEGS> lc{segs, blk.seg0, blk.nseg, 0, 0};
+    lc.sg = segs(blk.seg0);
+    lc.skip(0);
+    TA a[D][R];
+    TB b[D][NB];
+    auto load = [&](int d) {
+      gptr<const TA> ak = at<const TA>(Abase, lc.sg.a_off) + a_koff<PK>(lc.k, lc.sg.sak);
+      typedef const TB __attribute__((address_space(4))) *sptr;  // uniform: scalar loads
+      const sptr bk = (sptr)(at<const TB>(Bbase, lc.sg.b_off) +
+                             ((PK & kPackB) ? (int64_t)(lc.k >> 2) * lc.sg.sbk + (lc.k & 3)
+                                            : (int64_t)lc.k * lc.sg.sbk));
+#pragma unroll
+      for (int q = 0; q < R; ++q) {
+        const int row = m0 + 64 * q + lane;
+        a[d][q] = load_or_zero<TA>(ak + (int64_t)row * lc.sg.sam, row < blk.M);
+      }
+#pragma unroll
+      for (int n = 0; n < NB; ++n) b[d][n] = bk[n < N ? (int64_t)n * lc.sg.sbn : 0];
+    };
+#pragma unroll
+    for (int d = 0; d < D; ++d)
+      if (d < total) {
+        load(d);
+        lc.skip(1);
+      }
+    for (int base = 0; base < total; base += D) {
+#pragma unroll
+      for (int d = 0; d < D; ++d) {
+        if (base + d >= total) break;
+#pragma unroll
+        for (int n = 0; n < NB; ++n)
+#pragma unroll
+          for (int q = 0; q < R; ++q) acc[q][n] += (double)a[d][q] * (double)b[d][n];
+        if (base + d + D < total) {
+          load(d);
+          lc.skip(1);
+        }
+      }
+    }
+    drain_loads();
+  }
+  gptr<TC> Cp = at<TC>(Cbase, blk.c_off) + (int64_t)m0 * blk.ldc;
+  const int rows = min(64 * R, blk.M - m0);
+  if (blk.csn == 1 && blk.ldc == N) {
+    __builtin_amdgcn_wave_barrier();  // the last tile's reads
+#pragma unroll
+    for (int q = 0; q < R; ++q)
+#pragma unroll
+      for (int n = 0; n < NB; ++n)
+        if (n < N) out[(64 * q + lane) * N + n] = acc[q][n];
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    for (int e = lane; e < rows * N; e += 64) store_c(Cp + e, out[e], blk);
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+  } else {
+#pragma unroll
+    for (int q = 0; q < R; ++q)
+#pragma unroll
+      for (int n = 0; n < NB; ++n)
+        if (64 * q + lane < rows && n < N)
+          store_c(Cp + ((int64_t)(64 * q + lane) * blk.ldc + n * blk.csn), acc[q][n], blk);
+  }
+}
+
 // Split-K row tile: the four waves take interleaved k values of the same 64 rows.
 template <typename TA, typename TB, typename TC, int PK, typename SEGS>
 __device__ __forceinline__ void wg_rows(const char *__restrict__ Abase,
@@ -1072,6 +1157,13 @@ __global__ __launch_bounds__(64 * kWaves, 2) void k_grouped(const GTile *__restr
       continue;
     }
     const GBlk blk = blks[tl.blk];
+    if constexpr (CLS == TC_ROWS) {
+      __shared__ double out[kWaves][kShortRows * 64 * kShortRowsN];
+      if (tl.n0 > 64) {  // (uniform over the wave)
+        wave_rows_short<TA, TB, TC, PK>(A, B, C, blk, SegArray{segs}, tl.m0, lane, out[wave]);
+        continue;
+      }
+    }
     run_tile<PREC, TA, TB, TC, CPLX, CLS, PK>(tl.kind, A, B, C, blk, SegArray{segs}, tl.m0,
                                                tl.n0, lane, conj, dotx, dslot,
                                                (int64_t)kXcds * per_xcd);
@@ -1102,7 +1194,8 @@ __global__ __launch_bounds__(64 * WAVES, 2) void k_grouped_split(
     const GBlk blk = blks[tl.blk];
     const SegArray sa{segs};
     if constexpr (CLS == TC_ROWS) {
-      wg_rows<TA, TB, TC, PK>(A, B, C, blk, sa, tl.m0, lane, wave, red);
+      for (int m = tl.m0; m < min(blk.M, tl.m0 + tl.n0); m += 64)
+        wg_rows<TA, TB, TC, PK>(A, B, C, blk, sa, m, lane, wave, red);
     } else {
       switch (tl.kind) {
         case TK_1x1:
