@@ -86,11 +86,14 @@ void seal_block(GBlk &b, const GSeg *segs) {
   // the elements of a tile's chunk: up to 64 rows and 16 k, of up to 16 bytes
   const int64_t lim = int64_t(1) << 31;
   int64_t chunks = 0;
-  b.wide = 0;
+  b.wide = kContigA | kContigB;
   for (int i = b.seg0; i < b.seg0 + b.nseg; ++i) {
     const GSeg &s = segs[i];
     chunks += (s.K + 15) / 16;
-    if (16 * (64 * s.sam + 16 * s.sak) >= lim || 16 * (64 * s.sbn + 16 * s.sbk) >= lim) b.wide = 1;
+    if (16 * (64 * s.sam + 16 * s.sak) >= lim || 16 * (64 * s.sbn + 16 * s.sbk) >= lim)
+      b.wide |= kWideStrides;
+    if (s.sak != 1) b.wide &= ~kContigA;
+    if (s.sbk != 1) b.wide &= ~kContigB;
   }
   b.chunks = (int32_t)std::min<int64_t>(chunks, INT32_MAX);
 }

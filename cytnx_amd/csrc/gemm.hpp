@@ -35,8 +35,11 @@ struct GBlk {
   int32_t out0, nout;  // mix launches only: the item's outputs (MixOut)
   double alpha_im, beta_im;  // imaginary parts of alpha / beta (complex dtypes only)
   int32_t chunks;  // 16-deep K chunks of all segments (set by seal_blocks)
-  int32_t wide;    // a segment's strides are too large for 32-bit offsets in a direct tile
+  int32_t wide;    // what holds of its segments' strides (kWideStrides, kContigA, kContigB)
 };
+// A segment's strides are too large for 32-bit offsets in a direct tile; K is the contiguous index
+// of A, of B, in every segment.
+constexpr int kWideStrides = 1, kContigA = 2, kContigB = 4;
 
 // Mix launches (a grouped GEMM with a linear-combination epilogue).  An item is a GBlk whose
 // segments are separate products ("slices") X_s = A_s B_s of one M x N shape; the item writes

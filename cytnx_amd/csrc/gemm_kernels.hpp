@@ -381,9 +381,12 @@ struct ChunkCursor {
 
 // One operand's part of a wave's chunks: NR groups of 16 rows (A's m or B's n), one row per lane
 // and group, 4 consecutive k.
-template <typename T, int NR, bool QUAD>
+// WIDE: k is the contiguous index, and a lane's 4 k come in one or two 16-byte loads (which need
+// no more than 4-byte alignment) where 4 loads would each touch the cache lines of all 16 rows.
+// The last, partial chunk of a segment goes by elements: what lies past K may be anything.
+template <typename T, int NR, bool QUAD, bool WIDE>
 struct ChunkSide {
-  using qe = typename std::conditional<QUAD, T, float>::type;  // (packed operands are real)
+  using qe = typename std::conditional<QUAD || WIDE, T, float>::type;  // (real operands)
   typedef qe t4 __attribute__((ext_vector_type(4)));
   uint64_t base;     // address of (row 0, k 0) of the next chunk (uniform)
   int64_t adv;       // bytes from chunk to chunk (uniform)
@@ -417,6 +420,19 @@ struct ChunkSide {
         v[i][3] = x.w;
       }
     } else {
+      if constexpr (WIDE) {
+        if (kleft >= 16) {  // (uniform)
+#pragma unroll
+          for (int i = 0; i < NR; ++i) {
+            const t4 x = buffer_get<t4>(rs, off[i], 0);
+            v[i][0] = x.x;
+            v[i][1] = x.y;
+            v[i][2] = x.z;
+            v[i][3] = x.w;
+          }
+          return;
+        }
+      }
 #pragma unroll
       for (int j = 0; j < 4; ++j)
 #pragma unroll
@@ -428,14 +444,15 @@ struct ChunkSide {
 
 // The chunks of a wave in order, like ChunkCursor, for tiles whose addresses fit 32-bit offsets.
 // Past the last chunk every load reads zeros.  ONE: the block has a single segment.
-template <typename TA, typename TB, int MI, int NI, int PK, bool ONE, typename SEGS>
+// W: sides read with wide loads (bit 0 A, bit 1 B).
+template <typename TA, typename TB, int MI, int NI, int PK, bool ONE, int W, typename SEGS>
 struct ChunkStream {
   SEGS segs;
   int seg0, nseg, step, m0, n0, mt, nt, r, g;
   int s, k0, K;  // current segment, chunk start within it, and its extent
   GSeg nx;       // the next segment, read while this one's chunks run
-  ChunkSide<TA, MI, (PK & kPackA) != 0> a;
-  ChunkSide<TB, NI, (PK & kPackB) != 0> b;
+  ChunkSide<TA, MI, (PK & kPackA) != 0, (W & 1) != 0> a;
+  ChunkSide<TB, NI, (PK & kPackB) != 0, (W & 2) != 0> b;
   // to the chunk `first` chunks from the start (nseg > 0)
   __device__ __forceinline__ void start(int first, const char *Abase, const char *Bbase) {
     s = 0;
@@ -560,7 +577,7 @@ __device__ __forceinline__ void mfma_accumulate(ACC &acc,
   const int nt = min(16 * NI, blk.N - n0);
   const int total = (blk.chunks - slice + nslices - 1) / nslices;
   if (total <= 0) return;
-  if (blk.wide) {
+  if (blk.wide & kWideStrides) {
     ChunkCursor<TA, TB, SEGS> cur{segs, blk.seg0, blk.nseg, nslices, m0, n0, 0, 0};
     cur.enter(Abase, Bbase);
     cur.skip(slice, Abase, Bbase);  // also steps over empty leading segments
@@ -573,14 +590,28 @@ __device__ __forceinline__ void mfma_accumulate(ACC &acc,
     drain_loads();
     return;
   }
-  ChunkStream<TA, TB, MI, NI, PK, std::is_same<SEGS, SegOne>::value, SEGS> st{
-      segs, blk.seg0, blk.nseg, nslices, m0, n0, mt, nt, r, g};
-  st.start(slice, Abase, Bbase);
-  constexpr int D = ACC::depth;
-  Frag<TA, TB, MI, NI> f[D];
-  run_chunks<D, std::is_same<SEGS, SegOne>::value>(
-      total, [&](int d) { st.load(f[d]); }, [&]() { st.next(Abase, Bbase); },
-      [&](int d) { mma_frag(acc, f[d]); });
+  auto run = [&](auto w) {
+    ChunkStream<TA, TB, MI, NI, PK, std::is_same<SEGS, SegOne>::value, decltype(w)::value, SEGS>
+        st{segs, blk.seg0, blk.nseg, nslices, m0, n0, mt, nt, r, g};
+    st.start(slice, Abase, Bbase);
+    constexpr int D = ACC::depth;
+    Frag<TA, TB, MI, NI> f[D];
+    run_chunks<D, std::is_same<SEGS, SegOne>::value>(
+        total, [&](int d) { st.load(f[d]); }, [&]() { st.next(Abase, Bbase); },
+        [&](int d) { mma_frag(acc, f[d]); });
+  };
+  // The loads' widths are fixed per pipeline (a choice between them at every chunk would cost the
+  // exact waits); unpacked real operands only, one side at a time.
+  if constexpr (PK == 0 && std::is_arithmetic<TA>::value) {
+    if (blk.wide & kContigA)
+      run(std::integral_constant<int, 1>{});
+    else if (blk.wide & kContigB)
+      run(std::integral_constant<int, 2>{});
+    else
+      run(std::integral_constant<int, 0>{});
+  } else {
+    run(std::integral_constant<int, 0>{});
+  }
 }
 
 template <typename TC>
@@ -895,7 +926,7 @@ __device__ __forceinline__ void wave_rows(const char *__restrict__ Abase,
 // ahead for all rows, B comes through scalar loads, and where the block is contiguous in C its
 // rows are put together in LDS, so that the stores are.  `out`: kShortRows * 64 * kShortRowsN
 // values of this wave.  The MPO step of an environment update at bond dimension 2048 (19 MB
-// written, K of 1 to 4, N of 1 or 3): 22.2 us with one row per lane, @@ us so.
+// written, K of 1 to 4, N of 1 or 3): 21.4 us with one row per lane, 12.6 us so.
 template <typename TA, typename TB, typename TC, int PK, typename SEGS>
 __device__ __forceinline__ void wave_rows_short(const char *__restrict__ Abase,
                                                 const char *__restrict__ Bbase,
@@ -1331,7 +1362,7 @@ __device__ __forceinline__ void mfma_accumulate_multi(RealAcc<PREC, MI, NI> (&ac
     drain_loads();
     return;
   }
-  ChunkStream<TA, TB, MI, NI, PK, NACC == 1, SEGS> st{segs, 0, nseg, 1, m0, n0, mt, nt, r, g};
+  ChunkStream<TA, TB, MI, NI, PK, NACC == 1, 0, SEGS> st{segs, 0, nseg, 1, m0, n0, mt, nt, r, g};
   st.start(0, Abase, Bbase);
   Frag<TA, TB, MI, NI> f[D];
   run_chunks<D, NACC == 1>(
@@ -1370,7 +1401,7 @@ __global__ __launch_bounds__(64 * WAVES, MI *NI == 4 && WAVES == 4 ? 2 : 4) void
       for (int q = 0; q < NACC; ++q) acc[q].zero();
       mfma_accumulate_multi<PREC, TA, TB, MI, NI, NACC, PK>(
           acc, A, B, SegStride{slices, it.seg0 + wave, WAVES}, mine, it.M, it.N, tl.m0, tl.n0,
-          lane, it.wide != 0);
+          lane, (it.wide & kWideStrides) != 0);
 #pragma unroll
       for (int q = 0; q < NACC; ++q) {
         const int sl = wave + q * WAVES;
