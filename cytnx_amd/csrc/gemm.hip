@@ -51,7 +51,7 @@ constexpr int64_t kFewReal = 512, kFewCplx = 1024, kMany64 = 192;
 }  // namespace
 
 Tiling default_tiling(const std::vector<GBlk> &blks, const std::vector<GSeg> &segs, bool cplx) {
-  int64_t n16 = 0, n64 = 0, work = 0;
+  int64_t n16 = 0, n64 = 0, work = 0, pad64 = 0, pad32 = 0;
   bool narrow = !cplx, lds = true;
   for (const GBlk &b : blks) {
     if (b.M <= 0 || b.N <= 0) continue;
@@ -60,7 +60,10 @@ Tiling default_tiling(const std::vector<GBlk> &blks, const std::vector<GSeg> &se
     n64 += tiles_of(b, 64);
     if (b.N > kRowsN) narrow = false;
     for (int s = b.seg0; s < b.seg0 + b.nseg; ++s) {
-      work += t * ((segs[s].K + 15) / 16);
+      const int64_t chunks = (segs[s].K + 15) / 16;
+      work += t * chunks;
+      pad64 += 16 * tiles_of(b, 64) * chunks;
+      pad32 += 4 * tiles_of(b, 32) * chunks;
       lds = lds && lds_ok(b, segs[s]);
     }
   }
@@ -70,7 +73,12 @@ Tiling default_tiling(const std::vector<GBlk> &blks, const std::vector<GSeg> &se
   if (work <= 2 * n16) return {narrow || n16 > 4 * kFewReal ? -1 : (int)TK_1x1, 0};
   if (n16 <= (cplx ? kFewCplx : kFewReal)) return {TK_1x1, 4};
   if (!lds || narrow) return {-1, 0};
-  return {!cplx && n64 >= kMany64 ? TK_L64 : TK_L32, 0};
+  if (cplx || n64 < kMany64) return {TK_L32, 0};
+  // Ragged blocks: 64x64 tiles that cover much more than 32x32 ones lose it again.  Real blocks
+  // of 160 x 160, K = 400, 120 of them (1.44 times the area): direct 32x32 tiles 59 us in FP64 and
+  // 34 in FP32, 64x64 79 and 54; of 300 x 300 (the same area), 60 of them: 111 and 60 against 90
+  // and 61.
+  return {20 * pad64 > 23 * pad32 ? TK_2x2 : TK_L64, 0};
 }
 
 // One block of one segment (a dense product): the same rule with the whole K in one segment.  A
