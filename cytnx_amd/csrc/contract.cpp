@@ -115,6 +115,9 @@ struct cxa_bc_plan {
 namespace cxa {
 namespace {
 
+// 16x16 tiles from which a mix launch takes larger ones by itself (build_variant)
+constexpr int64_t kManyMix = 2400;
+
 // tile kinds a mix launch can run (every slice of an item stays in the wave's registers)
 bool mix_kind_ok(int kind) {
   return kind == TK_1x1 || kind == TK_2x1 || kind == TK_1x2 || kind == TK_2x2;
@@ -127,9 +130,23 @@ int build_variant(cxa_bc_plan *p, int prec) {
   // the host tile list lives only until it is uploaded: one buffer per thread keeps its pages
   thread_local std::vector<GTile> tiles;
   if (p->mix) {
-    v.launch_kind = mix_kind_ok(v.kind) ? v.kind : TK_1x1;
+    // By itself: 16x16 tiles with a wave per slice while their workgroups fill the chip only a few
+    // times, larger tiles (less operand traffic) beyond; the sums are the same.  Two-site matvec
+    // at bond dimension 2048, 3035 tiles of 16x16: FP64 54.6 us, as 32x32 48.2; FP32 39.3 us, as
+    // 16x32 on four waves 34.6.  At 1448, 1722 tiles: FP64 29.1 and 32.2, FP32 19.4 and 20.3.
+    int own = TK_1x1, own_split = 0;
+    if (v.kind < 0 && v.split_mode < 0 && prec != CXA_PREC_FP32X3) {
+      int64_t n16 = 0;
+      for (const GBlk &b : p->blks) n16 += (int64_t)((b.M + 15) / 16) * ((b.N + 15) / 16);
+      if (n16 >= kManyMix) {
+        own = prec == CXA_PREC_FP64 ? TK_2x2 : TK_1x2;
+        own_split = prec == CXA_PREC_FP64 ? 0 : 1;
+      }
+    }
+    v.launch_kind = mix_kind_ok(v.kind) ? v.kind : own;
     v.tile_class = make_tiles(p->blks, p->segs, tiles, &v.per_xcd, v.launch_kind, false);
-    v.splitk = v.split_mode == 1 ? 1 : 0;  // mix plans: four-wave workgroups (two slices each)
+    // mix plans: four-wave workgroups (two slices each)
+    v.splitk = v.split_mode == 1 || (v.split_mode < 0 && own_split) ? 1 : 0;
   } else {
     int kind = v.kind, auto_split = -1;
     if (kind < 0 && v.split_mode < 0 && prec != CXA_PREC_FP32X3 && !(p->chain && real)) {
