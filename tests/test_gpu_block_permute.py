@@ -48,3 +48,14 @@ def test_blocks(rank, ident):
         for shp, n, a, b in zip(BLOCKS[rank], sizes, so, do):
             want[b:b + n] = src[a:a + n].view(shp).permute([int(x) for x in order]).reshape(-1)
         assert torch.equal(dst, want)
+
+
+@pytest.mark.parametrize("ident", sorted(DTYPES))
+def test_output_run_cuts(ident):
+    """Output runs around the tile heights they are cut at, alone and inside outer axes."""
+    from cytnx_amd.tensor import Tensor
+    for h in (31, 33, 119, 120, 121, 127, 128, 129, 136, 200, 255, 257, 300):
+        for shape, order in (((h, 40), (1, 0)), ((3, h, 2, 17), (3, 0, 2, 1)), ((h, 5, 9), (2, 1, 0))):
+            x = torch.randn(shape, dtype=DTYPES[ident], device="cuda")
+            got = Tensor.from_storage(x.reshape(-1), shape).permute(*order).contiguous()
+            assert torch.equal(got.storage(), x.permute(order).reshape(-1))
