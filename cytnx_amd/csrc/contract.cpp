@@ -150,7 +150,7 @@ int build_variant(cxa_bc_plan *p, int prec) {
   } else {
     int kind = v.kind, auto_split = -1;
     if (kind < 0 && v.split_mode < 0 && prec != CXA_PREC_FP32X3 && !(p->chain && real)) {
-      const Tiling t = default_tiling(p->blks, p->segs, !real);
+      const Tiling t = default_tiling(p->blks, p->segs, !real, p->dtype == CXA_C64);
       kind = t.kind;
       auto_split = t.kind < 0 ? -1 : t.split;
     }
@@ -516,7 +516,9 @@ int make_block_plan(int dtype, int rankL, int nbL, const uint64_t *itoiL, const 
   // (First contraction of an environment update at chi = 2048, three MPO states taken apart:
   // 103 us with the copies, of which 58 us are 18 permute launches, 39 us in place.  Gradient of
   // a 32-site MPS energy, chi = 512, complex: 11.5 -> 8.8 ms, 286 permutes of adjoints fewer.)
-  // Real steps of chains keep their copies, and with them the order of their K.
+  // Real steps of chains keep their copies, and with them the order of their K; so does complex64
+  // where K would be taken apart (and it keeps the operands' roles and an unsplit K): in a long
+  // chain of contractions, such as an energy gradient, its roundings are what the result is off by.
   auto worth = [&]() {
     auto pad = [](int64_t x) { return (double)((x + 15) / 16 * 16); };
     double cost = 0.0, whole = 0.0;
@@ -528,6 +530,7 @@ int make_block_plan(int dtype, int rankL, int nbL, const uint64_t *itoiL, const 
       for (int pi : by_target[t]) {
         const Pair &pr = pairs[pi];
         const Runs rk = runs_k(pr);
+        if (dtype == CXA_C64 && (rk.split > 1 || rk.n > 1)) return false;
         nseg += mn * rk.split;
         cost += (double)mn * (double)rk.split * pad(rm.r[rm.main].ext) *
                 pad(rn.r[rn.main].ext) * pad(rk.r[rk.main].ext);
@@ -717,7 +720,7 @@ int make_block_plan(int dtype, int rankL, int nbL, const uint64_t *itoiL, const 
       }
     }
   }
-  if (rows_unit > cols_unit) {
+  if (rows_unit > cols_unit && dtype != CXA_C64) {
     p->swapped = true;
     for (GBlk &g : p->blks) {
       std::swap(g.M, g.N);
@@ -1307,7 +1310,7 @@ extern "C" int cxa_gemm_batch(int dtype, const char *transa, const char *transb,
   for (GBlk &b : blks) seal_block(b, segs.data());
   std::vector<GTile> tiles;
   int per_xcd = 0;
-  const Tiling tl = default_tiling(blks, segs, cplx);
+  const Tiling tl = default_tiling(blks, segs, cplx, dtype == CXA_C64);
   const int cls = make_tiles(blks, segs, tiles, &per_xcd, tl.kind, !cplx);
   if (tiles.empty()) return CXA_OK;
   hipStream_t s = (hipStream_t)stream;

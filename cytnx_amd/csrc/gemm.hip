@@ -50,7 +50,8 @@ constexpr int64_t kFewReal = 512, kFewCplx = 1024, kMany64 = 192;
 
 }  // namespace
 
-Tiling default_tiling(const std::vector<GBlk> &blks, const std::vector<GSeg> &segs, bool cplx) {
+Tiling default_tiling(const std::vector<GBlk> &blks, const std::vector<GSeg> &segs, bool cplx,
+                      bool in_order) {
   int64_t n16 = 0, n64 = 0, work = 0, pad64 = 0, pad32 = 0;
   bool narrow = !cplx, lds = true;
   for (const GBlk &b : blks) {
@@ -71,7 +72,7 @@ Tiling default_tiling(const std::vector<GBlk> &blks, const std::vector<GSeg> &se
   // their rows (their default), others take one wave per tile: the smallest tiles while they
   // are few (4.2 us against 4.5 for 128 blocks of 128 x 10, K = 10)
   if (work <= 2 * n16) return {narrow || n16 > 4 * kFewReal ? -1 : (int)TK_1x1, 0};
-  if (n16 <= (cplx ? kFewCplx : kFewReal)) return {TK_1x1, 4};
+  if (n16 <= (cplx ? kFewCplx : kFewReal)) return {TK_1x1, in_order ? 0 : 4};
   if (!lds || narrow) return {-1, 0};
   if (cplx || n64 < kMany64) return {TK_L32, 0};
   // Ragged blocks: 64x64 tiles that cover much more than 32x32 ones lose it again.  Real blocks

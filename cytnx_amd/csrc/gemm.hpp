@@ -152,7 +152,9 @@ int default_kind(int M, int N);
 struct Tiling {
   int kind, split;
 };
-Tiling default_tiling(const std::vector<GBlk> &blks, const std::vector<GSeg> &segs, bool cplx);
+// (in_order: no split, every element's K is summed front to back.)
+Tiling default_tiling(const std::vector<GBlk> &blks, const std::vector<GSeg> &segs, bool cplx,
+                      bool in_order);
 Tiling single_tiling(const GBlk &blk, const GSeg &seg, bool cplx);
 
 // Fill in what the kernels need to know about a block's segments (chunks, wide).

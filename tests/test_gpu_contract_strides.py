@@ -112,7 +112,7 @@ def test_random_axis_orders(seed, name):
         _contract(ba, bb, c1, c2, dt, code, [int(x) for x in rng.permutation(rc)], conj)
 
 
-@pytest.mark.parametrize("name", ["f64", "c64"])
+@pytest.mark.parametrize("name", ["f64", "c128"])
 def test_large_blocks_in_place(name):
     """A middle index contracted, and results in the operands' own axis order: no workspace."""
     dt, code = _DT[name]
