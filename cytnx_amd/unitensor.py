@@ -107,8 +107,19 @@ def enumerate_blocks(bonds: Sequence[Bond]) -> np.ndarray:
         cap = n.value
 
 
+class _Workspace:
+    """Device scratch of one execution of a plan (passed to the library as its address): from the
+    current stream's pool, so that executions on other streams have their own, and given back to
+    that pool once the call has been enqueued and this object is dropped."""
+    __slots__ = ("_buf", "_as_parameter_")
+
+    def __init__(self, nbytes: int, device: int):
+        self._buf = torch.empty(nbytes, dtype=torch.uint8, device=torch_device(device))
+        self._as_parameter_ = ctypes.c_void_p(self._buf.data_ptr())
+
+
 class _Plan:
-    """Owns a cxa_bc_plan handle and its workspace."""
+    """Owns a cxa_bc_plan handle."""
 
     def __init__(self, handle: int, device: int):
         self.handle = handle
@@ -121,15 +132,12 @@ class _Plan:
         self.flops = f.value
         self.ws_bytes = ws.value
         self.npairs = npairs.value
-        self._ws = None
 
-    def workspace(self) -> int:
-        if self.ws_bytes == 0:
-            return 0
-        if self._ws is None:
-            self._ws = torch.empty(self.ws_bytes, dtype=torch.uint8,
-                                   device=torch_device(self.device))
-        return self._ws.data_ptr()
+    def workspace(self) -> Optional[_Workspace]:
+        """Scratch for one execution on the device's current stream (None: it needs none).  Plans
+        are shared by every thread and stream that contracts the same structure, so the scratch
+        is not the plan's."""
+        return _Workspace(self.ws_bytes, self.device) if self.ws_bytes else None
 
     def __del__(self):
         try:
