@@ -150,7 +150,7 @@ int build_variant(cxa_bc_plan *p, int prec) {
   } else {
     int kind = v.kind, auto_split = -1;
     if (kind < 0 && v.split_mode < 0 && prec != CXA_PREC_FP32X3 && !(p->chain && real)) {
-      const Tiling t = default_tiling(p->blks, p->segs, !real, p->dtype == CXA_C64);
+      const Tiling t = plan_tiling(p->blks, p->segs, prec, !real, p->dtype == CXA_C64);
       kind = t.kind;
       auto_split = t.kind < 0 ? -1 : t.split;
     }
@@ -1310,7 +1310,8 @@ extern "C" int cxa_gemm_batch(int dtype, const char *transa, const char *transb,
   for (GBlk &b : blks) seal_block(b, segs.data());
   std::vector<GTile> tiles;
   int per_xcd = 0;
-  const Tiling tl = default_tiling(blks, segs, cplx, dtype == CXA_C64);
+  const Tiling tl = default_tiling(
+      blks, segs, dtype == CXA_F32 ? CXA_PREC_FP32 : CXA_PREC_FP64, cplx, dtype == CXA_C64);
   const int cls = make_tiles(blks, segs, tiles, &per_xcd, tl.kind, !cplx);
   if (tiles.empty()) return CXA_OK;
   hipStream_t s = (hipStream_t)stream;

@@ -48,10 +48,27 @@ int64_t tiles_of(const GBlk &b, int t) {
 // per SIMD (n = 1600, complex128: 578 us against 525).
 constexpr int64_t kFewReal = 512, kFewCplx = 1024, kMany64 = 192;
 
+// Few tiles (under two per SIMD of a 256-CU device), each with a long K (in chunks of 16).
+constexpr int64_t kSplitTiles = 2048, kSplitChunks = 8;
+
+// Whether the default tiles of these (real) blocks have their K split over four waves.
+bool splits_by_default(const std::vector<GBlk> &blks, const std::vector<GSeg> &segs) {
+  int64_t n = 0, work = 0;
+  for (const GBlk &b : blks) {
+    if (b.M <= 0 || b.N <= 0) continue;
+    const int kind = default_kind(b.M, b.N);
+    const int64_t t = (int64_t)((b.M + tile_rows(kind) - 1) / tile_rows(kind)) *
+                      ((b.N + tile_cols(kind) - 1) / tile_cols(kind));
+    n += t;
+    for (int s = b.seg0; s < b.seg0 + b.nseg; ++s) work += t * ((segs[s].K + 15) / 16);
+  }
+  return n < kSplitTiles && work >= kSplitChunks * n;
+}
+
 }  // namespace
 
-Tiling default_tiling(const std::vector<GBlk> &blks, const std::vector<GSeg> &segs, bool cplx,
-                      bool in_order) {
+Tiling default_tiling(const std::vector<GBlk> &blks, const std::vector<GSeg> &segs, int prec,
+                      bool cplx, bool in_order) {
   int64_t n16 = 0, n64 = 0, work = 0, pad64 = 0, pad32 = 0;
   bool narrow = !cplx, lds = true;
   for (const GBlk &b : blks) {
@@ -71,6 +88,7 @@ Tiling default_tiling(const std::vector<GBlk> &blks, const std::vector<GSeg> &se
   // K of up to two chunks: an output-bound launch (the MPO steps).  Narrow real blocks stream
   // their rows (their default), others take one wave per tile: the smallest tiles while they
   // are few (4.2 us against 4.5 for 128 blocks of 128 x 10, K = 10)
+  if (narrow && prec == CXA_PREC_FP32) return {-1, 0};
   if (work <= 2 * n16) return {narrow || n16 > 4 * kFewReal ? -1 : (int)TK_1x1, 0};
   if (n16 <= (cplx ? kFewCplx : kFewReal)) return {TK_1x1, in_order ? 0 : 4};
   if (!lds || narrow) return {-1, 0};
@@ -80,6 +98,14 @@ Tiling default_tiling(const std::vector<GBlk> &blks, const std::vector<GSeg> &se
   // 34 in FP32, 64x64 79 and 54; of 300 x 300 (the same area), 60 of them: 111 and 60 against 90
   // and 61.
   return {20 * pad64 > 23 * pad32 ? TK_2x2 : TK_L64, 0};
+}
+
+Tiling plan_tiling(const std::vector<GBlk> &blks, const std::vector<GSeg> &segs, int prec,
+                   bool cplx, bool in_order) {
+  const Tiling t = default_tiling(blks, segs, prec, cplx, in_order);
+  const bool four_sums = t.split > 0 || (prec == CXA_PREC_FP32 && is_lds(t.kind));
+  if (!cplx && t.kind >= 0 && !four_sums && splits_by_default(blks, segs)) return {-1, 0};
+  return t;
 }
 
 // One block of one segment (a dense product): the same rule with the whole K in one segment.  A
@@ -211,9 +237,8 @@ bool prefer_splitk(const std::vector<GBlk> &blks, const std::vector<GSeg> &segs,
     work += w;
   }
   if (n == 0) return false;
-  // few tiles (under two per SIMD of a 256-CU device) that each walk a long K range
   const double avg = (double)work / (double)n;
-  return n < 2048 && avg >= (tile_class == TC_ROWS ? 64.0 : 8.0);
+  return n < kSplitTiles && avg >= (tile_class == TC_ROWS ? 64.0 : (double)kSplitChunks);
 }
 
 }  // namespace cxa
