@@ -59,3 +59,18 @@ def test_narrow_blocks_sum_in_fp64(nb, M, N, K):
     linalg.Gemm_Batch([1.0], A, B, [0.0], C, [nb])
     got = torch.stack([x.storage().view(M, N) for x in C]).double()
     assert bool(((got - want).abs() <= bound).all())
+
+
+@pytest.mark.parametrize("nb,M,N,K", [(1, 100, 75, 133), (3, 64, 64, 1000), (2, 33, 17, 16), (1, 40, 70, 65)])
+def test_fp32_lds_tiles_sum_as_the_split_does(nb, M, N, K):
+    """LDS tiles of both sizes: the bits of 16 x 16 tiles whose K is split over four waves."""
+    print("lds and split", nb, M, N, K, flush=True)
+    a, b = _rand(nb * M * K, 3), _rand(nb * K * N, 4)
+    plan = strided_batch_plan(nb, M, N, K, (M * K, K, 1), (K * N, N, 1), (M * N, N), 4)
+    got = []
+    for kind, split in ((0, 1), (6, 0), (7, 0)):
+        c = torch.zeros(nb * M * N, dtype=torch.float32, device="cuda")
+        _lib.check(_lib.lib().cxa_block_contract_set_config(plan.handle, -1, kind, split))
+        _exec(plan, a, b, c)
+        got.append(c)
+    assert torch.equal(got[0], got[1]) and torch.equal(got[0], got[2])
