@@ -89,8 +89,10 @@ struct cxa_bc_plan {
   const cxa::GBlk *dev_blks = nullptr;
   const cxa::GSeg *dev_segs = nullptr;
   const cxa::MixOut *dev_outs = nullptr;
-  PlanVariant var[3];  // indexed by CXA_PREC_*
-  std::mutex mu;       // guards building a variant on first use
+  // Indexed by CXA_PREC_*; the second three are those of executions as a step of a matvec chain
+  // where they differ from the plan's own (variant_index).
+  PlanVariant var[6];
+  std::mutex mu;  // guards building a variant on first use
   bool copyA = false, copyB = false;
   std::vector<cxa::CopyJob> jobsA, jobsB, jobsC;  // blocks too large for the batched copy
   // the other operand (output) blocks, permuted into (out of) the workspace by one batched
@@ -106,8 +108,7 @@ struct cxa_bc_plan {
   // mix plans (cxa_mix_contract_plan): blks are items, segs their slices, outs the outputs
   bool mix = false;
   std::vector<cxa::MixOut> outs;
-  // a step of a matvec chain (bc_join_chain)
-  bool chain = false;
+  bool chain = false;  // made as a step of a matvec chain (CXA_PLAN_CHAIN)
   // blks / segs describe the transposed products: their A operand is R's buffer, B is L's
   bool swapped = false;
 };
@@ -123,9 +124,21 @@ bool mix_kind_ok(int kind) {
   return kind == TK_1x1 || kind == TK_2x1 || kind == TK_1x2 || kind == TK_2x2;
 }
 
-int build_variant(cxa_bc_plan *p, int prec) {
+// The variant that an execution runs.  Real steps of a chain keep the direct tiles: their tile list
+// fixes the order in which a fused Lanczos iteration sums its dot products, and with it the last
+// bits of alpha and beta, from which the sign of an unconverged Ritz vector follows.  (The LDS
+// tiles would take the FP64 .R launch at chi = 2048 from 37 to 35 us and change nothing at 1024.)
+// A plan that was not made for a chain keeps its own tile lists beside those of its chains, so that
+// putting it into one changes nothing for executions by themselves, in flight or captured.
+int variant_index(const cxa_bc_plan *p, int prec, bool step) {
+  return step && !p->chain && !p->mix && !is_complex(p->dtype) ? 3 + prec : prec;
+}
+
+int build_variant(cxa_bc_plan *p, int index) {
   const bool real = p->dtype == CXA_F64 || p->dtype == CXA_F32;
-  PlanVariant &v = p->var[prec];
+  const int prec = index % 3;
+  const bool chain = p->chain || index >= 3;
+  PlanVariant &v = p->var[index];
   v.built = false;
   // the host tile list lives only until it is uploaded: one buffer per thread keeps its pages
   thread_local std::vector<GTile> tiles;
@@ -149,7 +162,7 @@ int build_variant(cxa_bc_plan *p, int prec) {
     v.splitk = v.split_mode == 1 || (v.split_mode < 0 && own_split) ? 1 : 0;
   } else {
     int kind = v.kind, auto_split = -1;
-    if (kind < 0 && v.split_mode < 0 && prec != CXA_PREC_FP32X3 && !(p->chain && real)) {
+    if (kind < 0 && v.split_mode < 0 && prec != CXA_PREC_FP32X3 && !(chain && real)) {
       const Tiling t = plan_tiling(p->blks, p->segs, prec, !real, p->dtype == CXA_C64);
       kind = t.kind;
       auto_split = t.kind < 0 ? -1 : t.split;
@@ -235,7 +248,7 @@ int upload_plan(cxa_bc_plan *p) {
     p->dev_bjobsC = at(7);
     p->dev_btasksC = (const BatchCopyTask *)at(8);
   }
-  if (p->chain) return CXA_OK;  // cxa_chain_create makes the tile list (bc_join_chain)
+  if (p->chain) return CXA_OK;  // cxa_chain_create makes the tile list
   return build_variant(p, native_prec(p->dtype));
 }
 
@@ -261,10 +274,11 @@ void split_copies(int es, const std::vector<CopyJob> &all, std::vector<CopyJob> 
 
 // Make (once) the tile list of one precision.  A host-side copy runs, so an exec inside a graph
 // capture refuses a precision that was never prepared.
-int bc_ensure(const cxa_bc_plan *cp, int prec, hipStream_t s) {
+int bc_ensure(const cxa_bc_plan *cp, int prec, hipStream_t s, bool step) {
   cxa_bc_plan *p = const_cast<cxa_bc_plan *>(cp);
+  const int index = variant_index(p, prec, step);
   std::lock_guard<std::mutex> lk(p->mu);
-  if (p->var[prec].built) return CXA_OK;
+  if (p->var[index].built) return CXA_OK;
   if (s) {
     hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
     CXA_HIP(hipStreamIsCapturing(s, &st));
@@ -273,23 +287,7 @@ int bc_ensure(const cxa_bc_plan *cp, int prec, hipStream_t s) {
               "which cannot happen during a graph capture (run or configure it once first)",
               prec);
   }
-  return build_variant(p, prec);
-}
-
-// Real steps of a chain keep the direct tiles: their tile list fixes the order in which a fused
-// Lanczos iteration sums its dot products, and with it the last bits of alpha and beta, from
-// which the sign of an unconverged Ritz vector follows.  (The LDS tiles would take the FP64 .R
-// launch at chi = 2048 from 37 to 35 us and change nothing at 1024.)
-int bc_join_chain(const cxa_bc_plan *cp) {
-  cxa_bc_plan *p = const_cast<cxa_bc_plan *>(cp);
-  std::lock_guard<std::mutex> lk(p->mu);
-  const int prec = native_prec(p->dtype);
-  PlanVariant &v = p->var[prec];
-  const bool was = p->chain;
-  p->chain = true;
-  const bool same = was || p->mix || is_complex(p->dtype) || v.kind >= 0 || v.split_mode >= 0;
-  if (v.built && same) return CXA_OK;
-  return build_variant(p, prec);
+  return build_variant(p, index);
 }
 
 int bc_prepare(const cxa_bc_plan *p) {
@@ -516,9 +514,10 @@ int make_block_plan(int dtype, int rankL, int nbL, const uint64_t *itoiL, const 
   // (First contraction of an environment update at chi = 2048, three MPO states taken apart:
   // 103 us with the copies, of which 58 us are 18 permute launches, 39 us in place.  Gradient of
   // a 32-site MPS energy, chi = 512, complex: 11.5 -> 8.8 ms, 286 permutes of adjoints fewer.)
-  // Real steps of chains keep their copies, and with them the order of their K; so does complex64
-  // where K would be taken apart (and it keeps the operands' roles and an unsplit K): in a long
-  // chain of contractions, such as an energy gradient, its roundings are what the result is off by.
+  // Real plans made for a chain keep their copies, and with them the order of their K.  So does
+  // complex64 where K would be taken apart, and it keeps the operands' roles and an unsplit K: its
+  // results are then the same bits either way, where the error of an energy gradient is no smaller
+  // with K taken apart (means over 8 seeds: 1.8e-6 and 1.3e-6 as it is, 1.9e-6 and 1.5e-6 so).
   auto worth = [&]() {
     auto pad = [](int64_t x) { return (double)((x + 15) / 16 * 16); };
     double cost = 0.0, whole = 0.0;
@@ -923,8 +922,8 @@ extern "C" int cxa_block_contract_set_config(cxa_bc_plan *p, int prec, int kind,
   CXA_CHECK(!p->mix || split <= 1, CXA_ERR_UNSUPPORTED,
             "mix plans run eight- or four-wave workgroups (split 0 or 1)");
   std::lock_guard<std::mutex> lk(p->mu);
-  for (int q = 0; q < 3; ++q) {
-    if (prec >= 0 && q != prec) continue;
+  for (int q = 0; q < 6; ++q) {
+    if (prec >= 0 && q % 3 != prec) continue;
     PlanVariant &v = p->var[q];
     if (v.kind == kind && v.split_mode == split && v.built) continue;
     v.kind = kind;
@@ -953,7 +952,7 @@ extern "C" int cxa_block_contract_set_tile(cxa_bc_plan *p, int kind) {
   CXA_CHECK(p, CXA_ERR_INVALID, "cxa_block_contract_set_tile: null plan");
   CXA_CHECK(kind >= -1 && kind < TK_COUNT, CXA_ERR_INVALID, "unknown tile kind %d", kind);
   std::lock_guard<std::mutex> lk(p->mu);
-  for (int q = 0; q < 3; ++q) {
+  for (int q = 0; q < 6; ++q) {
     p->var[q].kind = kind;
     if (!p->var[q].built) continue;  // made with this kind on first use
     int rc = build_variant(p, q);
@@ -1023,9 +1022,9 @@ int bc_exec_typed(const cxa_bc_plan *p, const void *L, const void *R, void *C, i
     std::swap(g.a_dt, g.b_dt);
     conj = (conj & 1) << 1 | (conj & 2) >> 1;
   }
-  int rc = bc_ensure(p, prec_eff, s);
+  int rc = bc_ensure(p, prec_eff, s, lay->step);
   if (rc) return rc;
-  const PlanVariant &v = p->var[prec_eff];
+  const PlanVariant &v = p->var[variant_index(p, prec_eff, lay->step)];
   g.tiles = (const GTile *)v.d_tiles.p;
   g.blks = p->dev_blks;
   g.segs = lay->segs ? lay->segs : p->dev_segs;
@@ -1163,8 +1162,8 @@ int bc_dot_slots(const cxa_bc_plan *p, int prec) {
   if (p->wsC) return 0;  // the epilogue takes the output in place, unit-stride along n
   for (const GBlk &b : p->blks)
     if (b.csn != 1) return 0;
-  if (bc_ensure(p, prec, nullptr)) return 0;
-  const PlanVariant &v = p->var[prec];
+  if (bc_ensure(p, prec, nullptr, true)) return 0;
+  const PlanVariant &v = p->var[variant_index(p, prec, true)];
   if (v.tile_class == 1 || v.ntiles == 0) return 0;  // make_tiles' row-streaming class
   return v.ntiles;
 }
@@ -1177,7 +1176,7 @@ extern "C" int cxa_block_contract_set_split(cxa_bc_plan *p, int mode) {
   CXA_CHECK(p, CXA_ERR_INVALID, "cxa_block_contract_set_split: null plan");
   CXA_CHECK(mode >= -1 && mode <= 2, CXA_ERR_INVALID, "split mode must be -1, 0, 1 or 2");
   std::lock_guard<std::mutex> lk(p->mu);
-  for (int q = 0; q < 3; ++q) {
+  for (int q = 0; q < 6; ++q) {
     p->var[q].split_mode = mode;
     if (!p->var[q].built) continue;  // made with this mode on first use
     int rc = build_variant(p, q);

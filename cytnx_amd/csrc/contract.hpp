@@ -17,6 +17,7 @@ struct ExecLayout {
   const GSeg *segs = nullptr;
   const MixOut *outs = nullptr;
   bool a_k4 = false, b_k4 = false, c_k4 = false;
+  bool step = false;  // as a step of a matvec chain, with the tile lists of one
   // dot-product epilogue (GemmLaunch::dot_x / dot_part): dot_part gets bc_dot_slots entries
   const double *dot_x = nullptr;
   double *dot_part = nullptr;
@@ -78,12 +79,11 @@ int bc_mix_pack_outs(const cxa_bc_plan *mix, const std::vector<PackRegion> &regi
 bool bc_is_mix(const cxa_bc_plan *p);
 // Make a plan's tile list for one precision if it is not made yet (the plan makes only its own
 // precision at creation); refused while `s` is capturing a graph.  bc_prepare makes all three.
-int bc_ensure(const cxa_bc_plan *p, int prec, hipStream_t s);
+// step: the list that executions as a step of a matvec chain run.
+int bc_ensure(const cxa_bc_plan *p, int prec, hipStream_t s, bool step = false);
 int bc_prepare(const cxa_bc_plan *p);
-// The plan becomes a step of a matvec chain (its FP64 default tiling is then the direct one).
-int bc_join_chain(const cxa_bc_plan *p);
-// Tile slots a dot-product epilogue of an execution at precision prec writes (the launch's tile
-// list length), or 0 when that launch cannot carry one (mix, complex, row-streaming tiles).
+// Tile slots a dot-product epilogue of an execution as a chain's step at precision prec writes
+// (the launch's tile list length), or 0 when that launch cannot carry one (mix, complex, row-streaming tiles).
 int bc_dot_slots(const cxa_bc_plan *p, int prec);
 int64_t bc_workspace_elems(const cxa_bc_plan *p);
 double bc_flops(const cxa_bc_plan *p);

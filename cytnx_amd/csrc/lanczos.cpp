@@ -308,7 +308,7 @@ extern "C" int cxa_chain_create(int nsteps, cxa_bc_plan *const *plans, const voi
               k);
     CXA_CHECK(!cplx || !bc_is_mix(plans[k]), CXA_ERR_UNSUPPORTED,
               "cxa_chain_create: mix plans are real (step %d)", k);
-    CXA_RC(bc_join_chain(plans[k]));
+    CXA_RC(bc_ensure(plans[k], CXA_PREC_FP64, nullptr, true));
     c->plans.push_back(plans[k]);
     c->fixed.push_back(fixed[k]);
     c->fixed_left.push_back(fixed_is_left[k] ? 1 : 0);
@@ -460,7 +460,7 @@ extern "C" int cxa_chain_prepare(cxa_chain *c, int prec, cxa_stream_t stream) {
             "cxa_chain_prepare: complex chains run in FP64 only");
   c->prec = prec;
   for (int k = 0; k < c->nsteps; ++k) {  // tile lists of this precision, before any capture
-    const int rc = bc_ensure(c->plans[k], prec, nullptr);
+    const int rc = bc_ensure(c->plans[k], prec, nullptr, true);
     if (rc) return rc;
   }
   if (prec != CXA_PREC_FP32 || !c->fixed32.empty()) return CXA_OK;
@@ -499,13 +499,17 @@ namespace {
 // instead of x.
 int chain_step(cxa_chain *c, int k, const void *x, void *y, hipStream_t s,
                const double *dotx = nullptr, double *dotp = nullptr, bool pk = false) {
+  cxa::ExecLayout lay;
+  lay.step = true;
   if (c->dtype != CXA_F64) {  // complex chain: FP64, every operand as the plan lays it out
     const void *in = k == 0 ? x : c->mid64[k - 1];
     void *outp = k == c->nsteps - 1 ? y : c->mid64[k];
     const int dt = c->dtype;
     return c->fixed_left[k]
-               ? bc_exec_typed(c->plans[k], c->fixed[k], in, outp, dt, dt, dt, c->prec, c->ws, s)
-               : bc_exec_typed(c->plans[k], in, c->fixed[k], outp, dt, dt, dt, c->prec, c->ws, s);
+               ? bc_exec_typed(c->plans[k], c->fixed[k], in, outp, dt, dt, dt, c->prec, c->ws, s, 0,
+                               &lay)
+               : bc_exec_typed(c->plans[k], in, c->fixed[k], outp, dt, dt, dt, c->prec, c->ws, s, 0,
+                               &lay);
   }
   const bool f32 = c->prec == CXA_PREC_FP32;
   const bool last = k == c->nsteps - 1;
@@ -514,7 +518,6 @@ int chain_step(cxa_chain *c, int k, const void *x, void *y, hipStream_t s,
   void *outp = last ? y : (f32 ? c->mid32[k] : c->mid64[k]);
   const int out_dt = (last || !f32) ? CXA_F64 : CXA_F32;
   const int fx_dt = f32 ? CXA_F32 : CXA_F64;
-  cxa::ExecLayout lay;
   lay.dot_x = dotx;
   lay.dot_part = dotp;
   if (c->fixed_left[k])
@@ -670,7 +673,7 @@ extern "C" int cxa_chain_tune(cxa_chain *c, const void *x, void *y, int reps, in
       if (c->dtype != CXA_F64 &&
           (cand[ci][0] == TK_4x2 || cand[ci][0] == TK_ROWS || cand[ci][0] == TK_L64))
         continue;
-      // real FP64 steps keep the direct tiles (bc_join_chain); FP32X3 has no LDS tiles
+      // real FP64 steps keep the direct tiles (variant_index); FP32X3 has no LDS tiles
       if (c->dtype == CXA_F64 && c->prec != CXA_PREC_FP32 && is_lds(cand[ci][0])) continue;
       if ((rc = cxa_block_contract_set_config(plan, c->prec, cand[ci][0], cand[ci][1]))) break;
       double per = 0.0, per_plain = 0.0;

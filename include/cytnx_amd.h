@@ -187,7 +187,9 @@ int cxa_u1_enumerate_blocks(int rank, const int *btype, const int64_t *nq, const
  */
 typedef struct cxa_bc_plan cxa_bc_plan;
 /* or'ed into the dtype of a plan that will be a step of a matvec chain: its tile list is made by
- * cxa_chain_create (or its first exec) instead of at creation, with the tilings of chain steps. */
+ * cxa_chain_create (or its first exec) instead of at creation, with the tilings of chain steps.
+ * A plan made without it can be a chain's step as well: the chain then runs tile lists of its own,
+ * and the plan's (get_config) stay as they are for executions by themselves. */
 #define CXA_PLAN_CHAIN 256
 int cxa_block_contract_plan(int dtype, int rankL, int nbL, const uint64_t *itoiL,
                             const uint64_t *shapeL, const int64_t *offL, int rankR, int nbR,
