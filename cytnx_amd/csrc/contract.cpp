@@ -77,6 +77,7 @@ struct PlanVariant {
   int splitk = 0;  // waves per tile of the split-K launch, 0 = none (mix plans: 1 = four-wave)
   int tile_class = 0;
   int launch_kind = -1;  // mix plans and LDS tiles: the one tile kind of the launch
+  bool lean = false;     // GemmLaunch::lean
 };
 
 struct cxa_bc_plan {
@@ -186,6 +187,7 @@ int build_variant(cxa_bc_plan *p, int index) {
                        prefer_splitk(p->blks, p->segs, tiles, v.tile_class)));
     // eight-wave split-K only for MFMA tiles (row tiles always split over four waves)
     v.splitk = !split ? 0 : (v.split_mode == 2 && v.tile_class == 0 ? 8 : 4);
+    v.lean = v.tile_class == 0 && !split && lean_tiles(p->blks, p->segs, prec, !real);
   }
   v.ntiles = (int)tiles.size();
   v.nlive = 0;
@@ -1035,6 +1037,7 @@ int bc_exec_typed(const cxa_bc_plan *p, const void *L, const void *R, void *C, i
   g.per_xcd = v.per_xcd;
   g.splitk = v.splitk;
   g.tile_class = v.tile_class;
+  g.lean = v.lean;
   g.conj = is_complex(p->dtype) ? conj : 0;
   g.dot_x = lay->dot_x;
   g.dot_part = lay->dot_part;
@@ -1309,8 +1312,7 @@ extern "C" int cxa_gemm_batch(int dtype, const char *transa, const char *transb,
   for (GBlk &b : blks) seal_block(b, segs.data());
   std::vector<GTile> tiles;
   int per_xcd = 0;
-  const Tiling tl = default_tiling(
-      blks, segs, dtype == CXA_F32 ? CXA_PREC_FP32 : CXA_PREC_FP64, cplx, dtype == CXA_C64);
+  const Tiling tl = default_tiling(blks, segs, native_prec(dtype), cplx, dtype == CXA_C64);
   const int cls = make_tiles(blks, segs, tiles, &per_xcd, tl.kind, !cplx);
   if (tiles.empty()) return CXA_OK;
   hipStream_t s = (hipStream_t)stream;
@@ -1345,6 +1347,7 @@ extern "C" int cxa_gemm_batch(int dtype, const char *transa, const char *transb,
   g.tile_class = cls;
   g.kind0 = tl.kind;
   g.splitk = tl.split;
+  g.lean = cls == 0 && !tl.split && lean_tiles(blks, segs, native_prec(dtype), cplx);
   rc = launch_grouped_gemm(g, s);
   if (rc) return rc;
   // the task arrays go back to the pool on return: wait for the launch that reads them

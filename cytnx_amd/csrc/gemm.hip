@@ -32,89 +32,127 @@ int64_t tiles_of(const GBlk &b, int t) {
   return (int64_t)((b.M + t - 1) / t) * ((b.N + t - 1) / t);
 }
 
-// The choice from the number of 16 x 16 tiles, their mean K in 16-deep chunks and the number of
-// 64 x 64 tiles.  A 16 x 16 tile is the finest split of the output, and a wave works through its
-// K one MFMA after another, so few tiles leave SIMDs idle: up to kFew of them (two, complex four,
-// times the CUs) the four waves of a workgroup share a tile's K, which then also hides their load
-// latency.  Above that the LDS tiles read every operand element once per 32 or 64 rows instead
-// of once per 16, in contiguous runs.  Measured (us, split 16 x 16 / 32 x 32 LDS):
-//   real, product of n = 128: 3.9 / 5.2, 256: 4.9 / 7.3, 512 (1024 tiles): 21.2 / 11.5;
-//   complex128, n = 256: 6.4 / 13.9, 384 x 960 x 192 (288 tiles): 27 / 43, 512: 30 / 26;
-//   block contractions of a chi = 512 complex128 MPS (about 830 tiles): 12-20 / 31 (the direct
-//   32 x 32 tiles 100); two-site .R launch in FP64, chi = 512: 4.8 / 5.8, 2048: 43 / 35.
-// 64 x 64 tiles (a quarter of the chunk loads and barriers per flop) pay once they give most CUs
-// a tile: n = 700 (121 tiles) 36 us against 23 in FP64, 900 (225 tiles) 44 against 46, 1600 165
-// against 177.  They are real-only: a complex 64 x 64 tile's registers leave one or two waves
-// per SIMD (n = 1600, complex128: 578 us against 525).
-constexpr int64_t kFewReal = 512, kFewCplx = 1024, kMany64 = 192;
+// The choice, from counts of tiles and the mean K in chunks of 16.  A 16 x 16 tile is the finest split
+// of the output, and a wave works through its K one MFMA after another, so few tiles leave SIMDs
+// idle: up to kFew of them (two, complex four, times the CUs; single products half) the four waves
+// of a workgroup share a tile's K, which then also hides their load latency.  Beyond, tiles of one
+// wave: the default ones from kManyDirect of them (three per CU), else 16 x 16.  With more than
+// kShortChunks of K (lists of complex128 blocks kShortC128) the LDS tiles, which read every operand
+// element once per 32 or 64 rows instead of once per 16 or 32, unless they cover more than 1.15
+// times the area of the default tiles.  64 x 64 tiles (a quarter of the chunk loads and barriers
+// per flop) from kMany64 of them, real types only: a complex one's registers leave one or two
+// waves per SIMD.
+// Measured, us:
+//   split 16x16 / LDS 32x32: real products of n = 128 3.9 / 5.2, 256 4.9 / 7.3, 512 (1024 tiles)
+//   21.2 / 11.5; complex128 n = 256 6.4 / 13.9, 384 x 960 x 192 (288 tiles) 27 / 43, 512 30 / 26;
+//   default / 16x16: FP32 20000 x 33 x 20 (625 of them) 5.0 / 4.8, 600 x 600, K = 100 7.0 / 5.7, 1000 x
+//   1000 (1024) 7.3 / 9.5, 200 blocks of 60 x 60 (800), K = 50 5.7 / 7.4;
+//   direct / LDS (64x64 of real types): 3000 x 3000, K = 33 FP32 19.0 / 30.7, complex64 41.7 / 67.6; K =
+//   100 FP32 31 / 41, FP64 47.7 / 45.1, complex128 137 / 147; 1600 x 1600 complex128, K = 200 87 / 77,
+//   1000 x 1000 (1024 LDS tiles) 37 / 43; 60 blocks of 160 x 160, K = 400 complex128 107 / 86;
+//   covering twice the area: 100000 x 10 x 100 FP64 19.6 / 30.7, 10 x 400 x 20000 FP64 13 / 31; 200
+//   blocks of 300 x 8, K = 100 complex64 15.6 / 24.5.
+constexpr int64_t kFewReal = 512, kFewCplx = 1024, kMany64 = 192, kManyDirect = 768;
+constexpr int64_t kShortChunks = 7, kShortC128 = 13, kRoundLow = 768, kRoundHigh = 1400;
+
+// Blocks counted in tiles and in their work, the chunks of K times the area that the tiles cover.
+struct Cover {
+  int64_t n16 = 0, n32 = 0, n64 = 0, def = 0;     // tiles: by size, and of the default kinds
+  int64_t work = 0;                               // chunks of K over all 16 x 16 tiles
+  int64_t area32 = 0, area64 = 0, area_def = 0;   // times the area covered, in 16 x 16
+  bool lds = true, wide = false;  // LDS tiles can, direct tiles need 64-bit offsets
+  void add(const GBlk &b, const GSeg *segs) {
+    if (b.M <= 0 || b.N <= 0) return;
+    const int kind = default_kind(b.M, b.N);
+    const int64_t t16 = tiles_of(b, 16), t32 = tiles_of(b, 32), t64 = tiles_of(b, 64);
+    const int64_t td = (int64_t)((b.M + tile_rows(kind) - 1) / tile_rows(kind)) *
+                       ((b.N + tile_cols(kind) - 1) / tile_cols(kind));
+    if (b.wide & kWideStrides) wide = true;
+    int64_t chunks = 0;
+    for (int s = 0; s < b.nseg; ++s) {
+      chunks += (segs[s].K + 15) / 16;
+      lds = lds && lds_ok(b, segs[s]);
+    }
+    n16 += t16;
+    n32 += t32;
+    n64 += t64;
+    def += td;
+    work += t16 * chunks;
+    area32 += 4 * t32 * chunks;
+    area64 += 16 * t64 * chunks;
+    area_def += tile_rows(kind) * tile_cols(kind) / 256 * td * chunks;
+  }
+  // lean tiles (TC_LEAN): of complex128 always
+  bool lean(int prec, bool cplx) const {
+    return !wide && ((cplx && prec == CXA_PREC_FP64) || work <= kShortChunks * n16);
+  }
+  // direct tiles rather than LDS ones (c128: a list of complex128 blocks)
+  bool stay_direct(bool c128) const { return work <= (c128 ? kShortC128 : kShortChunks) * n16; }
+  // direct tiles: the default ones where they are many, 16 x 16 otherwise
+  int direct(int kind) const { return def >= kManyDirect ? kind : (int)TK_1x1; }
+  // beyond the few tiles and the short K: LDS tiles unless they cover much more than direct ones or
+  // (c128) are about the four that a CU holds at a time, in a single round
+  int large(int kind, bool cplx, bool c128) const {
+    if (!lds) return kind;
+    const bool l64 = !cplx && n64 >= kMany64;
+    const bool round = c128 && n32 >= kRoundLow && n32 < kRoundHigh;
+    if (!round && 20 * (l64 ? area64 : area32) <= 23 * area_def) return l64 ? TK_L64 : TK_L32;
+    return direct(kind);
+  }
+};
 
 // Few tiles (under two per SIMD of a 256-CU device), each with a long K (in chunks of 16).
 constexpr int64_t kSplitTiles = 2048, kSplitChunks = 8;
 
-// Whether the default tiles of these (real) blocks have their K split over four waves.
-bool splits_by_default(const std::vector<GBlk> &blks, const std::vector<GSeg> &segs) {
-  int64_t n = 0, work = 0;
-  for (const GBlk &b : blks) {
-    if (b.M <= 0 || b.N <= 0) continue;
-    const int kind = default_kind(b.M, b.N);
-    const int64_t t = (int64_t)((b.M + tile_rows(kind) - 1) / tile_rows(kind)) *
-                      ((b.N + tile_cols(kind) - 1) / tile_cols(kind));
-    n += t;
-    for (int s = b.seg0; s < b.seg0 + b.nseg; ++s) work += t * ((segs[s].K + 15) / 16);
-  }
-  return n < kSplitTiles && work >= kSplitChunks * n;
-}
-
 }  // namespace
+
+bool lean_tiles(const std::vector<GBlk> &blks, const std::vector<GSeg> &segs, int prec,
+                bool cplx) {
+  Cover c;
+  for (const GBlk &b : blks) c.add(b, segs.data() + b.seg0);
+  return c.lean(prec, cplx);
+}
 
 Tiling default_tiling(const std::vector<GBlk> &blks, const std::vector<GSeg> &segs, int prec,
                       bool cplx, bool in_order) {
-  int64_t n16 = 0, n64 = 0, work = 0, pad64 = 0, pad32 = 0;
-  bool narrow = !cplx, lds = true;
+  Cover c;
+  bool narrow = !cplx;
   for (const GBlk &b : blks) {
-    if (b.M <= 0 || b.N <= 0) continue;
-    const int64_t t = tiles_of(b, 16);
-    n16 += t;
-    n64 += tiles_of(b, 64);
-    if (b.N > kRowsN) narrow = false;
-    for (int s = b.seg0; s < b.seg0 + b.nseg; ++s) {
-      const int64_t chunks = (segs[s].K + 15) / 16;
-      work += t * chunks;
-      pad64 += 16 * tiles_of(b, 64) * chunks;
-      pad32 += 4 * tiles_of(b, 32) * chunks;
-      lds = lds && lds_ok(b, segs[s]);
-    }
+    c.add(b, segs.data() + b.seg0);
+    if (b.M > 0 && b.N > kRowsN) narrow = false;
   }
-  // K of up to two chunks: an output-bound launch (the MPO steps).  Narrow real blocks stream
-  // their rows (their default), others take one wave per tile: the smallest tiles while they
-  // are few (4.2 us against 4.5 for 128 blocks of 128 x 10, K = 10)
   if (narrow && prec == CXA_PREC_FP32) return {-1, 0};
-  if (work <= 2 * n16) return {narrow || n16 > 4 * kFewReal ? -1 : (int)TK_1x1, 0};
-  if (n16 <= (cplx ? kFewCplx : kFewReal)) return {TK_1x1, in_order ? 0 : 4};
-  if (!lds || narrow) return {-1, 0};
-  if (cplx || n64 < kMany64) return {TK_L32, 0};
-  // Ragged blocks: 64x64 tiles that cover much more than 32x32 ones lose it again.  Real blocks
-  // of 160 x 160, K = 400, 120 of them (1.44 times the area): direct 32x32 tiles 59 us in FP64 and
-  // 34 in FP32, 64x64 79 and 54; of 300 x 300 (the same area), 60 of them: 111 and 60 against 90
-  // and 61.
-  return {20 * pad64 > 23 * pad32 ? TK_2x2 : TK_L64, 0};
+  if (c.work <= 2 * c.n16) return {narrow ? -1 : c.direct(-1), 0};
+  if (c.n16 <= (cplx ? kFewCplx : kFewReal)) return {TK_1x1, in_order ? 0 : 4};
+  if (narrow) return {-1, 0};
+  const bool c128 = cplx && prec == CXA_PREC_FP64;
+  return {c.stay_direct(c128) ? c.direct(-1) : c.large(-1, cplx, c128), 0};
 }
 
 Tiling plan_tiling(const std::vector<GBlk> &blks, const std::vector<GSeg> &segs, int prec,
                    bool cplx, bool in_order) {
   const Tiling t = default_tiling(blks, segs, prec, cplx, in_order);
-  const bool four_sums = t.split > 0 || (prec == CXA_PREC_FP32 && is_lds(t.kind));
-  if (!cplx && t.kind >= 0 && !four_sums && splits_by_default(blks, segs)) return {-1, 0};
-  return t;
+  const bool four_sums = t.split > 0 || (prec == CXA_PREC_FP32 && t.kind == TK_L64);
+  if (cplx || t.kind < 0 || four_sums) return t;
+  Cover c;
+  for (const GBlk &b : blks) c.add(b, segs.data() + b.seg0);
+  // (the default tiles' share of the work: their chunks of K, not those of 16 x 16 tiles)
+  int64_t work = 0;
+  for (const GBlk &b : blks) {
+    Cover one;
+    one.add(b, segs.data() + b.seg0);
+    if (one.n16) work += one.def * (one.work / one.n16);
+  }
+  return c.def < kSplitTiles && work >= kSplitChunks * c.def ? Tiling{-1, 0} : t;
 }
 
-// One block of one segment (a dense product): the same rule with the whole K in one segment.  A
-// tall K = 10 product of 36864 x 10 takes 4.5 us in direct tiles and 7.9 in LDS tiles.
-Tiling single_tiling(const GBlk &b, const GSeg &s, bool cplx) {
-  const int64_t n16 = tiles_of(b, 16);
-  if (n16 <= (cplx ? kFewCplx : kFewReal) / 2) return {TK_1x1, s.K > 32 ? 4 : 0};
-  if (s.K <= 32 || !lds_ok(b, s)) return {default_kind(b.M, b.N), 0};
-  return {!cplx && tiles_of(b, 64) >= kMany64 ? TK_L64 : TK_L32, 0};
+// One block of one segment (a dense product): the same rule with the whole K in one segment.
+Tiling single_tiling(const GBlk &b, const GSeg &s, int prec, bool cplx) {
+  Cover c;
+  c.add(b, &s);
+  const int kind = default_kind(b.M, b.N);
+  if (c.n16 <= (cplx ? kFewCplx : kFewReal) / 2 && s.K > 32) return {TK_1x1, 4};
+  return {c.stay_direct(false) ? c.direct(kind) : c.large(kind, cplx, false), 0, c.lean(prec, cplx)};
 }
 
 void seal_block(GBlk &b, const GSeg *segs) {

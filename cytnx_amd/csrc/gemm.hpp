@@ -91,6 +91,7 @@ struct GemmLaunch {
   // interleaved over its waves (mix launches: nonzero = four-wave workgroups)
   int splitk = 0;
   int tile_class = 0;   // the class make_tiles returned
+  bool lean = false;    // MFMA tiles of short K: kernels of fewer registers (TC_LEAN)
   const MixOut *outs = nullptr;  // non-null: mix launch (blks are items, segs are slices)
   int conj = 0;  // complex dtypes: bit 0 conjugates A, bit 1 conjugates B
   // B is k4-packed (real dtypes, B = FP32 in FP32 mode or FP64 otherwise): element (k, n) of a
@@ -151,6 +152,7 @@ int default_kind(int M, int N);
 // the waves a tile's K range is split over (0 or 4).
 struct Tiling {
   int kind, split;
+  bool lean = false;  // (single launches)
 };
 // (in_order: no split, every element's K is summed front to back.)
 // Narrow FP32 blocks always keep the row tiles, which sum in FP64.  Error against 64 bits, rows /
@@ -160,12 +162,15 @@ Tiling default_tiling(const std::vector<GBlk> &blks, const std::vector<GSeg> &se
                       bool cplx, bool in_order);
 // The same for plans, whose default tiles (kind -1) may split K (prefer_splitk).  Four partial sums
 // of K are not given up for one: real lists whose default tiles split K keep them unless the
-// choice splits K too or, in FP32, is an LDS tile, which sums K in four accumulators.  Error against
+// choice splits K too or, in FP32, is the 64x64 LDS tile, which sums K in four accumulators (so
+// does the 32x32 one, but 600 x 600 x 400 takes 11.0 us in it and 9.5 split).  Error against
 // 100 bits of an environment update at bond dimension 1448, split / one sum: FP64 4.3e-16 /
 // 5.8e-16, FP32 2.3e-7 / 3.1e-7; of 60 blocks of 160 x 160, K = 400, in FP32: 1.8e-7 / 3.6e-7.
 Tiling plan_tiling(const std::vector<GBlk> &blks, const std::vector<GSeg> &segs, int prec,
                    bool cplx, bool in_order);
-Tiling single_tiling(const GBlk &blk, const GSeg &seg, bool cplx);
+// Whether the unsplit MFMA tiles of (sealed) blocks are lean ones (GemmLaunch::lean).
+bool lean_tiles(const std::vector<GBlk> &blks, const std::vector<GSeg> &segs, int prec, bool cplx);
+Tiling single_tiling(const GBlk &blk, const GSeg &seg, int prec, bool cplx);
 
 // Fill in what the kernels need to know about a block's segments (chunks, wide).
 void seal_block(GBlk &blk, const GSeg *segs);

@@ -566,7 +566,9 @@ __device__ __forceinline__ void run_chunks(int total, LOAD load, NEXT next, USE 
 // A ring of ACC::depth fragment sets keeps that many chunks' loads in flight across the
 // whole range (segment boundaries included): the MFMAs of chunk c issue while chunks
 // c+1 .. c+depth-1 are still arriving, and chunk c+depth is loaded into the set just consumed.
-template <typename TA, typename TB, int MI, int NI, int PK, typename ACC, typename SEGS>
+// LEAN: see TC_LEAN; no split of K (nslices 1) and no kWideStrides.
+template <typename TA, typename TB, int MI, int NI, int PK, bool LEAN = false, typename ACC,
+          typename SEGS>
 __device__ __forceinline__ void mfma_accumulate(ACC &acc,
                                                 const char *__restrict__ Abase,
                                                 const char *__restrict__ Bbase, const GBlk &blk,
@@ -577,7 +579,7 @@ __device__ __forceinline__ void mfma_accumulate(ACC &acc,
   const int nt = min(16 * NI, blk.N - n0);
   const int total = (blk.chunks - slice + nslices - 1) / nslices;
   if (total <= 0) return;
-  if (blk.wide & kWideStrides) {
+  if (!LEAN && (blk.wide & kWideStrides)) {
     ChunkCursor<TA, TB, SEGS> cur{segs, blk.seg0, blk.nseg, nslices, m0, n0, 0, 0};
     cur.enter(Abase, Bbase);
     cur.skip(slice, Abase, Bbase);  // also steps over empty leading segments
@@ -591,14 +593,36 @@ __device__ __forceinline__ void mfma_accumulate(ACC &acc,
     return;
   }
   auto run = [&](auto w) {
-    ChunkStream<TA, TB, MI, NI, PK, std::is_same<SEGS, SegOne>::value, decltype(w)::value, SEGS>
-        st{segs, blk.seg0, blk.nseg, nslices, m0, n0, mt, nt, r, g};
-    st.start(slice, Abase, Bbase);
-    constexpr int D = ACC::depth;
-    Frag<TA, TB, MI, NI> f[D];
-    run_chunks<D, std::is_same<SEGS, SegOne>::value>(
-        total, [&](int d) { st.load(f[d]); }, [&]() { st.next(Abase, Bbase); },
-        [&](int d) { mma_frag(acc, f[d]); });
+    if constexpr (LEAN) {
+      const int nseg = std::is_same<SEGS, SegOne>::value ? 1 : blk.nseg;  // (total > 0)
+      for (int s = 0; s < nseg; ++s) {
+        const GSeg sg = segs(blk.seg0 + s);
+        ChunkSide<TA, MI, false, (decltype(w)::value & 1) != 0> a;
+        ChunkSide<TB, NI, false, (decltype(w)::value & 2) != 0> b;
+        a.enter((uint64_t)(uintptr_t)(at<const TA>(Abase, sg.a_off) + (int64_t)m0 * sg.sam), sg.sam,
+                sg.sak, mt, 1, r, g);
+        b.enter((uint64_t)(uintptr_t)(at<const TB>(Bbase, sg.b_off) + (int64_t)n0 * sg.sbn), sg.sbn,
+                sg.sbk, nt, 1, r, g);
+        for (int k0 = 0; k0 < sg.K; k0 += 16) {
+          Frag<TA, TB, MI, NI> f;
+          a.load(f.a, sg.K - k0, g);
+          b.load(f.b, sg.K - k0, g);
+          a.base += a.adv;
+          b.base += b.adv;
+          mma_frag(acc, f);
+        }
+      }
+      drain_loads();
+    } else {
+      ChunkStream<TA, TB, MI, NI, PK, std::is_same<SEGS, SegOne>::value, decltype(w)::value, SEGS>
+          st{segs, blk.seg0, blk.nseg, nslices, m0, n0, mt, nt, r, g};
+      st.start(slice, Abase, Bbase);
+      constexpr int D = ACC::depth;
+      Frag<TA, TB, MI, NI> f[D];
+      run_chunks<D, std::is_same<SEGS, SegOne>::value>(
+          total, [&](int d) { st.load(f[d]); }, [&]() { st.next(Abase, Bbase); },
+          [&](int d) { mma_frag(acc, f[d]); });
+    }
   };
   // The loads' widths are fixed per pipeline (a choice between them at every chunk would cost the
   // exact waits); unpacked real operands only, one side at a time.
@@ -658,7 +682,7 @@ __device__ __forceinline__ void dot_epilogue(double cx, double xx, double *slot,
 }
 
 template <int PREC, typename TA, typename TB, typename TC, int MI, int NI, int PK,
-          typename SEGS>
+          bool LEAN = false, typename SEGS>
 __device__ __forceinline__ void wave_tile_real(const char *__restrict__ Abase,
                                                const char *__restrict__ Bbase,
                                                char *__restrict__ Cbase, const GBlk &blk,
@@ -690,7 +714,7 @@ __device__ __forceinline__ void wave_tile_real(const char *__restrict__ Abase,
               row < mt && col < nt);
         }
   }
-  mfma_accumulate<TA, TB, MI, NI, PK>(acc, Abase, Bbase, blk, segs, m0, n0, lane, 0, 1);
+  mfma_accumulate<TA, TB, MI, NI, PK, LEAN>(acc, Abase, Bbase, blk, segs, m0, n0, lane, 0, 1);
   gptr<TC> Cp = at<TC>(Cbase, blk.c_off);
 #pragma unroll
   for (int i = 0; i < MI; ++i)
@@ -1050,7 +1074,7 @@ struct CplxOf<cf> {
   using vec = f2v;
 };
 
-template <typename CT, int MI, int NI, typename SEGS>
+template <typename CT, int MI, int NI, bool LEAN = false, typename SEGS>
 __device__ __forceinline__ void wave_tile_cplx(const char *__restrict__ Abase,
                                                const char *__restrict__ Bbase,
                                                char *__restrict__ Cbase, const GBlk &blk,
@@ -1062,7 +1086,7 @@ __device__ __forceinline__ void wave_tile_cplx(const char *__restrict__ Abase,
   acc.zero();
   acc.sa = (conj & 1) ? op_t(-1) : op_t(1);
   acc.sb = (conj & 2) ? op_t(-1) : op_t(1);
-  mfma_accumulate<c2, c2, MI, NI, 0>(acc, Abase, Bbase, blk, segs, m0, n0, lane, 0, 1);
+  mfma_accumulate<c2, c2, MI, NI, 0, LEAN>(acc, Abase, Bbase, blk, segs, m0, n0, lane, 0, 1);
   const int r = lane & 15, g = lane >> 4;
   const int mt = min(16 * MI, blk.M - m0), nt = min(16 * NI, blk.N - n0);
   gptr<c2> Cp = at<c2>(Cbase, blk.c_off);
@@ -1123,8 +1147,18 @@ __device__ __forceinline__ void wg_tile_cplx(const char *__restrict__ Abase,
 }
 
 // Tile classes: each class is its own kernel instantiation so that it carries only its own
-// register budget (occupancy matters most for the memory-bound row tiles).
-enum TileClass { TC_MIXED = 0, TC_ROWS = 1, TC_BIG = 2, TC_LDS = 3 };
+// register budget (occupancy matters most for the memory-bound row tiles).  TC_LEAN is TC_MIXED for
+// launches of short K.
+enum TileClass { TC_MIXED = 0, TC_ROWS = 1, TC_BIG = 2, TC_LDS = 3, TC_LEAN = 4 };
+// A lean tile walks the segments and their chunks one at a time, with one set of fragments and
+// 32-bit offsets only, so that four waves (complex128: three) fit a SIMD where the ring's registers
+// leave two: with few chunks of K there is little to pipeline, and other waves hide the latency of
+// a tile's first loads and its stores.  Products of 3000 x 3000, us, ring / lean: FP32 K = 17 17.6 / 15.9, 100 32.1 / 31.2; FP64
+// K = 5 22.9 / 17.5, 17 26.6 / 22.5; complex64 K = 17 37.5 / 32.1, 50 58.1 / 51.4.  Complex128 tiles
+// hold so many values that the ring had no depth for them: they are always lean (200 blocks of
+// 300 x 8, K = 200: 42 / 40; 100000 x 10, K = 200: 96 / 85).
+template <typename T>
+constexpr int kLeanWaves = std::is_same<T, cd>::value ? 3 : std::is_same<T, cf>::value ? 5 : 4;
 
 template <int PREC, typename TA, typename TB, typename TC, bool CPLX, int CLS, int PK,
           typename SEGS>
@@ -1132,12 +1166,13 @@ __device__ __forceinline__ void run_tile(int kind, const char *A, const char *B,
                                          const GBlk &blk, SEGS segs, int m0, int n0, int lane,
                                          int conj, const double *dotx = nullptr,
                                          double *dslot = nullptr, int64_t nslots = 0) {
+  constexpr bool L = CLS == TC_LEAN;
   if constexpr (CPLX) {
     switch (kind) {
-      case TK_1x1: wave_tile_cplx<TA, 1, 1>(A, B, C, blk, segs, m0, n0, lane, conj); break;
-      case TK_2x1: wave_tile_cplx<TA, 2, 1>(A, B, C, blk, segs, m0, n0, lane, conj); break;
-      case TK_1x2: wave_tile_cplx<TA, 1, 2>(A, B, C, blk, segs, m0, n0, lane, conj); break;
-      default: wave_tile_cplx<TA, 2, 2>(A, B, C, blk, segs, m0, n0, lane, conj); break;
+      case TK_1x1: wave_tile_cplx<TA, 1, 1, L>(A, B, C, blk, segs, m0, n0, lane, conj); break;
+      case TK_2x1: wave_tile_cplx<TA, 2, 1, L>(A, B, C, blk, segs, m0, n0, lane, conj); break;
+      case TK_1x2: wave_tile_cplx<TA, 1, 2, L>(A, B, C, blk, segs, m0, n0, lane, conj); break;
+      default: wave_tile_cplx<TA, 2, 2, L>(A, B, C, blk, segs, m0, n0, lane, conj); break;
     }
   } else if constexpr (CLS == TC_ROWS) {
     wave_rows<TA, TB, TC, PK>(A, B, C, blk, segs, m0, lane);
@@ -1147,20 +1182,20 @@ __device__ __forceinline__ void run_tile(int kind, const char *A, const char *B,
   } else {
     switch (kind) {
       case TK_1x1:
-        wave_tile_real<PREC, TA, TB, TC, 1, 1, PK>(A, B, C, blk, segs, m0, n0, lane, dotx, dslot,
-                                                   nslots);
+        wave_tile_real<PREC, TA, TB, TC, 1, 1, PK, L>(A, B, C, blk, segs, m0, n0, lane, dotx, dslot,
+                                                      nslots);
         break;
       case TK_2x1:
-        wave_tile_real<PREC, TA, TB, TC, 2, 1, PK>(A, B, C, blk, segs, m0, n0, lane, dotx, dslot,
-                                                   nslots);
+        wave_tile_real<PREC, TA, TB, TC, 2, 1, PK, L>(A, B, C, blk, segs, m0, n0, lane, dotx, dslot,
+                                                      nslots);
         break;
       case TK_1x2:
-        wave_tile_real<PREC, TA, TB, TC, 1, 2, PK>(A, B, C, blk, segs, m0, n0, lane, dotx, dslot,
-                                                   nslots);
+        wave_tile_real<PREC, TA, TB, TC, 1, 2, PK, L>(A, B, C, blk, segs, m0, n0, lane, dotx, dslot,
+                                                      nslots);
         break;
       default:
-        wave_tile_real<PREC, TA, TB, TC, 2, 2, PK>(A, B, C, blk, segs, m0, n0, lane, dotx, dslot,
-                                                   nslots);
+        wave_tile_real<PREC, TA, TB, TC, 2, 2, PK, L>(A, B, C, blk, segs, m0, n0, lane, dotx, dslot,
+                                                      nslots);
         break;
     }
   }
@@ -1169,12 +1204,10 @@ __device__ __forceinline__ void run_tile(int kind, const char *A, const char *B,
 // grouped launch: tiles, blocks and segments come from device arrays; one wave per tile.
 // Workgroup w runs on XCD w % kXcds and takes tiles from that XCD's range of the list.
 template <int PREC, typename TA, typename TB, typename TC, bool CPLX, int CLS, int PK>
-__global__ __launch_bounds__(64 * kWaves, 2) void k_grouped(const GTile *__restrict__ tiles,
-                                                        int per_xcd, const GBlk *__restrict__ blks,
-                                                        const GSeg *__restrict__ segs,
-                                                        const char *A, const char *B, char *C,
-                                                        int conj, const double *dotx,
-                                                        double *dotp) {
+__global__ __launch_bounds__(64 * kWaves, CLS == TC_LEAN ? kLeanWaves<TA> : 2) void k_grouped(
+    const GTile *__restrict__ tiles, int per_xcd, const GBlk *__restrict__ blks,
+    const GSeg *__restrict__ segs, const char *A, const char *B, char *C, int conj,
+    const double *dotx, double *dotp) {
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int x = blockIdx.x % kXcds;
@@ -1552,19 +1585,21 @@ int launch_mix_t(const GemmLaunch &g, hipStream_t s) {
 
 // single-block launch: one block with one segment, tiles derived from the launch index, so a
 // plain GEMM needs no device-side task list (mixed MFMA class)
-template <int PREC, typename TA, typename TB, typename TC, bool CPLX>
-__global__ __launch_bounds__(64 * kWaves, 2) void k_single(GBlk blk, GSeg seg, int kind,
-                                                       int tiles_n, int ntiles, const char *A,
-                                                       const char *B, char *C, int conj) {
+template <int PREC, typename TA, typename TB, typename TC, bool CPLX, int CLS>
+__global__ __launch_bounds__(64 * kWaves, CLS == TC_LEAN ? kLeanWaves<TA> : 2) void k_single(
+    GBlk blk, GSeg seg, int kind, int tiles_n, int ntiles, const char *A, const char *B, char *C,
+    int conj) {
+  // (checked by launch_t: as constants they take no registers and no arithmetic per element)
+  blk.csn = 1;
+  blk.alpha = 1.0;
+  blk.beta = blk.alpha_im = blk.beta_im = 0.0;
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int tr = kind == TK_1x1 || kind == TK_1x2 ? 16 : 32;
   const int tc = kind == TK_1x1 || kind == TK_2x1 ? 16 : 32;
   for (int t = blockIdx.x * kWaves + wave; t < ntiles; t += gridDim.x * kWaves) {
     const int m0 = (t / tiles_n) * tr, n0 = (t % tiles_n) * tc;
-    run_tile<PREC, TA, TB, TC, CPLX, TC_MIXED, 0>(kind, A, B, C, blk, SegOne{seg}, m0, n0,
-                                                      lane,
-                                               conj);
+    run_tile<PREC, TA, TB, TC, CPLX, CLS, 0>(kind, A, B, C, blk, SegOne{seg}, m0, n0, lane, conj);
   }
 }
 
@@ -1629,10 +1664,19 @@ void launch_real(const GemmLaunch &g, int cls, int wg_grid, int wave_grid, hipSt
     hipLaunchKernelGGL((k_grouped<PREC, TA, TB, TC, false, TC_BIG, PK>), dim3(wave_grid),
                        dim3(64 * kWaves), 0, s, g.tiles, P, g.blks, g.segs, A, B, C, g.conj, dx,
                        dp);
-  else
+  else {
+    if constexpr (PK == 0 && PREC != CXA_PREC_FP32X3) {
+      if (g.lean && !dp) {
+        hipLaunchKernelGGL((k_grouped<PREC, TA, TB, TC, false, TC_LEAN, PK>), dim3(wave_grid),
+                           dim3(64 * kWaves), 0, s, g.tiles, P, g.blks, g.segs, A, B, C, g.conj,
+                           nullptr, nullptr);
+        return;
+      }
+    }
     hipLaunchKernelGGL((k_grouped<PREC, TA, TB, TC, false, TC_MIXED, PK>), dim3(wave_grid),
                        dim3(64 * kWaves), 0, s, g.tiles, P, g.blks, g.segs, A, B, C, g.conj, dx,
                        dp);
+  }
 }
 
 template <int PREC, typename TA, typename TB, typename TC, bool CPLX>
@@ -1648,7 +1692,9 @@ int launch_t(const GemmLaunch &g, hipStream_t s) {
       return fail(CXA_ERR_INVALID, "single-block GEMM: packed layouts are not supported");
     const GBlk &b = g.blk0;
     if (b.M <= 0 || b.N <= 0) return CXA_OK;
-    const Tiling tl = single_tiling(b, g.seg0, CPLX);
+    if (b.csn != 1 || b.alpha != 1.0 || b.beta != 0.0 || b.alpha_im != 0.0 || b.beta_im != 0.0)
+      return fail(CXA_ERR_INVALID, "single-block GEMM: plain products with unit stride along n only");
+    const Tiling tl = single_tiling(b, g.seg0, PREC, CPLX);
     int kind = tl.kind;
     if constexpr (PREC != CXA_PREC_FP32X3) {
       if (is_lds(kind)) {
@@ -1682,9 +1728,19 @@ int launch_t(const GemmLaunch &g, hipStream_t s) {
       return fail(CXA_ERR_UNSUPPORTED, "GEMM too large: %lld tiles", (long long)nt64);
     const int ntiles = (int)nt64;
     const int grid = std::min((ntiles + kWaves - 1) / kWaves, 8192);
-    hipLaunchKernelGGL((k_single<PREC, TA, TB, TC, CPLX>), dim3(grid), dim3(64 * kWaves), 0, s,
-                       b, g.seg0, kind, tiles_n, ntiles, (const char *)g.A, (const char *)g.B,
-                       (char *)g.C, g.conj);
+    auto launch = [&](auto cls) {
+      hipLaunchKernelGGL((k_single<PREC, TA, TB, TC, CPLX, decltype(cls)::value>), dim3(grid),
+                         dim3(64 * kWaves), 0, s, b, g.seg0, kind, tiles_n, ntiles,
+                         (const char *)g.A, (const char *)g.B, (char *)g.C, g.conj);
+    };
+    if constexpr (PREC != CXA_PREC_FP32X3) {
+      if (tl.lean) {
+        launch(std::integral_constant<int, TC_LEAN>{});
+        CXA_HIP(hipGetLastError());
+        return CXA_OK;
+      }
+    }
+    launch(std::integral_constant<int, TC_MIXED>{});
     CXA_HIP(hipGetLastError());
     return CXA_OK;
   }
@@ -1731,11 +1787,18 @@ int launch_t(const GemmLaunch &g, hipStream_t s) {
       hipLaunchKernelGGL((k_grouped_split_cplx<TA, 4>), dim3(wg_grid), dim3(64 * 4), 0, s, g.tiles,
                          P, g.blks, g.segs, (const char *)g.A, (const char *)g.B, (char *)g.C,
                          g.conj);
-    else
-      hipLaunchKernelGGL((k_grouped<PREC, TA, TB, TC, true, TC_MIXED, 0>), dim3(wave_grid),
-                       dim3(64 * kWaves), 0, s, g.tiles, P, g.blks, g.segs,
-                       (const char *)g.A, (const char *)g.B, (char *)g.C, g.conj, nullptr,
-                       nullptr);
+    else {
+      auto launch = [&](auto c) {
+        hipLaunchKernelGGL((k_grouped<PREC, TA, TB, TC, true, decltype(c)::value, 0>),
+                           dim3(wave_grid), dim3(64 * kWaves), 0, s, g.tiles, P, g.blks, g.segs,
+                           (const char *)g.A, (const char *)g.B, (char *)g.C, g.conj, nullptr,
+                           nullptr);
+      };
+      if (g.lean)
+        launch(std::integral_constant<int, TC_LEAN>{});
+      else
+        launch(std::integral_constant<int, TC_MIXED>{});
+    }
   }
   CXA_HIP(hipGetLastError());
   return CXA_OK;
