@@ -77,7 +77,7 @@ struct PlanVariant {
   int splitk = 0;  // waves per tile of the split-K launch, 0 = none (mix plans: 1 = four-wave)
   int tile_class = 0;
   int launch_kind = -1;  // mix plans and LDS tiles: the one tile kind of the launch
-  bool lean = false;     // GemmLaunch::lean
+  bool lean = false, rows4 = false;  // GemmLaunch::lean, rows4
 };
 
 struct cxa_bc_plan {
@@ -187,6 +187,7 @@ int build_variant(cxa_bc_plan *p, int index) {
                        prefer_splitk(p->blks, p->segs, tiles, v.tile_class)));
     // eight-wave split-K only for MFMA tiles (row tiles always split over four waves)
     v.splitk = !split ? 0 : (v.split_mode == 2 && v.tile_class == 0 ? 8 : 4);
+    v.rows4 = v.tile_class == 1 && has_rows4(tiles);
     v.lean = v.tile_class == 0 && !split && lean_tiles(p->blks, p->segs, prec, !real);
   }
   v.ntiles = (int)tiles.size();
@@ -1038,6 +1039,7 @@ int bc_exec_typed(const cxa_bc_plan *p, const void *L, const void *R, void *C, i
   g.splitk = v.splitk;
   g.tile_class = v.tile_class;
   g.lean = v.lean;
+  g.rows4 = v.rows4;
   g.conj = is_complex(p->dtype) ? conj : 0;
   g.dot_x = lay->dot_x;
   g.dot_part = lay->dot_part;
@@ -1347,6 +1349,7 @@ extern "C" int cxa_gemm_batch(int dtype, const char *transa, const char *transb,
   g.tile_class = cls;
   g.kind0 = tl.kind;
   g.splitk = tl.split;
+  g.rows4 = cls == 1 && has_rows4(tiles);
   g.lean = cls == 0 && !tl.split && lean_tiles(blks, segs, native_prec(dtype), cplx);
   rc = launch_grouped_gemm(g, s);
   if (rc) return rc;

@@ -201,6 +201,20 @@ int make_tiles(const std::vector<GBlk> &blks, const std::vector<GSeg> &segs,
   std::stable_sort(order.begin(), order.end(), [&](int x, int y) { return key(x) < key(y); });
   thread_local std::vector<Item> items;
   items.clear();
+  auto k_of = [&](const GBlk &b) {
+    int64_t ksum = 0;
+    for (int s = 0; s < b.nseg; ++s) ksum += segs[b.seg0 + s].K;
+    return ksum;
+  };
+  // rows of short K (the MPO steps, K of a few): a wave's four loads and stores take less than
+  // reading its tile, block and segment records, so it takes four times the rows
+  auto short_rows = [&](const GBlk &b) {
+    return b.N <= kShortRowsN && b.M > tile_rows(TK_ROWS) && k_of(b) <= kShortRowsK;
+  };
+  int64_t rows = 0;
+  if (cls == TC_ROWS)
+    for (int bi : order)
+      if (short_rows(blks[bi])) rows += blks[bi].M;
   for (int bi : order) {
     const GBlk &b = blks[bi];
     int kind;
@@ -212,13 +226,9 @@ int make_tiles(const std::vector<GBlk> &blks, const std::vector<GSeg> &segs,
       kind = kind_override;
     else
       kind = default_kind(b.M, b.N);
-    int64_t ksum = 0;
-    for (int s = 0; s < b.nseg; ++s) ksum += segs[b.seg0 + s].K;
+    const int64_t ksum = k_of(b);
     int tr = tile_rows(kind), tc = kind == TK_ROWS ? b.N : tile_cols(kind);
-    // rows of short K (the MPO steps, K of a few): a wave's four loads and stores take less than
-    // reading its tile, block and segment records, so it takes four times the rows
-    if (kind == TK_ROWS && ksum <= kShortRowsK && b.N <= kShortRowsN && b.M > tr)
-      tr *= kShortRows;
+    if (kind == TK_ROWS && rows >= kShortRowsMin && short_rows(b)) tr *= kShortRows;
     for (int m0 = 0; m0 < b.M; m0 += tr)
       for (int n0 = 0; n0 < b.N; n0 += tc)
         items.push_back({GTile{(int32_t)bi, m0, kind == TK_ROWS ? tr : n0, kind}, (ksum + 16) * tr * tc});
@@ -253,6 +263,12 @@ int make_tiles(const std::vector<GBlk> &blks, const std::vector<GSeg> &segs,
   }
   *per_xcd = (int)P;
   return cls;
+}
+
+bool has_rows4(const std::vector<GTile> &tiles) {
+  for (const GTile &t : tiles)
+    if (t.blk >= 0 && t.kind == TK_ROWS && t.n0 > tile_rows(TK_ROWS)) return true;
+  return false;
 }
 
 bool prefer_splitk(const std::vector<GBlk> &blks, const std::vector<GSeg> &segs,

@@ -69,8 +69,13 @@ inline int tile_cols(int kind) {
 }
 
 constexpr int kRowsN = 8;  // widest block the row-streaming path takes
-// Rows per lane of a row tile with short K, and the K and N up to which it is taken.
-constexpr int kShortRows = 4, kShortRowsK = 32, kShortRowsN = 4;
+// Rows per lane of a row tile with short K, the K and N up to which it is taken, and the rows of such
+// blocks from which it is: with fewer, its tiles leave CUs without work (N = K = 3 in FP64, one row /
+// four: 10^5 rows 4.6 / 5.0 us, 1.5 x 10^5 5.3 / 5.1, 3 x 10^5 6.9 / 5.8).  With longer rows of A the
+// lines that a wave comes back to for its next k no longer stay in its cache (N = 4 in FP64, 4 x 10^6
+// rows: K = 8 144 / 119 us, 12 204 / 277; N = 1, K = 32 747 / 1462).
+constexpr int kShortRows = 4, kShortRowsK = 8, kShortRowsN = 4;
+constexpr int64_t kShortRowsMin = 1 << 17;
 
 struct GTile {
   int32_t blk, m0, n0, kind;  // (TK_ROWS: n0 is the tile's rows, 64 or 64 * kShortRows)
@@ -91,6 +96,7 @@ struct GemmLaunch {
   // interleaved over its waves (mix launches: nonzero = four-wave workgroups)
   int splitk = 0;
   int tile_class = 0;   // the class make_tiles returned
+  bool rows4 = false;   // row tiles: some of them have kShortRows rows per lane
   bool lean = false;    // MFMA tiles of short K: kernels of fewer registers (TC_LEAN)
   const MixOut *outs = nullptr;  // non-null: mix launch (blks are items, segs are slices)
   int conj = 0;  // complex dtypes: bit 0 conjugates A, bit 1 conjugates B
@@ -168,6 +174,8 @@ Tiling default_tiling(const std::vector<GBlk> &blks, const std::vector<GSeg> &se
 // 5.8e-16, FP32 2.3e-7 / 3.1e-7; of 60 blocks of 160 x 160, K = 400, in FP32: 1.8e-7 / 3.6e-7.
 Tiling plan_tiling(const std::vector<GBlk> &blks, const std::vector<GSeg> &segs, int prec,
                    bool cplx, bool in_order);
+// Whether a list of row tiles holds any of kShortRows rows per lane.
+bool has_rows4(const std::vector<GTile> &tiles);
 // Whether the unsplit MFMA tiles of (sealed) blocks are lean ones (GemmLaunch::lean).
 bool lean_tiles(const std::vector<GBlk> &blks, const std::vector<GSeg> &segs, int prec, bool cplx);
 Tiling single_tiling(const GBlk &blk, const GSeg &seg, int prec, bool cplx);

@@ -1149,7 +1149,10 @@ __device__ __forceinline__ void wg_tile_cplx(const char *__restrict__ Abase,
 // Tile classes: each class is its own kernel instantiation so that it carries only its own
 // register budget (occupancy matters most for the memory-bound row tiles).  TC_LEAN is TC_MIXED for
 // launches of short K.
-enum TileClass { TC_MIXED = 0, TC_ROWS = 1, TC_BIG = 2, TC_LDS = 3, TC_LEAN = 4 };
+// TC_ROWS4 is TC_ROWS for launches that hold tiles of kShortRows rows per lane (GemmLaunch::rows4): their
+// registers (83 to 99 for 40 to 55) and LDS would hold the others to five workgroups a CU (10^6 rows
+// of N = 6, K = 10: FP32 46 us for 39; 300000 of N = 8, K = 20: 44 for 34).
+enum TileClass { TC_MIXED = 0, TC_ROWS = 1, TC_BIG = 2, TC_LDS = 3, TC_LEAN = 4, TC_ROWS4 = 5 };
 // A lean tile walks the segments and their chunks one at a time, with one set of fragments and
 // 32-bit offsets only, so that four waves (complex128: three) fit a SIMD where the ring's registers
 // leave two: with few chunks of K there is little to pipeline, and other waves hide the latency of
@@ -1174,7 +1177,7 @@ __device__ __forceinline__ void run_tile(int kind, const char *A, const char *B,
       case TK_1x2: wave_tile_cplx<TA, 1, 2, L>(A, B, C, blk, segs, m0, n0, lane, conj); break;
       default: wave_tile_cplx<TA, 2, 2, L>(A, B, C, blk, segs, m0, n0, lane, conj); break;
     }
-  } else if constexpr (CLS == TC_ROWS) {
+  } else if constexpr (CLS == TC_ROWS || CLS == TC_ROWS4) {
     wave_rows<TA, TB, TC, PK>(A, B, C, blk, segs, m0, lane);
   } else if constexpr (CLS == TC_BIG) {
     wave_tile_real<PREC, TA, TB, TC, 4, 2, PK>(A, B, C, blk, segs, m0, n0, lane, dotx, dslot,
@@ -1221,7 +1224,7 @@ __global__ __launch_bounds__(64 * kWaves, CLS == TC_LEAN ? kLeanWaves<TA> : 2) v
       continue;
     }
     const GBlk blk = blks[tl.blk];
-    if constexpr (CLS == TC_ROWS) {
+    if constexpr (CLS == TC_ROWS4) {
       __shared__ double out[kWaves][kShortRows * 64 * kShortRowsN];
       if (tl.n0 > 64) {  // (uniform over the wave)
         wave_rows_short<TA, TB, TC, PK>(A, B, C, blk, SegArray{segs}, tl.m0, lane, out[wave]);
@@ -1656,6 +1659,10 @@ void launch_real(const GemmLaunch &g, int cls, int wg_grid, int wave_grid, hipSt
   else if (g.splitk && cls == TC_MIXED)
     hipLaunchKernelGGL((k_grouped_split<PREC, TA, TB, TC, TC_MIXED, kWaves, PK>), dim3(wg_grid),
                        dim3(64 * kWaves), 0, s, g.tiles, P, g.blks, g.segs, A, B, C, dx, dp);
+  else if (cls == TC_ROWS && g.rows4)
+    hipLaunchKernelGGL((k_grouped<PREC, TA, TB, TC, false, TC_ROWS4, PK>), dim3(wave_grid),
+                       dim3(64 * kWaves), 0, s, g.tiles, P, g.blks, g.segs, A, B, C, g.conj,
+                       nullptr, nullptr);
   else if (cls == TC_ROWS)
     hipLaunchKernelGGL((k_grouped<PREC, TA, TB, TC, false, TC_ROWS, PK>), dim3(wave_grid),
                        dim3(64 * kWaves), 0, s, g.tiles, P, g.blks, g.segs, A, B, C, g.conj,
