@@ -1,4 +1,4 @@
-// Grouped GEMM launches in FP32 with an FP32 A operand, and complex64.
+// Grouped GEMM launches in FP32 with an FP32 A operand.
 #define CXA_GEMM_TU fp32
 #include "gemm_kernels.hpp"
 
@@ -13,8 +13,7 @@ int launch_gemm_fp32(const GemmLaunch &g, hipStream_t s) {
   CXA_F32_CASE(float, double, float, CXA_F32, CXA_F64, CXA_F32)
   CXA_F32_CASE(float, double, double, CXA_F32, CXA_F64, CXA_F64)
 #undef CXA_F32_CASE
-  if (a == CXA_C64 && b == CXA_C64 && c == CXA_C64)
-    return launch_t<CXA_PREC_FP32, cf, cf, cf, true>(g, s);
+  if (a == CXA_C64 && b == CXA_C64 && c == CXA_C64) return launch_gemm_c64(g, s);
   if (a == CXA_F64) return launch_gemm_fp32_a64(g, s);
   return fail(CXA_ERR_UNSUPPORTED, "grouped GEMM: FP32 with dtypes (%d,%d,%d)", a, b, c);
 }

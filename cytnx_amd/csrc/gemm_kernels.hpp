@@ -1817,6 +1817,7 @@ int launch_t(const GemmLaunch &g, hipStream_t s) {
 int launch_gemm_fp64(const GemmLaunch &g, hipStream_t s);
 int launch_gemm_fp32(const GemmLaunch &g, hipStream_t s);
 int launch_gemm_fp32_a64(const GemmLaunch &g, hipStream_t s);
+int launch_gemm_c64(const GemmLaunch &g, hipStream_t s);
 int launch_gemm_fp32x3(const GemmLaunch &g, hipStream_t s);
 int launch_mix(const GemmLaunch &g, hipStream_t s);
 
