@@ -403,6 +403,27 @@ int make_block_plan(int dtype, int rankL, int nbL, const uint64_t *itoiL, const 
   }
   p->npairs = (int64_t)pairs.size();
 
+  // Extents of the output blocks, axis by axis, as their operands have them: strides are taken
+  // apart along these axes.  (An output whose shapes only multiply to the same rows and columns
+  // is the same row-major matrix; a permuted one has no such meaning.)
+  std::vector<uint64_t> extC(shapeC, shapeC + (int64_t)nbC * rankC);
+  std::vector<char> seenC(nbC, 0);
+  for (const Pair &pr : pairs) {
+    const uint64_t *sa = shapeL + (int64_t)pr.a * rankL, *sb = shapeR + (int64_t)pr.b * rankR;
+    uint64_t *ec = extC.data() + (int64_t)pr.t * rankC;
+    int64_t M = 1, N = 1;
+    bool same = true;
+    for (int i = 0; i < rankC; ++i) {
+      (i < n1 ? M : N) *= (int64_t)ec[i];
+      same = same && ec[i] == (i < n1 ? sa[nc1[i]] : sb[nc2[i - n1]]);
+    }
+    CXA_CHECK(pr.M == M && pr.N == N && (same || (!out_axes && !seenC[pr.t])), CXA_ERR_INVALID,
+              "block contract: output block %d shape does not match its pair (%lld x %lld)", pr.t,
+              (long long)pr.M, (long long)pr.N);
+    seenC[pr.t] = 1;
+    for (int i = 0; i < rankC; ++i) ec[i] = i < n1 ? sa[nc1[i]] : sb[nc2[i - n1]];
+  }
+
   // Row-major strides of an array with `rank` extents.
   auto strides_of = [](int rank, const uint64_t *ext, int64_t *st) {
     int64_t acc = 1;
@@ -438,7 +459,7 @@ int make_block_plan(int dtype, int rankL, int nbL, const uint64_t *itoiL, const 
     uint64_t ext[32];
     int64_t st[32];
     for (int i = 0; i < rankC; ++i)
-      ext[i] = shapeC[(int64_t)b * rankC + (out_axes ? (int)out_axes[i] : i)];
+      ext[i] = extC[(int64_t)b * rankC + (out_axes ? (int)out_axes[i] : i)];
     strides_of(rankC, ext, st);
     for (int i = 0; i < rankC; ++i)
       stC[(size_t)b * 32 + (out_axes ? (int)out_axes[i] : i)] = st[i];
@@ -479,7 +500,7 @@ int make_block_plan(int dtype, int rankL, int nbL, const uint64_t *itoiL, const 
     return R;
   };
   auto runs_m = [&](int t) {
-    const uint64_t *sc = shapeC + (int64_t)t * rankC;
+    const uint64_t *sc = extC.data() + (int64_t)t * rankC;
     return runs_of(n1, sc, [&, t](int i, int j) {
       if (stC[(size_t)t * 32 + i] != (int64_t)sc[j] * stC[(size_t)t * 32 + j]) return false;
       for (int pi : by_target[t]) {
@@ -490,7 +511,7 @@ int make_block_plan(int dtype, int rankL, int nbL, const uint64_t *itoiL, const 
     });
   };
   auto runs_n = [&](int t) {
-    const uint64_t *sc = shapeC + (int64_t)t * rankC + n1;
+    const uint64_t *sc = extC.data() + (int64_t)t * rankC + n1;
     return runs_of(n2, sc, [&, t](int i, int j) {
       if (stC[(size_t)t * 32 + n1 + i] != (int64_t)sc[j] * stC[(size_t)t * 32 + n1 + j])
         return false;
@@ -547,7 +568,7 @@ int make_block_plan(int dtype, int rankL, int nbL, const uint64_t *itoiL, const 
   std::vector<CopyJob> copiesC;
   if (!in_place && out_axes && rankC <= 16) {
     for (int t = 0; t < nbC; ++t) {
-      const uint64_t *sc = shapeC + (int64_t)t * rankC;
+      const uint64_t *sc = extC.data() + (int64_t)t * rankC;
       CopyJob j{};
       int64_t n = 1;
       for (int i = 0; i < rankC; ++i) {
@@ -638,7 +659,7 @@ int make_block_plan(int dtype, int rankL, int nbL, const uint64_t *itoiL, const 
   int64_t rows_unit = 0, cols_unit = 0;  // output elements whose m or n is C's unit stride
   p->blks.reserve(nbC);
   for (int t = 0; t < nbC; ++t) {
-    const uint64_t *sc = shapeC + (int64_t)t * rankC;
+    const uint64_t *sc = extC.data() + (int64_t)t * rankC;
     int64_t M = 1, N = 1;
     for (int i = 0; i < n1; ++i) M *= (int64_t)sc[i];
     for (int i = 0; i < n2; ++i) N *= (int64_t)sc[n1 + i];
@@ -646,9 +667,6 @@ int make_block_plan(int dtype, int rankL, int nbL, const uint64_t *itoiL, const 
               "block contract: output block too large");
     for (int pi : by_target[t]) {
       const Pair &pr = pairs[pi];
-      CXA_CHECK(pr.M == M && pr.N == N, CXA_ERR_INVALID,
-                "block contract: output block %d shape does not match its pair (%lld x %lld)", t,
-                (long long)pr.M, (long long)pr.N);
       CXA_CHECK(pr.K <= INT32_MAX, CXA_ERR_UNSUPPORTED, "block contract: K too large");
       p->flops += 2.0 * cplx * (double)pr.M * (double)pr.N * (double)pr.K;
     }
