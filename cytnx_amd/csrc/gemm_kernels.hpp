@@ -1715,7 +1715,8 @@ int launch_t(const GemmLaunch &g, hipStream_t s) {
         return CXA_OK;
       }
     }
-    if (kind == TK_ROWS || kind == TK_4x2) kind = TK_2x2;  // single launches: mixed class
+    // single launches: mixed class (FP32X3 has no LDS tiles)
+    if (kind == TK_ROWS || kind == TK_4x2 || is_lds(kind)) kind = TK_2x2;
     if constexpr (PREC != CXA_PREC_FP32X3) {
       if (tl.split > 0) {
         const int64_t tn = (b.N + 15) / 16, n = (int64_t)((b.M + 15) / 16) * tn;
