@@ -83,7 +83,8 @@ bool bc_is_mix(const cxa_bc_plan *p);
 int bc_ensure(const cxa_bc_plan *p, int prec, hipStream_t s, bool step = false);
 int bc_prepare(const cxa_bc_plan *p);
 // Tile slots a dot-product epilogue of an execution as a chain's step at precision prec writes
-// (the launch's tile list length), or 0 when that launch cannot carry one (mix, complex, row-streaming tiles).
+// (the launch's tile list length), or 0 when that launch cannot carry one (mix, complex,
+// row-streaming tiles).
 int bc_dot_slots(const cxa_bc_plan *p, int prec);
 int64_t bc_workspace_elems(const cxa_bc_plan *p);
 double bc_flops(const cxa_bc_plan *p);

@@ -1,6 +1,6 @@
 // Grouped MFMA GEMM: precision dispatch and host-side tile planning (the kernels are in
-// gemm_kernels.hpp, instantiated by gemm_fp64.hip, gemm_fp32.hip, gemm_fp32x3.hip and
-// gemm_mix.hip).
+// gemm_kernels.hpp, instantiated by gemm_fp64.hip, gemm_fp32.hip, gemm_c64.hip, gemm_fp32x3.hip
+// and gemm_mix.hip).
 #define CXA_GEMM_TU main
 #include "gemm_kernels.hpp"
 
@@ -32,8 +32,8 @@ int64_t tiles_of(const GBlk &b, int t) {
   return (int64_t)((b.M + t - 1) / t) * ((b.N + t - 1) / t);
 }
 
-// The choice, from counts of tiles and the mean K in chunks of 16.  A 16 x 16 tile is the finest split
-// of the output, and a wave works through its K one MFMA after another, so few tiles leave SIMDs
+// The choice, from counts of tiles and the mean K in chunks of 16.  A 16 x 16 tile is the finest
+// split of the output, and a wave works through its K one MFMA after another, so few tiles leave SIMDs
 // idle: up to kFew of them (two, complex four, times the CUs; single products half) the four waves
 // of a workgroup share a tile's K, which then also hides their load latency.  Beyond, tiles of one
 // wave: the default ones from kManyDirect of them (three per CU), else 16 x 16.  With more than
@@ -45,13 +45,13 @@ int64_t tiles_of(const GBlk &b, int t) {
 // Measured, us:
 //   split 16x16 / LDS 32x32: real products of n = 128 3.9 / 5.2, 256 4.9 / 7.3, 512 (1024 tiles)
 //   21.2 / 11.5; complex128 n = 256 6.4 / 13.9, 384 x 960 x 192 (288 tiles) 27 / 43, 512 30 / 26;
-//   default / 16x16: FP32 20000 x 33 x 20 (625 of them) 5.0 / 4.8, 600 x 600, K = 100 7.0 / 5.7, 1000 x
-//   1000 (1024) 7.3 / 9.5, 200 blocks of 60 x 60 (800), K = 50 5.7 / 7.4;
-//   direct / LDS (64x64 of real types): 3000 x 3000, K = 33 FP32 19.0 / 30.7, complex64 41.7 / 67.6; K =
-//   100 FP32 31 / 41, FP64 47.7 / 45.1, complex128 137 / 147; 1600 x 1600 complex128, K = 200 87 / 77,
-//   1000 x 1000 (1024 LDS tiles) 37 / 43; 60 blocks of 160 x 160, K = 400 complex128 107 / 86;
-//   covering twice the area: 100000 x 10 x 100 FP64 19.6 / 30.7, 10 x 400 x 20000 FP64 13 / 31; 200
-//   blocks of 300 x 8, K = 100 complex64 15.6 / 24.5.
+//   default / 16x16: FP32 20000 x 33 x 20 (625 of them) 5.0 / 4.8, 600 x 600, K = 100 7.0 / 5.7,
+//   1000 x 1000 (1024) 7.3 / 9.5, 200 blocks of 60 x 60 (800), K = 50 5.7 / 7.4;
+//   direct / LDS (64x64 of real types): 3000 x 3000, K = 33 FP32 19.0 / 30.7, complex64 41.7 / 67.6;
+//   K = 100 FP32 31 / 41, FP64 47.7 / 45.1, complex128 137 / 147; 1600 x 1600 complex128, K = 200
+//   87 / 77, 1000 x 1000 (1024 LDS tiles) 37 / 43; 60 blocks of 160 x 160, K = 400 complex128
+//   107 / 86; covering twice the area: 100000 x 10 x 100 FP64 19.6 / 30.7, 10 x 400 x 20000 FP64
+//   13 / 31; 200 blocks of 300 x 8, K = 100 complex64 15.6 / 24.5.
 constexpr int64_t kFewReal = 512, kFewCplx = 1024, kMany64 = 192, kManyDirect = 768;
 constexpr int64_t kShortChunks = 7, kShortC128 = 13, kRoundLow = 768, kRoundHigh = 1400;
 
@@ -152,7 +152,8 @@ Tiling single_tiling(const GBlk &b, const GSeg &s, int prec, bool cplx) {
   c.add(b, &s);
   const int kind = default_kind(b.M, b.N);
   if (c.n16 <= (cplx ? kFewCplx : kFewReal) / 2 && s.K > 32) return {TK_1x1, 4};
-  return {c.stay_direct(false) ? c.direct(kind) : c.large(kind, cplx, false), 0, c.lean(prec, cplx)};
+  return {c.stay_direct(false) ? c.direct(kind) : c.large(kind, cplx, false), 0,
+          c.lean(prec, cplx)};
 }
 
 void seal_block(GBlk &b, const GSeg *segs) {
@@ -231,7 +232,8 @@ int make_tiles(const std::vector<GBlk> &blks, const std::vector<GSeg> &segs,
     if (kind == TK_ROWS && rows >= kShortRowsMin && short_rows(b)) tr *= kShortRows;
     for (int m0 = 0; m0 < b.M; m0 += tr)
       for (int n0 = 0; n0 < b.N; n0 += tc)
-        items.push_back({GTile{(int32_t)bi, m0, kind == TK_ROWS ? tr : n0, kind}, (ksum + 16) * tr * tc});
+        items.push_back({GTile{(int32_t)bi, m0, kind == TK_ROWS ? tr : n0, kind},
+                         (ksum + 16) * tr * tc});
   }
   // kXcds contiguous ranges of equal tile count (at these sizes a tile's time is mostly its
   // fixed chain of dependent loads, so equal counts balance better than equal flops, and the

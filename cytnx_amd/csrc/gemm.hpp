@@ -6,8 +6,8 @@
 //   C_blk[m, n] = alpha * sum_seg sum_k A_seg[m, k] * B_seg[k, n]  (+ beta * C_blk[m, n])
 // with every operand a strided matrix view (any row/column strides), so permutes that keep an
 // operand a strided matrix are fused into the loads.  Output blocks are cut into wave tiles
-// (GTile); one wave owns one tile and loops over all of its segments, so accumulation order
-// is fixed and no atomics are used.
+// (GTile); one wave, or the four of a workgroup (split-K and LDS tiles), owns one tile and loops
+// over all of its segments, so accumulation order is fixed and no atomics are used.
 #pragma once
 
 #include <hip/hip_runtime.h>
@@ -34,7 +34,7 @@ struct GBlk {
   int32_t seg0, nseg;
   int32_t out0, nout;  // mix launches only: the item's outputs (MixOut)
   double alpha_im, beta_im;  // imaginary parts of alpha / beta (complex dtypes only)
-  int32_t chunks;  // 16-deep K chunks of all segments (set by seal_blocks)
+  int32_t chunks;  // 16-deep K chunks of all segments (set by seal_block)
   int32_t wide;    // what holds of its segments' strides (kWideStrides, kContigA, kContigB)
 };
 // A segment's strides are too large for 32-bit offsets in a direct tile; K is the contiguous index
@@ -69,11 +69,11 @@ inline int tile_cols(int kind) {
 }
 
 constexpr int kRowsN = 8;  // widest block the row-streaming path takes
-// Rows per lane of a row tile with short K, the K and N up to which it is taken, and the rows of such
-// blocks from which it is: with fewer, its tiles leave CUs without work (N = K = 3 in FP64, one row /
-// four: 10^5 rows 4.6 / 5.0 us, 1.5 x 10^5 5.3 / 5.1, 3 x 10^5 6.9 / 5.8).  With longer rows of A the
-// lines that a wave comes back to for its next k no longer stay in its cache (N = 4 in FP64, 4 x 10^6
-// rows: K = 8 144 / 119 us, 12 204 / 277; N = 1, K = 32 747 / 1462).
+// Rows per lane of a row tile with short K, the K and N up to which it is taken, and the rows of
+// such blocks from which it is: with fewer, its tiles leave CUs without work (N = K = 3 in FP64, one
+// row / four: 10^5 rows 4.6 / 5.0 us, 1.5 x 10^5 5.3 / 5.1, 3 x 10^5 6.9 / 5.8).  With longer rows
+// of A the lines that a wave comes back to for its next k no longer stay in its cache (N = 4 in
+// FP64, 4 x 10^6 rows: K = 8 144 / 119 us, 12 204 / 277; N = 1, K = 32 747 / 1462).
 constexpr int kShortRows = 4, kShortRowsK = 8, kShortRowsN = 4;
 constexpr int64_t kShortRowsMin = 1 << 17;
 
@@ -141,7 +141,9 @@ constexpr int kXcds = 8;
 // common length *per_xcd (a multiple of 4) with tiles of blk = -1, which the kernels skip.
 // All tiles of a launch share one class (its kernel instantiation), returned: 0 = MFMA tiles
 // up to 32x32, 1 = row streaming (taken when every block has N <= 8 and allow_rows), 2 = 64x32
-// MFMA tiles (only on request).  allow_rows is false for complex dtypes.
+// MFMA tiles and 3 = LDS tiles (both only on request; default_tiling requests LDS tiles).  The
+// launch takes the lean kernels of class 0 and the ones of four rows a lane of class 1 by flags of
+// its own (GemmLaunch::lean, rows4).  allow_rows is false for complex dtypes.
 int make_tiles(const std::vector<GBlk> &blks, const std::vector<GSeg> &segs,
                std::vector<GTile> &tiles, int *per_xcd, int kind_override = -1,
                bool allow_rows = true);

@@ -1149,17 +1149,17 @@ __device__ __forceinline__ void wg_tile_cplx(const char *__restrict__ Abase,
 // Tile classes: each class is its own kernel instantiation so that it carries only its own
 // register budget (occupancy matters most for the memory-bound row tiles).  TC_LEAN is TC_MIXED for
 // launches of short K.
-// TC_ROWS4 is TC_ROWS for launches that hold tiles of kShortRows rows per lane (GemmLaunch::rows4): their
-// registers (83 to 99 for 40 to 55) and LDS would hold the others to five workgroups a CU (10^6 rows
-// of N = 6, K = 10: FP32 46 us for 39; 300000 of N = 8, K = 20: 44 for 34).
+// TC_ROWS4 is TC_ROWS for launches that hold tiles of kShortRows rows per lane (GemmLaunch::rows4):
+// their registers (83 to 99 for 40 to 55) and LDS would hold the others to five workgroups a CU
+// (10^6 rows of N = 6, K = 10: FP32 46 us for 39; 300000 of N = 8, K = 20: 44 for 34).
 enum TileClass { TC_MIXED = 0, TC_ROWS = 1, TC_BIG = 2, TC_LDS = 3, TC_LEAN = 4, TC_ROWS4 = 5 };
 // A lean tile walks the segments and their chunks one at a time, with one set of fragments and
 // 32-bit offsets only, so that four waves (complex128: three) fit a SIMD where the ring's registers
 // leave two: with few chunks of K there is little to pipeline, and other waves hide the latency of
-// a tile's first loads and its stores.  Products of 3000 x 3000, us, ring / lean: FP32 K = 17 17.6 / 15.9, 100 32.1 / 31.2; FP64
-// K = 5 22.9 / 17.5, 17 26.6 / 22.5; complex64 K = 17 37.5 / 32.1, 50 58.1 / 51.4.  Complex128 tiles
-// hold so many values that the ring had no depth for them: they are always lean (200 blocks of
-// 300 x 8, K = 200: 42 / 40; 100000 x 10, K = 200: 96 / 85).
+// a tile's first loads and its stores.  Products of 3000 x 3000, us, ring / lean: FP32 K = 17
+// 17.6 / 15.9, 100 32.1 / 31.2; FP64 K = 5 22.9 / 17.5, 17 26.6 / 22.5; complex64 K = 17 37.5 /
+// 32.1, 50 58.1 / 51.4.  Complex128 tiles hold so many values that the ring had no depth for them:
+// they are always lean (200 blocks of 300 x 8, K = 200: 42 / 40; 100000 x 10, K = 200: 96 / 85).
 template <typename T>
 constexpr int kLeanWaves = std::is_same<T, cd>::value ? 3 : std::is_same<T, cf>::value ? 5 : 4;
 
@@ -1407,11 +1407,10 @@ __device__ __forceinline__ void mfma_accumulate_multi(RealAcc<PREC, MI, NI> (&ac
 }
 
 template <int PREC, typename TA, typename TB, typename TC, int MI, int NI, int WAVES, int PK>
-__global__ __launch_bounds__(64 * WAVES, MI *NI == 4 && WAVES == 4 ? 2 : 4) void k_mix(const GTile *__restrict__ tiles,
-                                                   int per_xcd, const GBlk *__restrict__ items,
-                                                   const GSeg *__restrict__ slices,
-                                                   const MixOut *__restrict__ outs,
-                                                   const char *A, const char *B, char *C) {
+__global__ __launch_bounds__(64 * WAVES, MI *NI == 4 && WAVES == 4 ? 2 : 4) void k_mix(
+    const GTile *__restrict__ tiles, int per_xcd, const GBlk *__restrict__ items,
+    const GSeg *__restrict__ slices, const MixOut *__restrict__ outs, const char *A, const char *B,
+    char *C) {
   using acc_t = typename std::conditional<PREC == CXA_PREC_FP32, float, double>::type;
   constexpr int E = MI * NI * 4;              // accumulator values per lane and slice
   constexpr int NACC = kMixSlices / WAVES;    // slices per wave

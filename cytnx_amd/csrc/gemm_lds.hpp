@@ -8,9 +8,9 @@
 // arithmetic's type and put into LDS k-contiguous, and every wave reads its fragments from there
 // as 16-byte vectors: lane (r, g) = (lane % 16, lane / 16) takes the four consecutive k from 4 g of
 // row (column) r of every 16, so MFMA j sums k = 4 g + j over the four lane groups, as the direct
-// tiles do (the two give the same bits where a direct tile is not split, real FP32 aside).  A row's LDS stride is its bytes plus 16, an odd multiple of 16
-// bytes modulo the 256 bytes of one pass over the banks: the 16 rows of a lane group fall on
-// different banks.
+// tiles do (the two give the same bits where a direct tile is not split, real FP32 aside).  A row's
+// LDS stride is its bytes plus 16, an odd multiple of 16 bytes modulo the 256 bytes of one pass over
+// the banks: the 16 rows of a lane group fall on different banks.
 //
 // Lanes walk whichever index of an operand has the smaller stride (decided per segment), so that
 // row-major and column-major operands are both read in contiguous runs; the direct tiles of

@@ -692,11 +692,11 @@ int launch_tiled(const Reduced &r, const void *src, void *dst, hipStream_t s) {
                            0, s, (const T *)src, (T *)dst, q);
     } else {
       if (q.c > 1)
-        hipLaunchKernelGGL((permute_tiled32_once<T, MAXE, true>), grid_of(q.ntiles), dim3(kThreads), 0,
-                           s, (const T *)src, (T *)dst, q);
+        hipLaunchKernelGGL((permute_tiled32_once<T, MAXE, true>), grid_of(q.ntiles), dim3(kThreads),
+                           0, s, (const T *)src, (T *)dst, q);
       else
-        hipLaunchKernelGGL((permute_tiled32_once<T, MAXE, false>), grid_of(q.ntiles), dim3(kThreads), 0,
-                           s, (const T *)src, (T *)dst, q);
+        hipLaunchKernelGGL((permute_tiled32_once<T, MAXE, false>), grid_of(q.ntiles), dim3(kThreads),
+                           0, s, (const T *)src, (T *)dst, q);
     }
     return 0;
   }

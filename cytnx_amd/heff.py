@@ -622,14 +622,15 @@ class _Flat:
 
 
 def strided_batch_plan(nbatch: int, M: int, N: int, K: int, a: Sequence[int],
-                       b: Sequence[int], c: Sequence[int], dtype: int = 3, chain: bool = False) -> _Plan:
+                       b: Sequence[int], c: Sequence[int], dtype: int = 3,
+                       chain: bool = False) -> _Plan:
     """cxa_strided_batch_plan: C_b = A_b . B_b for b < nbatch with A_b[m, k] at
     a[0]*b + a[1]*m + a[2]*k, B_b[k, n] at b[0]*b + b[1]*k + b[2]*n and C_b[m, n] at
     c[0]*b + c[1]*m + n (element offsets); ``chain`` for a step of a matvec chain."""
     h = ctypes.c_void_p(0)
     _lib.check(_lib.lib().cxa_strided_batch_plan(
-        dtype | (PLAN_CHAIN if chain else 0), nbatch, M, N, K, a[0], a[1], a[2], b[0], b[1], b[2], c[0], c[1],
-        ctypes.byref(h)))
+        dtype | (PLAN_CHAIN if chain else 0), nbatch, M, N, K, a[0], a[1], a[2], b[0], b[1], b[2],
+        c[0], c[1], ctypes.byref(h)))
     return _Plan(h.value, torch.cuda.current_device())
 
 
