@@ -49,9 +49,9 @@ int64_t tiles_of(const GBlk &b, int t) {
 //   1000 x 1000 (1024) 7.3 / 9.5, 200 blocks of 60 x 60 (800), K = 50 5.7 / 7.4;
 //   direct / LDS (64x64 of real types): 3000 x 3000, K = 33 FP32 19.0 / 30.7, complex64 41.7 / 67.6;
 //   K = 100 FP32 31 / 41, FP64 47.7 / 45.1, complex128 137 / 147; 1600 x 1600 complex128, K = 200
-//   87 / 77, 1000 x 1000 (1024 LDS tiles) 37 / 43; 60 blocks of 160 x 160, K = 400 complex128
-//   107 / 86; covering twice the area: 100000 x 10 x 100 FP64 19.6 / 30.7, 10 x 400 x 20000 FP64
-//   13 / 31; 200 blocks of 300 x 8, K = 100 complex64 15.6 / 24.5.
+//   87 / 77, 1000 x 1000 (1024 LDS tiles) 37 / 43 in a list and 44 / 36 by itself; 60 blocks of
+//   160 x 160, K = 400 complex128 107 / 86; covering twice the area: 100000 x 10 x 100 FP64 19.6 /
+//   30.7, 10 x 400 x 20000 FP64 13 / 31; 200 blocks of 300 x 8, K = 100 complex64 15.6 / 24.5.
 constexpr int64_t kFewReal = 512, kFewCplx = 1024, kMany64 = 192, kManyDirect = 768;
 constexpr int64_t kShortChunks = 7, kShortC128 = 13, kRoundLow = 768, kRoundHigh = 1400;
 
