@@ -405,9 +405,12 @@ int make_block_plan(int dtype, int rankL, int nbL, const uint64_t *itoiL, const 
 
   // Extents of the output blocks, axis by axis, as their operands have them: strides are taken
   // apart along these axes.  (An output whose shapes only multiply to the same rows and columns
-  // is the same row-major matrix; a permuted one has no such meaning.)
+  // is the same row-major matrix; a permuted one has no such meaning.  Where the pairs of one
+  // output block disagree, nothing is taken apart along the free axes: every block is a matrix,
+  // permuted into the workspace where its strides are not those of one.)
   std::vector<uint64_t> extC(shapeC, shapeC + (int64_t)nbC * rankC);
   std::vector<char> seenC(nbC, 0);
+  bool flat = false;
   for (const Pair &pr : pairs) {
     const uint64_t *sa = shapeL + (int64_t)pr.a * rankL, *sb = shapeR + (int64_t)pr.b * rankR;
     uint64_t *ec = extC.data() + (int64_t)pr.t * rankC;
@@ -417,9 +420,10 @@ int make_block_plan(int dtype, int rankL, int nbL, const uint64_t *itoiL, const 
       (i < n1 ? M : N) *= (int64_t)ec[i];
       same = same && ec[i] == (i < n1 ? sa[nc1[i]] : sb[nc2[i - n1]]);
     }
-    CXA_CHECK(pr.M == M && pr.N == N && (same || (!out_axes && !seenC[pr.t])), CXA_ERR_INVALID,
+    CXA_CHECK(pr.M == M && pr.N == N && (same || !out_axes), CXA_ERR_INVALID,
               "block contract: output block %d shape does not match its pair (%lld x %lld)", pr.t,
               (long long)pr.M, (long long)pr.N);
+    if (seenC[pr.t] && !same) flat = true;
     seenC[pr.t] = 1;
     for (int i = 0; i < rankC; ++i) ec[i] = i < n1 ? sa[nc1[i]] : sb[nc2[i - n1]];
   }
@@ -499,8 +503,17 @@ int make_block_plan(int dtype, int rankL, int nbL, const uint64_t *itoiL, const 
       if (q != R.main) R.split *= R.r[q].ext;
     return R;
   };
+  // all axes as one (flat: their stride is the last axis')
+  auto one_run = [](int n, const uint64_t *ext) {
+    Runs R;
+    int64_t all = 1;
+    for (int i = 0; i < n; ++i) all *= (int64_t)ext[i];
+    R.r[R.n++] = Run{0, all == 1 ? 0 : n, all};
+    return R;
+  };
   auto runs_m = [&](int t) {
     const uint64_t *sc = extC.data() + (int64_t)t * rankC;
+    if (flat) return one_run(n1, sc);
     return runs_of(n1, sc, [&, t](int i, int j) {
       if (stC[(size_t)t * 32 + i] != (int64_t)sc[j] * stC[(size_t)t * 32 + j]) return false;
       for (int pi : by_target[t]) {
@@ -512,6 +525,7 @@ int make_block_plan(int dtype, int rankL, int nbL, const uint64_t *itoiL, const 
   };
   auto runs_n = [&](int t) {
     const uint64_t *sc = extC.data() + (int64_t)t * rankC + n1;
+    if (flat) return one_run(n2, sc);
     return runs_of(n2, sc, [&, t](int i, int j) {
       if (stC[(size_t)t * 32 + n1 + i] != (int64_t)sc[j] * stC[(size_t)t * 32 + n1 + j])
         return false;
@@ -565,7 +579,7 @@ int make_block_plan(int dtype, int rankL, int nbL, const uint64_t *itoiL, const 
            nseg <= 16 * (int64_t)pairs.size() + 64;
   };
   std::vector<int64_t> offT(offC, offC + nbC);  // where the products' output blocks go
-  bool in_place = !(p->chain && !is_complex(dtype)) && worth();
+  bool in_place = !flat && !(p->chain && !is_complex(dtype)) && worth();
   std::vector<CopyJob> copiesC;
   if (!in_place && out_axes && rankC <= 16) {
     for (int t = 0; t < nbC; ++t) {
@@ -646,6 +660,18 @@ int make_block_plan(int dtype, int rankL, int nbL, const uint64_t *itoiL, const 
       p->wsB += (n + 15) / 16 * 16;
       copiesB.push_back(j);
     }
+  }
+
+  if (flat) {
+    // (the stride of merged axes is that of the innermost one longer than 1)
+    auto last_stride = [](int64_t *st, const uint64_t *sh, const int *ax, int n) {
+      for (int i = 0; i + 1 < n; ++i)
+        if (sh[ax[n - 1]] == 1 && sh[ax[i]] != 1) st[n - 1] = st[i];
+    };
+    for (int a = 0; a < nbL; ++a)
+      last_stride(&stA[(size_t)a * 16], shapeL + (int64_t)a * rankL, axA, n1);
+    for (int b = 0; b < nbR; ++b)
+      last_stride(&stB[(size_t)b * 16] + ncomm, shapeR + (int64_t)b * rankR, axB + ncomm, n2);
   }
 
   split_copies(es, copiesA, p->jobsA, p->bjobsA, p->btasksA);
